@@ -764,7 +764,7 @@ __global__ __launch_bounds__(256) void dyn_coef_fwd_kernel(
 // dp_out[b][dp_stride(np)] (np rounded up to 32, zero padded), s_out[b];
 // per-workgroup partial sums of db (np values) and dalpha (3) in
 // part[blk][np + 3].  RES = false: the Sinkhorn adjoint's output is taken as
-// zero (as in dyn_coef16_bwd_kernel<false>), so no adjoint runs and dP_res,
+// zero (as in dyn_coef_el_bwd_kernel<S, false>), so no adjoint runs and dP_res,
 // db_res and dalpha_res are zeros.
 // ---------------------------------------------------------------------------
 template <int N, bool RES = true>
@@ -1228,143 +1228,349 @@ __global__ __launch_bounds__(skb::kThreads) void dyn_coef32_bwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// n = 4: one token per 16-lane DPP row.  Lane l holds element (l/4, l%4) of
-// t_res and, for l < 8, t_pre[l] (l < 4) or t_post[l-4] (the coefficient
-// order), so the Sinkhorn iterations are a few DPP steps per lane
-// (sk16_forward / sk16_backward) and the per-token loads and stores are
-// contiguous.  Lanes of tokens past the batch compute on token 0 and store
-// nothing.
+// n = 3..8: one token per S x S lanes (S = 4: n = 3, 4 on a 16-lane DPP row;
+// S = 8: n = 5..8 on a wave).  Lane l holds element (l / S, l % S) of t_res,
+// zero-padded to S x S, and, for l < 2n, t_pre[l] (l < n) or t_post[l - n]
+// (the coefficient order), so the Sinkhorn iterations are a few DPP steps per
+// lane (SkEl) and the per-token loads and stores are contiguous.  Lanes of
+// tokens past the batch compute on token 0 and store nothing.
+//
+// The K-split partials are the other latency here: few tokens go with many
+// splits (16 tokens, K = 16384: 64), and a loop that adds them one by one
+// waits for each.  A lane loads 8 splits at a time (past the last one it reads
+// the last again and adds zero), and with at most kCoefSplitTok tokens QS = 4
+// lane groups per token (S = 4) take every fourth split each.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void dyn_coef16_fwd_kernel(
+constexpr int kCoefUnroll = 8;
+constexpr int64_t kCoefSplitTok = 1024;
+
+template <int S, int QS>
+__global__ __launch_bounds__(256) void dyn_coef_el_fwd_kernel(
     const float* __restrict__ p_part, const float* __restrict__ ss_part, int ks, int64_t B, int64_t K,
     const float* __restrict__ a_pre, const float* __restrict__ a_post, const float* __restrict__ a_res,
     const float* __restrict__ b_pre, const float* __restrict__ b_post, const float* __restrict__ b_res,
-    float* __restrict__ coef, float* __restrict__ p_out, float* __restrict__ rh, int iters, float sk_eps,
+    float* __restrict__ coef, float* __restrict__ p_out, float* __restrict__ rh, int n, int iters, float sk_eps,
     float rms_eps) {
-    constexpr int N = 4;
-    constexpr int NP = 2 * N + N * N;
+    constexpr int L = SkEl<S>::kLanes;
+    static_assert(L * QS <= kWave, "a token's lane groups share a wave");
+    const int np = 2 * n + n * n;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t tok = gid >> 4;
-    const int l = (int)(gid & 15);
+    const int64_t tok = gid / (L * QS);
+    const int q0 = (int)(gid / L) % QS;
+    const int l = (int)(gid % L);
+    const int i = l / S, j = l % S;
+    const bool on = i < n && j < n;
     const bool tv = tok < B;
     const int64_t tk = tv ? tok : 0;
+    const int ores = on ? 2 * n + i * n + j : 0;
+    const int opq = l < 2 * n ? l : 0;
+    // partial rows of the lane's outputs: tile o / 32, column o % 32
+    const float* pres_p = p_part + (((int64_t)(ores >> 5) * ks) * B + tk) * kNPad + (ores & 31);
+    const float* ppq_p = p_part + tk * kNPad + opq;  // 2n <= 16: tile 0
     float pres = 0.f, ppq = 0.f, ss = 0.f;
-    for (int q = 0; q < ks; ++q) {
-        const float* pb = p_part + ((int64_t)q * B + tk) * kNPad;
-        ss += ss_part[(int64_t)q * B + tk];
-        pres += pb[2 * N + l];
-        ppq += pb[l & 7];
+    for (int qb = q0; qb < ks; qb += QS * kCoefUnroll) {
+        float vr[kCoefUnroll], vq[kCoefUnroll], vs[kCoefUnroll];
+#pragma unroll
+        for (int u = 0; u < kCoefUnroll; ++u) {
+            int q = qb + QS * u;
+            q = q < ks ? q : ks - 1;
+            const int64_t ro = (int64_t)q * B;
+            vr[u] = pres_p[ro * kNPad];
+            vq[u] = ppq_p[ro * kNPad];
+            vs[u] = ss_part[ro + tk];
+        }
+#pragma unroll
+        for (int u = 0; u < kCoefUnroll; ++u) {
+            const bool in = qb + QS * u < ks;
+            pres += in ? vr[u] : 0.f;
+            ppq += in ? vq[u] : 0.f;
+            ss += in ? vs[u] : 0.f;
+        }
+    }
+    if constexpr (QS == 4) {
+        pres = xor32_add(xor16_add(pres));
+        ppq = xor32_add(xor16_add(ppq));
+        ss = xor32_add(xor16_add(ss));
     }
     const float r_h = sqrtf(ss / (float)K + rms_eps);
     const float inv = 1.f / r_h;
-    const float h = (l < N) ? sigmoidf(ppq * a_pre[0] * inv + b_pre[l & 3])
-                            : 2.f * sigmoidf(ppq * a_post[0] * inv + b_post[(l - N) & 3]);
-    float e = expf(pres * a_res[0] * inv + b_res[l]);
-    sk16_forward(e, iters, sk_eps);
-    if (tv) {
-        float* cf = coef + tok * NP;
-        cf[2 * N + l] = e;
-        if (l < 2 * N) cf[l] = h;
+    const int hb = opq < n ? opq : opq - n;
+    const float h = (l < n) ? sigmoidf(ppq * a_pre[0] * inv + b_pre[hb])
+                            : 2.f * sigmoidf(ppq * a_post[0] * inv + b_post[hb]);
+    float e = on ? expf(pres * a_res[0] * inv + b_res[ores - 2 * n]) : 0.f;
+    SkEl<S>::forward(e, iters, SkEl<S>::pad_eps(i, n, sk_eps), SkEl<S>::pad_eps(j, n, sk_eps));
+    if (tv && q0 == 0) {
+        float* cf = coef + tok * np;
+        if (on) cf[ores] = e;
+        if (l < 2 * n) cf[l] = h;
         if (p_out) {
-            float* po = p_out + tok * NP;
-            po[2 * N + l] = pres;
-            if (l < 2 * N) po[l] = ppq;
+            float* po = p_out + tok * np;
+            if (on) po[ores] = pres;
+            if (l < 2 * n) po[l] = ppq;
         }
         if (l == 0 && rh) rh[tok] = r_h;
     }
 }
 
-int dyn_coef16_bwd_blocks(int64_t B) {
-    int64_t g = (B + 15) / 16;
+// Tokens per workgroup of the backward, and its workgroups (they stride over
+// groups of that many tokens).
+constexpr int coef_el_tokens(int S) { return 256 / (S * S); }
+static int dyn_coef_el_bwd_blocks(int n, int64_t B) {
+    const int per = coef_el_tokens(sk_el_size(n));
+    int64_t g = (B + per - 1) / per;
     if (g > 1024) g = 1024;
     return (int)(g < 1 ? 1 : g);
 }
 
-// Backward of dyn_coef16_fwd_kernel (the formulas of dyn_coef_bwd_kernel).
-// Workgroups stride over groups of 16 tokens; each lane sums its db / dalpha
-// terms over its tokens in order, then the block reduces them into
-// part[blk][27] = (db_pre[4], db_post[4], db_res[16], dalpha_pre, dalpha_post,
-// dalpha_res).  RES = false: the Sinkhorn adjoint's output is taken as zero
-// (a dM constant down each column, which the final column normalisation
-// removes), so dP_res, db_res and dalpha_res are zeros.
-template <bool RES>
-__global__ __launch_bounds__(256) void dyn_coef16_bwd_kernel(
+// Backward of dyn_coef_el_fwd_kernel (the formulas of dyn_coef_bwd_kernel).
+// Each lane sums its db / dalpha terms over its tokens in order, then the
+// block reduces them into part[blk][np + 3] = (db_pre, db_post, db_res,
+// dalpha_pre, dalpha_post, dalpha_res).  RES = false: the Sinkhorn adjoint's
+// output is taken as zero (a dM constant down each column, which the final
+// column normalisation removes), so dP_res, db_res and dalpha_res are zeros.
+template <int S, bool RES>
+__global__ __launch_bounds__(256) void dyn_coef_el_bwd_kernel(
     const float* __restrict__ scal, const float* __restrict__ coef, const float* __restrict__ p,
     const float* __restrict__ rh, int64_t B, int64_t K, const float* __restrict__ a_pre,
     const float* __restrict__ a_post, const float* __restrict__ a_res, const float* __restrict__ b_res,
-    float* __restrict__ dp_out, float* __restrict__ s_out, float* __restrict__ part, int iters, float sk_eps) {
-    constexpr int N = 4;
-    constexpr int NP = 2 * N + N * N;
-    constexpr int NS = N * N + 2 * N;
-    constexpr int NV = NP + 3;
-    __shared__ float red[4][NV];
-    const int l = threadIdx.x & 15;
+    float* __restrict__ dp_out, float* __restrict__ s_out, float* __restrict__ part, int n, int iters,
+    float sk_eps) {
+    constexpr int L = SkEl<S>::kLanes;
+    constexpr int TPB = coef_el_tokens(S);
+    constexpr int NVM = S * S + 2 * S + 3;
+    __shared__ float red[4][NVM];
+    const int np = 2 * n + n * n;
+    const int ns = n * n + 2 * n;
+    const int npt = dp_stride(np);
+    const int l = (int)(threadIdx.x % L);
+    const int i = l / S, j = l % S;
+    const bool on = i < n && j < n;
+    const bool pq = l < 2 * n;
+    const int er = on ? i * n + j : 0;
+    const int eq = pq ? l : 0;
+    const int hb = eq < n ? eq : eq - n;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const float ap = a_pre[0], aq = a_post[0], ar = a_res[0];
-    const float apq = (l < N) ? ap : aq;
+    const float apq = (l < n) ? ap : aq;
+    const float epr = SkEl<S>::pad_eps(i, n, sk_eps), epc = SkEl<S>::pad_eps(j, n, sk_eps);
     float acc_pp = 0.f, acc_res = 0.f, acc_a = 0.f, acc_b = 0.f, acc_c = 0.f;
-    const int64_t groups = (B + 15) / 16;
+    const int64_t groups = (B + TPB - 1) / TPB;
     for (int64_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {  // uniform trip count per block
-        const int64_t tok = grp * 16 + (threadIdx.x >> 4);
+        const int64_t tok = grp * TPB + threadIdx.x / L;
         const bool tv = tok < B;
         const int64_t tk = tv ? tok : 0;
-        const float* sc = scal + tk * (NS + 2);
-        const float* cf = coef + tk * NP;
-        const float* pv = p + tk * NP;
+        const float* sc = scal + tk * (ns + 2);
+        const float* cf = coef + tk * np;
+        const float* pv = p + tk * np;
         const float inv = 1.f / rh[tk];
-        const float pr = pv[2 * N + l];
+        const float pr = pv[2 * n + er];
         float dt_res = 0.f;
         if constexpr (RES) {
-            const float e = expf(pr * ar * inv + b_res[l]);
-            float g = sc[l];  // dM element
-            sk16_backward(g, e, iters, sk_eps);
-            dt_res = g * e;
+            const float e = on ? expf(pr * ar * inv + b_res[er]) : 0.f;
+            float g = on ? sc[er] : 0.f;  // dM element
+            SkEl<S>::backward(g, e, iters, epr, epc, on);
+            dt_res = on ? g * e : 0.f;
         }
-        const float hv = cf[l & 7];
-        // dh_post_act[q] at sc[N*N + q], dh_pre_act[q] at sc[N*N + N + q]
-        const float dh = (l < N) ? sc[N * N + N + (l & 3)] : sc[N * N + ((l - N) & 3)];
-        const float dt_pp = (l < N) ? dh * hv * (1.f - hv) : dh * hv * (1.f - 0.5f * hv);
-        const float lpp = (l < 2 * N) ? dt_pp * pv[l & 7] : 0.f;  // l_pre or l_post
-        const float lres = dt_res * pr;
-        const float tot = group_sum<16>(apq * lpp + ar * lres);
+        const float hv = cf[eq];
+        // dh_post_act[q] at sc[n^2 + q], dh_pre_act[q] at sc[n^2 + n + q]
+        const float dh = (l < n) ? sc[n * n + n + hb] : sc[n * n + hb];
+        const float dt_pp = (l < n) ? dh * hv * (1.f - hv) : dh * hv * (1.f - 0.5f * hv);
+        const float lpp = pq ? dt_pp * pv[eq] : 0.f;  // l_pre or l_post
+        const float lres = on ? dt_res * pr : 0.f;
+        const float tot = group_sum<L>(apq * lpp + ar * lres);
         if (tv) {
-            float* dp = dp_out + tok * kNPad;
-            dp[2 * N + l] = ar * dt_res * inv;
-            if (l < 2 * N) dp[l] = apq * dt_pp * inv;
-            else dp[2 * N + N * N + (l - 2 * N)] = 0.f;  // padding entries 24..31
+            float* dp = dp_out + tok * npt;
+            if (on) dp[2 * n + er] = ar * dt_res * inv;
+            if (pq) dp[l] = apq * dt_pp * inv;
+            for (int o = np + l; o < npt; o += L) dp[o] = 0.f;  // padding entries
             if (l == 0) s_out[tok] = -tot * inv * inv * inv / (float)K;
-            if (l < 2 * N) acc_pp += dt_pp;
+            if (pq) acc_pp += dt_pp;
             acc_res += dt_res;
-            if (l < N) acc_a += lpp * inv;
-            else if (l < 2 * N) acc_b += lpp * inv;
+            if (l < n) acc_a += lpp * inv;
+            else if (pq) acc_b += lpp * inv;
             acc_c += lres * inv;
         }
     }
-    // lanes of one slot: l, l+16, l+32, l+48 of every wave, then the waves
-    acc_a = group_sum<16>(acc_a);
-    acc_b = group_sum<16>(acc_b);
-    acc_c = group_sum<16>(acc_c);
+    // a token's lanes, then (S = 4) the wave's four tokens, then the waves
+    acc_a = group_sum<L>(acc_a);
+    acc_b = group_sum<L>(acc_b);
+    acc_c = group_sum<L>(acc_c);
     float v[5] = {acc_pp, acc_res, acc_a, acc_b, acc_c};
+    if constexpr (S == 4) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        v[k] = xor32_add(xor16_add(v[k]));
+        for (int k = 0; k < 5; ++k) v[k] = xor32_add(xor16_add(v[k]));
     }
-    if (lane < 16) {
-        if (l < 2 * N) red[wave][l] = v[0];
-        red[wave][2 * N + l] = v[1];
+    if (lane < L) {
+        if (pq) red[wave][l] = v[0];
+        if (on) red[wave][2 * n + er] = v[1];
         if (l == 0) {
-            red[wave][NP] = v[2];
-            red[wave][NP + 1] = v[3];
-            red[wave][NP + 2] = v[4];
+            red[wave][np] = v[2];
+            red[wave][np + 1] = v[3];
+            red[wave][np + 2] = v[4];
         }
     }
     __syncthreads();
-    if (threadIdx.x < NV) {
+    const int nv = np + 3;
+    if ((int)threadIdx.x < nv) {
         const int nw = blockDim.x >> 6;
         float t = 0.f;
         for (int w = 0; w < nw; ++w) t += red[w][threadIdx.x];
-        part[(int64_t)blockIdx.x * NV + threadIdx.x] = t;
+        part[(int64_t)blockIdx.x * nv + threadIdx.x] = t;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// n = 9..16: one token per wave, its zero-padded 16 x 16 matrix four elements
+// per lane (skw16: lane t holds row t / 4, columns 4 (t % 4) .. + 3).  Same
+// formulas and outputs as dyn_coef_gen_fwd_kernel / dyn_coef_gen_bwd_kernel,
+// whose row per lane makes a token's chain 16 columns of reductions per
+// iteration; the backward keeps the iteration state in registers
+// (iters <= skw16::kTMax).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void dyn_coef_w16_fwd_kernel(
+    const float* __restrict__ p_part, const float* __restrict__ ss_part, int ks, int64_t B, int64_t K,
+    const float* __restrict__ a_pre, const float* __restrict__ a_post, const float* __restrict__ a_res,
+    const float* __restrict__ b_pre, const float* __restrict__ b_post, const float* __restrict__ b_res,
+    float* __restrict__ coef, float* __restrict__ p_out, float* __restrict__ rh, int n, int iters, float sk_eps,
+    float rms_eps) {
+    constexpr int V = skw16::kV;
+    constexpr int U = 4;  // splits loaded at a time
+    const int np = 2 * n + n * n;
+    const int64_t tok = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const bool tv = tok < B;
+    const int64_t tk = tv ? tok : 0;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int i = skw16::row(), c0 = skw16::col0();
+    const int opq = lane < 2 * n ? lane : 0;
+    bool on[V];
+    int er[V];
+    const float* pp[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        on[k] = i < n && c0 + k < n;
+        er[k] = on[k] ? i * n + c0 + k : 0;
+        const int o = 2 * n + er[k];
+        pp[k] = p_part + (((int64_t)(o >> 5) * ks) * B + tk) * kNPad + (o & 31);
+    }
+    const float* pq_p = p_part + tk * kNPad + opq;  // 2n <= 32: tile 0
+    float pr[V] = {0.f, 0.f, 0.f, 0.f}, ppq = 0.f, ss = 0.f;
+    for (int qb = 0; qb < ks; qb += U) {
+        float vr[U][V], vq[U], vs[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int q = qb + u < ks ? qb + u : ks - 1;
+            const int64_t ro = (int64_t)q * B;
+#pragma unroll
+            for (int k = 0; k < V; ++k) vr[u][k] = pp[k][ro * kNPad];
+            vq[u] = pq_p[ro * kNPad];
+            vs[u] = ss_part[ro + tk];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = qb + u < ks;
+#pragma unroll
+            for (int k = 0; k < V; ++k) pr[k] += in ? vr[u][k] : 0.f;
+            ppq += in ? vq[u] : 0.f;
+            ss += in ? vs[u] : 0.f;
+        }
+    }
+    const float r_h = sqrtf(ss / (float)K + rms_eps);
+    const float inv = 1.f / r_h;
+    const int hb = opq < n ? opq : opq - n;
+    const float h = (lane < n) ? sigmoidf(ppq * a_pre[0] * inv + b_pre[hb])
+                               : 2.f * sigmoidf(ppq * a_post[0] * inv + b_post[hb]);
+    float e[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) e[k] = on[k] ? expf(pr[k] * a_res[0] * inv + b_res[er[k]]) : 0.f;
+    skw16::forward_n(e, n, iters, sk_eps);
+    if (tv) {
+        float* cf = coef + tok * np;
+        float* po = p_out ? p_out + tok * np : nullptr;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            if (on[k]) cf[2 * n + er[k]] = e[k];
+            if (on[k] && po) po[2 * n + er[k]] = pr[k];
+        }
+        if (lane < 2 * n) {
+            cf[lane] = h;
+            if (po) po[lane] = ppq;
+        }
+        if (lane == 0 && rh) rh[tok] = r_h;
+    }
+}
+
+__global__ __launch_bounds__(256) void dyn_coef_w16_bwd_kernel(
+    const float* __restrict__ scal, const float* __restrict__ coef, const float* __restrict__ p,
+    const float* __restrict__ rh, int64_t B, int64_t K, const float* __restrict__ a_pre,
+    const float* __restrict__ a_post, const float* __restrict__ a_res, const float* __restrict__ b_res,
+    float* __restrict__ dp_out, float* __restrict__ s_out, float* __restrict__ part, int n, int iters,
+    float sk_eps) {
+    constexpr int V = skw16::kV;
+    const int np = 2 * n + n * n;
+    const int ns = n * n + 2 * n;
+    const int npt = dp_stride(np);
+    const int64_t tok = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const bool tv = tok < B;
+    const int64_t tk = tv ? tok : 0;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int i = skw16::row(), c0 = skw16::col0();
+    const float ap = a_pre[0], aq = a_post[0], ar = a_res[0];
+    const float* sc = scal + tk * (ns + 2);
+    const float* cf = coef + tk * np;
+    const float* pv = p + tk * np;
+    const float inv = 1.f / rh[tk];
+    const bool pq = lane < 2 * n;
+    const int eq = pq ? lane : 0;
+    const int hb = eq < n ? eq : eq - n;
+    bool on[V];
+    int er[V];
+    float gm[V], e[V], pr[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        on[k] = i < n && c0 + k < n;
+        er[k] = on[k] ? i * n + c0 + k : 0;
+        pr[k] = pv[2 * n + er[k]];
+        gm[k] = on[k] ? sc[er[k]] : 0.f;
+        e[k] = on[k] ? expf(pr[k] * ar * inv + b_res[er[k]]) : 0.f;
+    }
+    skw16::backward_n(gm, e, n, iters, sk_eps);
+    const float hv = cf[eq];
+    // dh_post_act[q] at sc[n^2 + q], dh_pre_act[q] at sc[n^2 + n + q]
+    const float dh = (lane < n) ? sc[n * n + n + hb] : sc[n * n + hb];
+    const float dt_pp = (lane < n) ? dh * hv * (1.f - hv) : dh * hv * (1.f - 0.5f * hv);
+    const float apq = (lane < n) ? ap : aq;
+    const float lpp = pq ? dt_pp * pv[eq] : 0.f;
+    float lres = 0.f;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        gm[k] = on[k] ? gm[k] * e[k] : 0.f;  // dt_res
+        lres += on[k] ? gm[k] * pr[k] : 0.f;
+    }
+    const float tot = group_sum<kWave>(apq * lpp + ar * lres);
+    const float s_pre = group_sum<kWave>(lane < n ? lpp : 0.f);
+    const float s_post = group_sum<kWave>(lane < n ? 0.f : lpp);
+    const float s_res = group_sum<kWave>(lres);
+    if (!tv) return;
+    float* dp = dp_out + tok * npt;
+    float* pt = part + tok * (np + 3);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        if (on[k]) {
+            dp[2 * n + er[k]] = ar * gm[k] * inv;
+            pt[2 * n + er[k]] = gm[k];
+        }
+    }
+    if (pq) {
+        dp[lane] = apq * dt_pp * inv;
+        pt[lane] = dt_pp;
+    }
+    for (int o = np + lane; o < npt; o += kWave) dp[o] = 0.f;
+    if (lane == 0) {
+        s_out[tok] = -tot * inv * inv * inv / (float)K;
+        pt[np] = s_pre * inv;
+        pt[np + 1] = s_post * inv;
+        pt[np + 2] = s_res * inv;
     }
 }
 
@@ -2068,21 +2274,34 @@ hipError_t launch_proj_valu(int x_dtype, const void* x, const float* phi, int np
 }
 #endif  // MHC_KERNEL_TIMING
 
-#define MHC_DYN_N(n, ...)                                        \
-    switch (n) {                                                 \
-        case 2: { constexpr int N_ = 2; __VA_ARGS__; break; }    \
-        case 4: { constexpr int N_ = 4; __VA_ARGS__; break; }    \
-        case 8: { constexpr int N_ = 8; __VA_ARGS__; break; }    \
-        case 16: { constexpr int N_ = 16; __VA_ARGS__; break; }  \
-        case 32: { constexpr int N_ = 32; __VA_ARGS__; break; }  \
-        default: return hipErrorInvalidValue;                    \
-    }
+// n whose per-token coefficients run one element per lane (dyn_coef_el_*).
+static bool coef_el_n(int n) { return n >= 3 && n <= 8; }
 
 hipError_t launch_dyn_coef_fwd(int n, const float* p_part, const float* ss_part, int ks, int64_t B, int64_t K,
                                const float* a_pre, const float* a_post, const float* a_res, const float* b_pre,
                                const float* b_post, const float* b_res, float* coef, float* p_out, float* rh,
                                int iters, float sk_eps, float rms_eps, hipStream_t s) {
     if (B == 0) return hipSuccess;
+    if (coef_el_n(n)) {
+#define MHC_DCE_FWD(S_, QS_)                                                                                       \
+    MHC_LAUNCH_GGL((dyn_coef_el_fwd_kernel<S_, QS_>), dim3((unsigned)((B * S_ * S_ * QS_ + 255) / 256)), dim3(256), 0, \
+                       s, p_part, ss_part, ks, B, K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, n,   \
+                       iters, sk_eps, rms_eps)
+        if (sk_el_size(n) == 8) {
+            MHC_DCE_FWD(8, 1);
+        } else if (B <= kCoefSplitTok) {
+            MHC_DCE_FWD(4, 4);
+        } else {
+            MHC_DCE_FWD(4, 1);
+        }
+#undef MHC_DCE_FWD
+        return hipGetLastError();
+    }
+    if (n > 8 && n <= skw16::kN) {
+        MHC_LAUNCH_GGL(dyn_coef_w16_fwd_kernel, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, p_part, ss_part, ks, B,
+                       K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, n, iters, sk_eps, rms_eps);
+        return hipGetLastError();
+    }
     if (generic_layer_n(n)) {
 #define MHC_DCG_FWD(NM_)                                                                                          \
     MHC_LAUNCH_GGL((dyn_coef_gen_fwd_kernel<NM_>), dim3((unsigned)((B * NM_ + 255) / 256)), dim3(256), 0, s,     \
@@ -2092,29 +2311,23 @@ hipError_t launch_dyn_coef_fwd(int n, const float* p_part, const float* ss_part,
 #undef MHC_DCG_FWD
         return hipGetLastError();
     }
-    if (n == 4) {
-        MHC_LAUNCH_GGL(dyn_coef16_fwd_kernel, dim3((unsigned)((B * 16 + 255) / 256)), dim3(256), 0, s, p_part,
-                           ss_part, ks, B, K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, iters,
-                           sk_eps, rms_eps);
-        return hipGetLastError();
-    }
     if (n == skb::kN) {
         MHC_LAUNCH_GGL(dyn_coef32_fwd_kernel, dim3((unsigned)B), dim3(skb::kThreads), 0, s, p_part, ss_part, ks, B,
                            K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, iters, sk_eps, rms_eps);
         return hipGetLastError();
     }
+    if (n != 2) return hipErrorInvalidValue;
     const int64_t threads = B * pow2ceil(n);
     const unsigned blocks = (unsigned)((threads + 255) / 256);
-    MHC_DYN_N(n, MHC_LAUNCH_GGL((dyn_coef_fwd_kernel<N_>), dim3(blocks), dim3(256), 0, s, p_part, ss_part, ks, B,
-                                    K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, iters, sk_eps,
-                                    rms_eps));
+    MHC_LAUNCH_GGL((dyn_coef_fwd_kernel<2>), dim3(blocks), dim3(256), 0, s, p_part, ss_part, ks, B, K, a_pre, a_post,
+                   a_res, b_pre, b_post, b_res, coef, p_out, rh, iters, sk_eps, rms_eps);
     return hipGetLastError();
 }
 
 // Rows of the db / dalpha partials: one per workgroup, or one per token for
 // n >= 16 and for the generic-n kernel.
 int dyn_coef_bwd_blocks(int n, int64_t B) {
-    if (n == 4) return dyn_coef16_bwd_blocks(B);
+    if (coef_el_n(n)) return dyn_coef_el_bwd_blocks(n, B);
     if (n >= 16 || generic_layer_n(n)) return (int)(B < 1 ? 1 : B);
     return (int)((B * pow2ceil(n) + 255) / 256);
 }
@@ -2140,7 +2353,7 @@ static int dyn_coef_gen_nm(int n) { return n <= 16 ? 16 : (n <= 32 ? 32 : 64); }
 constexpr int kGenHistIters = 20;  // iterations the reserved region is sized for
 
 size_t dyn_coef_gen_hist_bytes(int n, int64_t B) {
-    if (!generic_layer_n(n) || B <= 0) return 0;
+    if (!generic_layer_n(n) || coef_el_n(n) || B <= 0) return 0;
     const int nm = dyn_coef_gen_nm(n), per_wg = 256 / nm;
     const int64_t wgs = (B + per_wg - 1) / per_wg;
     const size_t need = (size_t)wgs * per_wg * (size_t)skw_hist_floats(nm, n, kGenHistIters) * sizeof(float);
@@ -2161,6 +2374,24 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
                                const float* b_res, float* dp_out, float* s_out, float* part, int iters, float sk_eps,
                                float* hist, hipStream_t s, bool res_rows) {
     if (B == 0) return hipSuccess;
+    if (coef_el_n(n)) {
+        const unsigned eblocks = (unsigned)dyn_coef_el_bwd_blocks(n, B);
+#define MHC_DCE_BWD(S_, RES_)                                                                                         \
+    MHC_LAUNCH_GGL((dyn_coef_el_bwd_kernel<S_, RES_>), dim3(eblocks), dim3(256), 0, s, scal, coef, p, rh, B, K, a_pre, \
+                       a_post, a_res, b_res, dp_out, s_out, part, n, iters, sk_eps)
+        if (sk_el_size(n) == 8) {
+            if (res_rows) { MHC_DCE_BWD(8, true); } else { MHC_DCE_BWD(8, false); }
+        } else {
+            if (res_rows) { MHC_DCE_BWD(4, true); } else { MHC_DCE_BWD(4, false); }
+        }
+#undef MHC_DCE_BWD
+        return hipGetLastError();
+    }
+    if (n > 8 && n <= skw16::kN && res_rows && iters <= skw16::kTMax) {
+        MHC_LAUNCH_GGL(dyn_coef_w16_bwd_kernel, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, scal, coef, p, rh, B, K,
+                       a_pre, a_post, a_res, b_res, dp_out, s_out, part, n, iters, sk_eps);
+        return hipGetLastError();
+    }
     if (generic_layer_n(n)) {
         // one token per lane group, or (history in hist) as many token slots
         // as the history region holds, each taking several tokens
@@ -2186,17 +2417,6 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
 #undef MHC_DCG_BWD
         return hipGetLastError();
     }
-    const unsigned blocks = (unsigned)dyn_coef_bwd_blocks(n, B);
-    if (n == 4) {
-        if (res_rows) {
-            MHC_LAUNCH_GGL(dyn_coef16_bwd_kernel<true>, dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K, a_pre,
-                               a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
-        } else {
-            MHC_LAUNCH_GGL(dyn_coef16_bwd_kernel<false>, dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K,
-                               a_pre, a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
-        }
-        return hipGetLastError();
-    }
     if (!res_rows && n >= 16) {
         // no adjoint runs: the run-time-n kernel on n-lane groups
         const int64_t gblocks = (B * n + 255) / 256;
@@ -2214,17 +2434,6 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
         }
         return hipGetLastError();
     }
-    if (!res_rows && (n == 2 || n == 8)) {
-        if (n == 2) {
-            MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<2, false>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K,
-                               a_pre, a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
-        } else {
-            MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<8, false>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K,
-                               a_pre, a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
-        }
-        return hipGetLastError();
-    }
-    if (!res_rows) return hipErrorInvalidValue;
     if (n == skb::kN && iters <= skb::kTMax) {
         MHC_LAUNCH_GGL(dyn_coef32_bwd_kernel, dim3((unsigned)B), dim3(skb::kThreads), 0, s, scal, coef, p, rh, B, K,
                            a_pre, a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
@@ -2245,12 +2454,14 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
         }
         return hipGetLastError();
     }
-    switch (n) {
-        case 2: MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<2>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K,
-                                   a_pre, a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps); break;
-        case 8: MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<8>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K,
-                                   a_pre, a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps); break;
-        default: return hipErrorInvalidValue;
+    if (n != 2) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)dyn_coef_bwd_blocks(n, B);
+    if (res_rows) {
+        MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<2, true>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K, a_pre,
+                           a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
+    } else {
+        MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<2, false>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K, a_pre,
+                           a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);
     }
     return hipGetLastError();
 }

@@ -27,6 +27,28 @@ namespace mhc {
 
 template <int N> constexpr int coef_size() { return 2 * N + N * N; }
 
+// The shared N x N matrix (N = 3..8) on lanes 0 .. S^2 - 1 of one wave, one
+// element per lane: `at` = the lane's element r N + c when `on`.  The wave's
+// other lanes compute on zeros.
+template <int N>
+struct SkShared {
+    static constexpr int S = sk_el_size(N);
+    int at;
+    bool on;
+    float er, ec;
+    __device__ __forceinline__ SkShared(int lane, float eps) {
+        const int r = (lane / S) % S, c = lane % S;
+        at = r * N + c;
+        on = lane < S * S && r < N && c < N;
+        er = SkEl<S>::pad_eps(r, N, eps);
+        ec = SkEl<S>::pad_eps(c, N, eps);
+    }
+    __device__ __forceinline__ void forward(float& a, int iters) const { SkEl<S>::forward(a, iters, er, ec); }
+    __device__ __forceinline__ void backward(float& g, float x0, int iters) const {
+        SkEl<S>::backward(g, x0, iters, er, ec, on);
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Static coefficients: h_pre = sigmoid(H_pre), h_post = 2 sigmoid(H_post),
 // M = SK(exp(H_res)) (layer.py:144-160), computed once per call, plus the
@@ -71,12 +93,13 @@ __global__ __launch_bounds__(256) void static_coef_kernel(const float* __restric
         return;
     }
     if (r >= kWave) return;
-    if constexpr (N == 4) {
-        // the shared M = SK(exp(H_res)): one element per lane of lanes 0..15
-        // (the finalize's adjoint recomputes it with the same code)
-        float a = r < 16 ? expf(h_res[r]) : 0.f;
-        sk16_forward(a, iters, eps);
-        if (r < 16) saved[2 * N + r] = a;
+    if constexpr (N >= 3 && N <= 8) {
+        // the shared M = SK(exp(H_res)): one element per lane (the finalize's
+        // adjoint recomputes it with the same code)
+        const SkShared<N> k(r, eps);
+        float a = k.on ? expf(h_res[k.at]) : 0.f;
+        k.forward(a, iters);
+        if (k.on) saved[2 * N + k.at] = a;
     } else if constexpr (N == skw16::kN) {
         // the 16 x 16 matrix on wave 0, four elements per lane (the
         // finalize's adjoint recomputes it with the same code)
@@ -210,10 +233,11 @@ __device__ __forceinline__ void static_coefs_wave(const float* __restrict__ h_pr
         put(r, sigmoidf(h_pre[r]));
         put(N + r, 2.f * sigmoidf(h_post[r]));
     }
-    if constexpr (N == 4) {
-        float a = r < 16 ? expf(h_res[r]) : 0.f;
-        sk16_forward(a, iters, eps);
-        if (r < 16) put(2 * N + r, a);
+    if constexpr (N >= 3) {
+        const SkShared<N> k(r, eps);
+        float a = k.on ? expf(h_res[k.at]) : 0.f;
+        k.forward(a, iters);
+        if (k.on) put(2 * N + k.at, a);
     } else {
         float a[N];
 #pragma unroll
@@ -645,8 +669,8 @@ __global__ __launch_bounds__(256) void column_partial1_kernel(const float* __res
 //     dH_pre = dh_pre_act h_pre (1 - h_pre)
 //     dH_post = dh_post_act h_post (1 - h_post / 2)
 //     dH_res = SK^T(dM) * exp(H_res)
-// For n = 4 the Sinkhorn recompute and adjoint run one element per lane of a
-// 16-lane row, as the forward's coefficient kernel computes M.
+// For n = 3..8 the Sinkhorn recompute and adjoint run one element per lane
+// (SkEl), as the forward's coefficient kernel computes M.
 constexpr int kColSplit = 16;   // row groups of the first pass when rows are many
 constexpr int kDirectRows = 512;  // partial rows the finalize sums directly
 
@@ -701,16 +725,17 @@ __global__ __launch_bounds__(256) void layer_finalize_kernel(
             for (int k = 0; k < NS; ++k) v[k] += scal_part[(int64_t)r * NS + k];
         }
         block_sum<NS>(v, red);
-        if constexpr (N == 4) {
+        if constexpr (N >= 3 && N <= 8) {
             if (threadIdx.x < kWave) {
-                // one element per lane of lanes 0..15, as the forward computed M
-                const int l = threadIdx.x;
-                const float e = l < 16 ? expf(h_res[l]) : 0.f;
+                // one element per lane, as the forward computed M
+                const SkShared<N> k(threadIdx.x, eps);
+                const float e = k.on ? expf(h_res[k.at]) : 0.f;
                 float g = 0.f;
 #pragma unroll
-                for (int q = 0; q < 16; ++q) g = (l == q) ? v[q] : g;
-                sk16_backward(g, e, iters, eps);
-                if (l < 16) d_h_res[l] = g * e;
+                for (int q = 0; q < N * N; ++q) g = (k.at == q) ? v[q] : g;
+                if (!k.on) g = 0.f;
+                k.backward(g, e, iters);
+                if (k.on) d_h_res[k.at] = g * e;
             }
         } else if (threadIdx.x < kWave) {
             const int r = threadIdx.x;

@@ -6,10 +6,11 @@
 // column sums are lane-group butterflies.  The backward keeps the forward
 // history (post-row-step rows and row sums) in registers and applies the
 // exact adjoint (the reference's row step is approximate,
-// sinkhorn_knopp.cpp:1773-1795).  Small n = 4 batches run one element per
-// lane of a 16-lane DPP row instead (sk16_* in mhc_device.h); 8 < n <= 64
-// runs the masked wide kernels (skw_*), whose backward recomputes the
-// forward state per iteration instead of keeping a history.
+// sinkhorn_knopp.cpp:1773-1795).  Small batches at n = 3..8 run one element
+// per lane of a 16-lane DPP row or a wave instead (SkEl in mhc_device.h), 9 <= n
+// <= 32 a matrix per wave or workgroup (skw16, skb); n up to 64 (and adjoints
+// of more than 32 iterations) the masked wide kernels (skw_*), whose backward
+// recomputes the forward state per iteration instead of keeping a history.
 #include "mhc_device.h"
 #include "mhc_internal.h"
 
@@ -77,31 +78,42 @@ __global__ __launch_bounds__(256) void sinkhorn_bwd_kernel(const float* __restri
     if (ok) store_row<N>(grad_inp + m * N * N + r * N, g);
 }
 
-// n = 4: one matrix per 16-lane DPP row, one element per lane (lane 4 r + c);
-// the loads and stores are one contiguous float per lane.  The chain per
-// matrix is about 4x shorter than with one row per lane but issues more
-// instructions in total, so it is used for batches that leave the chip
-// latency-bound; large batches (throughput-bound) keep one row per lane.
-constexpr int64_t kSk16MaxBatch = 16384;
-__global__ __launch_bounds__(256) void sinkhorn16_fwd_kernel(const float* __restrict__ inp, float* __restrict__ out,
-                                                             int64_t batch, int iters, float eps) {
+// n = 3..8: one matrix per S x S lanes, one element per lane (SkEl).  The
+// chain per matrix is about S times shorter than with one row per lane but
+// issues more instructions in total, so it is used for batches that leave the
+// chip latency-bound; large batches (throughput-bound) keep one row per lane,
+// except where that form's adjoint recomputes its history (n = 5..8 past
+// SkHist's iterations: O(iters^2) steps).
+constexpr int64_t kSkElMaxBatch = 16384;
+template <int S>
+__global__ __launch_bounds__(256) void sinkhorn_el_fwd_kernel(const float* __restrict__ inp, float* __restrict__ out,
+                                                              int n, int64_t batch, int iters, float eps) {
+    constexpr int L = SkEl<S>::kLanes;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool ok = gid < batch * 16;
-    float a = ok ? inp[gid] : 0.f;
-    sk16_forward(a, iters, eps);
-    if (ok) out[gid] = a;
+    const int64_t m = gid / L;
+    const int r = (int)(gid % L) / S, c = (int)(gid % S);
+    const bool on = m < batch && r < n && c < n;
+    const int64_t at = m * n * n + r * n + c;
+    float a = on ? inp[at] : 0.f;
+    SkEl<S>::forward(a, iters, SkEl<S>::pad_eps(r, n, eps), SkEl<S>::pad_eps(c, n, eps));
+    if (on) out[at] = a;
 }
 
-__global__ __launch_bounds__(256) void sinkhorn16_bwd_kernel(const float* __restrict__ grad_out,
-                                                             const float* __restrict__ inp,
-                                                             float* __restrict__ grad_inp, int64_t batch, int iters,
-                                                             float eps) {
+template <int S>
+__global__ __launch_bounds__(256) void sinkhorn_el_bwd_kernel(const float* __restrict__ grad_out,
+                                                              const float* __restrict__ inp,
+                                                              float* __restrict__ grad_inp, int n, int64_t batch,
+                                                              int iters, float eps) {
+    constexpr int L = SkEl<S>::kLanes;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool ok = gid < batch * 16;
-    float g = ok ? grad_out[gid] : 0.f;
-    const float x0 = ok ? inp[gid] : 0.f;
-    sk16_backward(g, x0, iters, eps);
-    if (ok) grad_inp[gid] = g;
+    const int64_t m = gid / L;
+    const int r = (int)(gid % L) / S, c = (int)(gid % S);
+    const bool on = m < batch && r < n && c < n;
+    const int64_t at = m * n * n + r * n + c;
+    float g = on ? grad_out[at] : 0.f;
+    const float x0 = on ? inp[at] : 0.f;
+    SkEl<S>::backward(g, x0, iters, SkEl<S>::pad_eps(r, n, eps), SkEl<S>::pad_eps(c, n, eps), on);
+    if (on) grad_inp[at] = g;
 }
 
 // 8 < n <= 64: one matrix per group of NM = pow2ceil(n) lanes (16, 32 or
@@ -153,6 +165,82 @@ __global__ __launch_bounds__(256) void sinkhorn_wide_bwd_kernel(const float* __r
     }
 }
 
+// 9 <= n <= 16: one matrix per wave, four elements per lane (skw16); 17 <= n
+// <= 32: one matrix per 256-lane workgroup (skb).  The row-per-lane kernels
+// above walk 16 or 32 columns of lane-group reductions per iteration, and
+// their adjoint recomputes each iteration's state; these keep it in registers
+// (up to kTMax = 32 iterations).
+__global__ __launch_bounds__(256) void sinkhorn_w16_kernel(const float* __restrict__ grad_out,
+                                                           const float* __restrict__ inp, float* __restrict__ out,
+                                                           int n, int64_t batch, int iters, float eps) {
+    constexpr int V = skw16::kV;
+    const int64_t m = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const int i = skw16::row(), c0 = skw16::col0();
+    const int64_t at = (m * n + i) * n + c0;
+    bool on[V];
+    float a[V], g[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        on[k] = m < batch && i < n && c0 + k < n;
+        a[k] = on[k] ? inp[at + k] : 0.f;
+        g[k] = on[k] && grad_out ? grad_out[at + k] : 0.f;
+    }
+    if (grad_out) {  // the same for the whole grid
+        skw16::backward_n(g, a, n, iters, eps);
+    } else {
+        skw16::forward_n(a, n, iters, eps);
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        if (on[k]) out[at + k] = grad_out ? g[k] : a[k];
+    }
+}
+
+__global__ __launch_bounds__(skb::kThreads) void sinkhorn_b32_kernel(const float* __restrict__ grad_out,
+                                                                     const float* __restrict__ inp,
+                                                                     float* __restrict__ out, int n, int iters,
+                                                                     float eps) {
+    constexpr int V = skb::kV;
+    __shared__ float part[skb::kPartFloats];
+    __shared__ float hc[skb::kHistFloats];
+    const int64_t m = blockIdx.x;
+    const int i = skb::row(), c0 = skb::col0();
+    const int64_t at = (m * n + i) * n + c0;
+    bool on[V];
+    float a[V], g[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        on[k] = i < n && c0 + k < n;
+        a[k] = on[k] ? inp[at + k] : 0.f;
+        g[k] = on[k] && grad_out ? grad_out[at + k] : 0.f;
+    }
+    if (grad_out) {  // the same for the whole grid
+        skb::backward_n(g, a, n, iters, eps, part, hc);
+    } else {
+        skb::forward_n(a, n, iters, eps, part);
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        if (on[k]) out[at + k] = grad_out ? g[k] : a[k];
+    }
+}
+
+// Both directions of 9 <= n <= 32 (grad_out null: forward); false: the shape
+// or the iteration count stays with the row-per-lane kernels.
+static bool launch_sinkhorn_tiled(int n, const float* grad_out, const float* inp, float* out, int64_t batch, int iters,
+                                  float eps, hipStream_t s) {
+    if (n <= 8 || n > skb::kN || batch > 0x7fffffff) return false;
+    if (grad_out && iters > (n <= skw16::kN ? skw16::kTMax : skb::kTMax)) return false;
+    if (n <= skw16::kN) {
+        MHC_LAUNCH_GGL(sinkhorn_w16_kernel, dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, s, grad_out, inp, out, n,
+                       batch, iters, eps);
+    } else {
+        MHC_LAUNCH_GGL(sinkhorn_b32_kernel, dim3((unsigned)batch), dim3(skb::kThreads), 0, s, grad_out, inp, out, n,
+                       iters, eps);
+    }
+    return true;
+}
+
 #define MHC_SK_WIDE(n, ...)                                                   \
     if (n <= 16) {                                                            \
         constexpr int NM_ = 16; __VA_ARGS__;                                  \
@@ -184,9 +272,15 @@ hipError_t launch_sinkhorn_fwd(int n, const float* inp, float* out, int64_t batc
     const int64_t threads = batch * G;
     const unsigned blocks = (unsigned)((threads + 255) / 256);
     const int tok = timing_begin("sinkhorn_fwd", s);
-    if (n == 4 && batch < kSk16MaxBatch) {
-        MHC_LAUNCH_GGL(sinkhorn16_fwd_kernel, dim3((unsigned)((batch * 16 + 255) / 256)), dim3(256), 0, s, inp, out,
+    if (n >= 3 && n <= 8 && batch < kSkElMaxBatch) {
+        if (sk_el_size(n) == 4) {
+            MHC_LAUNCH_GGL(sinkhorn_el_fwd_kernel<4>, dim3((unsigned)((batch * 16 + 255) / 256)), dim3(256), 0, s, inp,
+                           out, n, batch, iters, eps);
+        } else {
+            MHC_LAUNCH_GGL(sinkhorn_el_fwd_kernel<8>, dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, s, inp, out, n,
                            batch, iters, eps);
+        }
+    } else if (launch_sinkhorn_tiled(n, nullptr, inp, out, batch, iters, eps, s)) {
     } else if (n > 8) {
         MHC_SK_WIDE(n, MHC_LAUNCH_GGL((sinkhorn_wide_fwd_kernel<NM_>), dim3(blocks), dim3(256), 0, s, inp, out, n,
                                           batch, iters, eps));
@@ -205,9 +299,16 @@ hipError_t launch_sinkhorn_bwd(int n, const float* grad_out, const float* inp, f
     const int64_t threads = batch * G;
     const unsigned blocks = (unsigned)((threads + 255) / 256);
     const int tok = timing_begin("sinkhorn_bwd", s);
-    if (n == 4 && batch < kSk16MaxBatch) {
-        MHC_LAUNCH_GGL(sinkhorn16_bwd_kernel, dim3((unsigned)((batch * 16 + 255) / 256)), dim3(256), 0, s,
-                           grad_out, inp, grad_inp, batch, iters, eps);
+    const bool recompute = n > 4 && n <= 8 && iters > SkHist<8>::TMAX;
+    if (n >= 3 && n <= 8 && (batch < kSkElMaxBatch || recompute)) {
+        if (sk_el_size(n) == 4) {
+            MHC_LAUNCH_GGL(sinkhorn_el_bwd_kernel<4>, dim3((unsigned)((batch * 16 + 255) / 256)), dim3(256), 0, s,
+                           grad_out, inp, grad_inp, n, batch, iters, eps);
+        } else {
+            MHC_LAUNCH_GGL(sinkhorn_el_bwd_kernel<8>, dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, s, grad_out,
+                           inp, grad_inp, n, batch, iters, eps);
+        }
+    } else if (launch_sinkhorn_tiled(n, grad_out, inp, grad_inp, batch, iters, eps, s)) {
     } else if (n > 8) {
         MHC_SK_WIDE(n, MHC_LAUNCH_GGL((sinkhorn_wide_bwd_kernel<NM_>), dim3(blocks), dim3(256), 0, s, grad_out,
                                           inp, grad_inp, n, batch, iters, eps));
