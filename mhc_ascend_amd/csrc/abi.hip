@@ -40,17 +40,17 @@ static int hip_status(hipError_t e) {
 
 static bool valid_dtype(int dt) { return dt == kF32 || dt == kBF16; }
 
-// The layer runs its fixed-n kernels for n in {2, 4, 8, 16, 32} and the
-// generic kernels (generic.hip) for every other n up to kGenMaxN, as the
-// reference takes any n up to MAX_EXPANSION_RATE = 64 (mhc_types.h:68); the
-// fused wrapper takes n = 2..8.
+// The layer runs its fixed-n kernels for n in {2..8, 16, 32} (n = 3, 5, 6, 7:
+// up to kWideMaxC channels) and the generic kernels (generic.hip) for every
+// other n up to kGenMaxN, as the reference takes any n up to
+// MAX_EXPANSION_RATE = 64 (mhc_types.h:68); the fused wrapper takes n = 2..32.
 static bool supported_layer_n(int n) {
     return n == 2 || n == 4 || n == 8 || n == 16 || n == 32 || generic_layer_n(n);
 }
 static bool supported_dynamic_n(int n) { return supported_layer_n(n); }
 // the standalone aggregate / distribute operators
 static bool supported_ops_n(int n) {
-    return n == 1 || n == 2 || n == 4 || n == 8 || n == 16 || n == 32 || generic_ops_n(n);
+    return (n >= 1 && n <= 8) || n == 16 || n == 32 || generic_ops_n(n);
 }
 
 // ---------------------------------------------------------------------------
@@ -281,7 +281,7 @@ int mhc_layer_static_fwd(const void* x, int32_t x_dtype, const void* weight, int
     MHC_REQUIRE(weight && h_pre && h_post && h_res && saved, "layer_static_fwd: null parameter pointer");
     MHC_REQUIRE(batch == 0 || (x && out), "layer_static_fwd: null x/out");
     hipStream_t s = (hipStream_t)stream;
-    if (layer_static_fwd_fused(n, hidden))
+    if (layer_static_fwd_fused(n, hidden) && rows_aligned(n, {x, weight, saved, out}))
         return hip_status(launch_layer_static_fwd(x_dtype, n, x, weight, weight_dtype, h_pre, h_post, h_res, saved,
                                                   num_iters, sinkhorn_eps, out, rms, batch, hidden, rmsnorm_eps, s));
     hipError_t e = launch_static_coef(n, h_pre, h_post, h_res, weight, weight_dtype, hidden, saved, num_iters,
@@ -302,31 +302,34 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // The static Sinkhorn adjoint keeps its per-iteration state in a workspace
 // region (kStaticSkHistBytes) for n >= 16 and the generic n; without it
 // those finalize kernels recompute the forward iterations.
-static bool static_sk_hist(int32_t n) { return n >= 16 || generic_layer_n(n); }
+static bool static_sk_hist(int32_t n) { return n >= 16 || (generic_layer_n(n) && !odd_row_n(n)); }
 
-static StaticBwdWs static_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype) {
+// aligned: rows_aligned() of the call's arrays (the row kernels differ)
+static StaticBwdWs static_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype, bool aligned) {
     StaticBwdWs w{};
-    w.grid = batch > 0 ? layer_bwd_grid(x_dtype, n, batch, hidden) : 1;
+    w.grid = batch > 0 ? layer_bwd_grid(x_dtype, n, batch, hidden, aligned) : 1;
     w.dw_off = 0;
     w.scal_off = align256((size_t)w.grid * hidden * sizeof(float));
     w.stage_off = w.scal_off + align256((size_t)w.grid * (n * n + 2 * n) * sizeof(float));
     w.hist_off = w.stage_off + align256(column_sums_stage_floats(hidden) * sizeof(float));
     // Sinkhorn adjoint history
     w.rows_off = w.hist_off + (static_sk_hist(n) ? kStaticSkHistBytes : 0);
-    w.total = w.rows_off + align256(batch > 0 ? layer_bwd_scratch_bytes(x_dtype, n, batch, hidden) : 0);
+    w.total = w.rows_off + align256(batch > 0 ? layer_bwd_scratch_bytes(x_dtype, n, batch, hidden, aligned) : 0);
     return w;
 }
 
 size_t mhc_layer_static_bwd_workspace_size(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype) {
     if (batch < 0 || n < 1 || hidden < 1) return 0;
-    return static_bwd_ws(batch, n, hidden, x_dtype).total;
+    const size_t a = static_bwd_ws(batch, n, hidden, x_dtype, true).total;
+    const size_t u = odd_row_n(n) ? static_bwd_ws(batch, n, hidden, x_dtype, false).total : 0;
+    return a > u ? a : u;
 }
 
-int mhc_layer_static_bwd(const float* grad_out, const void* x, int32_t x_dtype, int32_t weight_dtype,
-                         const float* h_pre, const float* h_post, const float* h_res, const float* saved,
-                         void* grad_x, void* grad_weight, float* grad_h_pre, float* grad_h_post, float* grad_h_res,
-                         void* workspace, size_t workspace_bytes, int64_t batch, int32_t n, int32_t hidden,
-                         int32_t num_iters, float sinkhorn_eps, float rmsnorm_eps, void* stream) {
+static int static_bwd(const float* grad_out, const void* x, int32_t x_dtype, int32_t weight_dtype,
+                      const float* h_pre, const float* h_post, const float* h_res, const float* saved, void* grad_x,
+                      void* grad_weight, float* grad_h_pre, float* grad_h_post, float* grad_h_res, void* workspace,
+                      size_t workspace_bytes, int64_t batch, int32_t n, int32_t hidden, int32_t num_iters,
+                      float sinkhorn_eps, float rmsnorm_eps, void* stream, bool aligned) {
     int st = check_layer_shape("layer_static_bwd", batch, n, hidden, x_dtype, num_iters);
     if (st) return st;
     MHC_REQUIRE(valid_dtype(weight_dtype), "layer_static_bwd: weight_dtype must be F32 or BF16");
@@ -334,7 +337,7 @@ int mhc_layer_static_bwd(const float* grad_out, const void* x, int32_t x_dtype, 
     MHC_REQUIRE(grad_weight && grad_h_pre && grad_h_post && grad_h_res, "layer_static_bwd: null gradient pointer");
     MHC_REQUIRE(batch == 0 || (grad_out && x && grad_x), "layer_static_bwd: null grad_out/x/grad_x");
     hipStream_t s = (hipStream_t)stream;
-    const StaticBwdWs w = static_bwd_ws(batch, n, hidden, x_dtype);
+    const StaticBwdWs w = static_bwd_ws(batch, n, hidden, x_dtype, aligned);
     if (!workspace || workspace_bytes < w.total)
         return fail(MHC_ERR_WORKSPACE, "layer_static_bwd: workspace smaller than mhc_layer_static_bwd_workspace_size()");
     float* dw_part = (float*)((char*)workspace + w.dw_off);
@@ -351,13 +354,23 @@ int mhc_layer_static_bwd(const float* grad_out, const void* x, int32_t x_dtype, 
     } else {
         e = launch_layer_bwd(x_dtype, n, 0, grad_out, x, saved + saved_w_offset(n), saved, 0, grad_x, dw_part,
                              scal_part, w.grid, batch, hidden, rmsnorm_eps, (float*)((char*)workspace + w.rows_off),
-                             s);
+                             s, nullptr, aligned);
     }
     if (e == hipSuccess)
         e = launch_column_finalize(n, weight_dtype, dw_part, rows, hidden, stage, grad_weight, scal_part, rows, h_pre,
                                   h_post, h_res, grad_h_pre, grad_h_post, grad_h_res, num_iters, sinkhorn_eps, s,
                                   static_sk_hist(n) ? (float*)((char*)workspace + w.hist_off) : nullptr);
     return hip_status(e);
+}
+
+int mhc_layer_static_bwd(const float* grad_out, const void* x, int32_t x_dtype, int32_t weight_dtype,
+                         const float* h_pre, const float* h_post, const float* h_res, const float* saved,
+                         void* grad_x, void* grad_weight, float* grad_h_pre, float* grad_h_post, float* grad_h_res,
+                         void* workspace, size_t workspace_bytes, int64_t batch, int32_t n, int32_t hidden,
+                         int32_t num_iters, float sinkhorn_eps, float rmsnorm_eps, void* stream) {
+    return static_bwd(grad_out, x, x_dtype, weight_dtype, h_pre, h_post, h_res, saved, grad_x, grad_weight, grad_h_pre,
+                      grad_h_post, grad_h_res, workspace, workspace_bytes, batch, n, hidden, num_iters, sinkhorn_eps,
+                      rmsnorm_eps, stream, rows_aligned(n, {grad_out, x, grad_x, saved, workspace}));
 }
 
 // ---- allocation-free static backward ---------------------------------------
@@ -401,7 +414,13 @@ int mhc_layer_static_bwd_noalloc(const float* grad_out, const void* x, int32_t x
                                  float sinkhorn_eps, float rmsnorm_eps, void* stream) {
     int st = check_layer_shape("layer_static_bwd_noalloc", batch, n, hidden, x_dtype, num_iters);
     if (st) return st;
-    const size_t need = static_bwd_ws(batch, n, hidden, x_dtype).total;
+    // the generic rows of n = 3, 5, 6, 7 where only theirs fit
+    bool aligned = rows_aligned(n, {grad_out, x, grad_x, saved});
+    size_t need = static_bwd_ws(batch, n, hidden, x_dtype, aligned).total;
+    if (need > kNoAllocScratchBytes && odd_row_n(n)) {
+        aligned = false;
+        need = static_bwd_ws(batch, n, hidden, x_dtype, false).total;
+    }
     if (need > kNoAllocScratchBytes)
         return fail(MHC_ERR_UNSUPPORTED, "layer_static_bwd_noalloc: this shape needs " + std::to_string(need) +
                                              " bytes of scratch, more than the library's " +
@@ -410,9 +429,9 @@ int mhc_layer_static_bwd_noalloc(const float* grad_out, const void* x, int32_t x
     void* ws = nullptr;
     st = scratch_on_current_device(&ws);
     if (st) return st;
-    return mhc_layer_static_bwd(grad_out, x, x_dtype, weight_dtype, h_pre, h_post, h_res, saved, grad_x, grad_weight,
-                                grad_h_pre, grad_h_post, grad_h_res, ws, kNoAllocScratchBytes, batch, n, hidden,
-                                num_iters, sinkhorn_eps, rmsnorm_eps, stream);
+    return static_bwd(grad_out, x, x_dtype, weight_dtype, h_pre, h_post, h_res, saved, grad_x, grad_weight, grad_h_pre,
+                      grad_h_post, grad_h_res, ws, kNoAllocScratchBytes, batch, n, hidden, num_iters, sinkhorn_eps,
+                      rmsnorm_eps, stream, aligned);
 }
 
 // ---- standalone operators ---------------------------------------------------
@@ -931,8 +950,11 @@ int mhc_layer_dynamic_infer(const void* x, int32_t x_dtype, const void* packed, 
 // element below.  Otherwise (n >= 8, rows the channel-loop kernels take,
 // other hidden sizes) x is upcast once (exactly) and dx accumulates in fp32
 // across the kernels.
-static bool dyn_bwd_f32_acc(int32_t n, int32_t hidden, int32_t x_dtype) {
-    return x_dtype == kBF16 && (2 * n + n * n > kProjTile || layer_bwd_is_wide(n, hidden) || hidden % 128 != 0);
+// aligned: rows_aligned() of the call's arrays (without it n = 3 takes the
+// element-wise rows).
+static bool dyn_bwd_f32_acc(int32_t n, int32_t hidden, int32_t x_dtype, bool aligned) {
+    return x_dtype == kBF16 &&
+           (2 * n + n * n > kProjTile || layer_bwd_is_wide(n, hidden) || hidden % 128 != 0 || !aligned);
 }
 
 struct DynBwdWs {
@@ -943,12 +965,12 @@ struct DynBwdWs {
         rows_off, total;
 };
 
-static DynBwdWs dyn_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype) {
+static DynBwdWs dyn_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype, bool aligned) {
     DynBwdWs w{};
     const int64_t np = 2 * n + n * n;
     const int64_t K = (int64_t)n * hidden;
-    w.wdt = dyn_bwd_f32_acc(n, hidden, x_dtype) ? kF32 : x_dtype;
-    w.grid = batch > 0 ? layer_bwd_grid(w.wdt, n, batch, hidden) : 1;
+    w.wdt = dyn_bwd_f32_acc(n, hidden, x_dtype, aligned) ? kF32 : x_dtype;
+    w.grid = batch > 0 ? layer_bwd_grid(w.wdt, n, batch, hidden, aligned) : 1;
     w.cblocks = batch > 0 ? dyn_coef_bwd_blocks(n, batch) : 1;
     w.tiles = batch > 0 ? proj_bwd_tiles(w.wdt, batch, (int64_t)n * hidden) : 1;
     size_t o = 0;
@@ -975,14 +997,20 @@ static DynBwdWs dyn_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_d
     // region dyn_coef_gen_hist_bytes sizes for the batch)
     w.hist_off = o;
     o += n >= 16 && !generic_layer_n(n) && batch > 0 ? kSkHistBytes : align256(dyn_coef_gen_hist_bytes(n, batch));
-    w.rows_off = o; o += align256(batch > 0 ? layer_bwd_scratch_bytes(w.wdt, n, batch, hidden) : 0);
+    w.rows_off = o; o += align256(batch > 0 ? layer_bwd_scratch_bytes(w.wdt, n, batch, hidden, aligned) : 0);
     w.total = o;
     return w;
 }
 
+static size_t dyn_bwd_ws_bytes(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype) {
+    const size_t a = dyn_bwd_ws(batch, n, hidden, x_dtype, true).total;
+    const size_t u = odd_row_n(n) ? dyn_bwd_ws(batch, n, hidden, x_dtype, false).total : 0;
+    return a > u ? a : u;
+}
+
 size_t mhc_layer_dynamic_bwd_workspace_size(int64_t batch, int32_t n, int32_t hidden, int32_t x_dtype) {
     if (batch < 0 || n < 1 || hidden < 1) return 0;
-    return dyn_bwd_ws(batch, n, hidden, x_dtype).total;
+    return dyn_bwd_ws_bytes(batch, n, hidden, x_dtype);
 }
 
 int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype, int32_t weight_dtype,
@@ -1000,7 +1028,8 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
                 "layer_dynamic_bwd: null parameter pointer");
     MHC_REQUIRE(grad_weight && grad_phi && grad_alpha && grad_b, "layer_dynamic_bwd: null gradient pointer");
     MHC_REQUIRE(batch == 0 || (grad_out && x && grad_x), "layer_dynamic_bwd: null grad_out/x/grad_x");
-    const DynBwdWs w = dyn_bwd_ws(batch, n, hidden, x_dtype);
+    const bool aligned = rows_aligned(n, {grad_out, x, grad_x, saved, workspace});
+    const DynBwdWs w = dyn_bwd_ws(batch, n, hidden, x_dtype, aligned);
     if (!workspace || workspace_bytes < w.total)
         return fail(MHC_ERR_WORKSPACE, "layer_dynamic_bwd: workspace smaller than mhc_layer_dynamic_bwd_workspace_size()");
     if (n >= 16 && !generic_layer_n(n) && batch > 0 && dyn_coef_bwd_hist_slots(n, batch, num_iters) < 1)
@@ -1036,7 +1065,7 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
         if (w.wdt != x_dtype) e = launch_weight_f32(x, x_dtype, batch * K, xw, s);
         if (e == hipSuccess)
             e = launch_layer_bwd(w.wdt, n, 1, grad_out, xk, w32, saved + d.coef_off, np, dxk, dw_part, scal, w.grid,
-                                 batch, hidden, rmsnorm_eps, (float*)(ws + w.rows_off), s, pscale);
+                                 batch, hidden, rmsnorm_eps, (float*)(ws + w.rows_off), s, pscale, aligned);
         if (e == hipSuccess)
             e = launch_dyn_coef_bwd(n, scal, saved + d.coef_off, saved + d.p_off, saved + d.rh_off, batch, K,
                                     alpha_pre, alpha_post, alpha_res, b_res, dp, stok, cpart, num_iters, sinkhorn_eps,
@@ -1145,7 +1174,7 @@ static RefBwdWs ref_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_d
     w.small_off = 256;
     w.saved_off = w.small_off + align256((size_t)(3 + np) * sizeof(float));
     w.work_off = w.saved_off + align256(dyn_saved(batch, n, hidden).total * sizeof(float));
-    size_t work = dyn_bwd_ws(batch, n, hidden, x_dtype).total;
+    size_t work = dyn_bwd_ws_bytes(batch, n, hidden, x_dtype);
     const size_t proj = proj_fwd_ws(batch, K, np).total;
     if (proj > work) work = proj;
     w.gphi_off = w.work_off + align256(work);

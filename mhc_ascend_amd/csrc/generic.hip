@@ -1,6 +1,6 @@
 // Kernels for expansion rates with no compiled instantiation: any n in
-// 1..64 outside {2, 4, 8, 16, 32} for the layer, outside {1, 2, 4, 8, 16, 32}
-// for the stream operators.  The reference takes n at run time up to
+// 1..64 outside {2..8, 16, 32} for the layer (and n = 3, 5, 6, 7 past
+// kWideMaxC channels), outside {1..8, 16, 32} for the stream operators.  The reference takes n at run time up to
 // MAX_EXPANSION_RATE = 64 (mhc_types.h:68, stream_ops.cpp:198-208,
 // sinkhorn_knopp.cpp:575-617); here the rates the paper uses
 // (benchmark.py:302-310) and their powers of two keep their fixed-n kernels
@@ -45,7 +45,7 @@ bool generic_layer_n(int n) {
     return n >= 1 && n <= kGenMaxN && !(n == 2 || n == 4 || n == 8 || n == 16 || n == 32);
 }
 bool generic_ops_n(int n) {
-    return n >= 1 && n <= kGenMaxN && !(n == 1 || n == 2 || n == 4 || n == 8 || n == 16 || n == 32);
+    return n > 8 && n <= kGenMaxN && n != 16 && n != 32;
 }
 
 #define MHC_GEN_NM(n, ...)                     \

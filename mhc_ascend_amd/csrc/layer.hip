@@ -845,7 +845,11 @@ hipError_t launch_fill_zero_carry(float* p0, int64_t n0, float* p1, int64_t n1, 
 #define MHC_DISPATCH_N(n, ...)                                   \
     switch (n) {                                                 \
         case 2: { constexpr int N_ = 2; __VA_ARGS__; break; }    \
+        case 3: { constexpr int N_ = 3; __VA_ARGS__; break; }    \
         case 4: { constexpr int N_ = 4; __VA_ARGS__; break; }    \
+        case 5: { constexpr int N_ = 5; __VA_ARGS__; break; }    \
+        case 6: { constexpr int N_ = 6; __VA_ARGS__; break; }    \
+        case 7: { constexpr int N_ = 7; __VA_ARGS__; break; }    \
         case 8: { constexpr int N_ = 8; __VA_ARGS__; break; }    \
         default: return hipErrorInvalidValue;                    \
     }
@@ -932,7 +936,11 @@ static const void* pick_fwd(int x_dtype, int out_dtype, int n, int vpt) {
     }
     switch (n) {
         case 2: { MHC_FWD_N(2); break; }
+        case 3: { MHC_FWD_N(3); break; }
         case 4: { MHC_FWD_N(4); break; }
+        case 5: { MHC_FWD_N(5); break; }
+        case 6: { MHC_FWD_N(6); break; }
+        case 7: { MHC_FWD_N(7); break; }
         case 8: { MHC_FWD_N(8); break; }
         default: break;
     }
@@ -949,7 +957,11 @@ static const void* pick_bwd(int x_dtype, int n, int vpt, int mode, bool pf) {
     const bool bf = x_dtype == kBF16;
     switch (n) {
         case 2: { if (bf) { MHC_BWD_FN(bf16_t, 2); } else { MHC_BWD_FN(float, 2); } break; }
+        case 3: { if (bf) { MHC_BWD_FN(bf16_t, 3); } else { MHC_BWD_FN(float, 3); } break; }
         case 4: { if (bf) { MHC_BWD_FN(bf16_t, 4); } else { MHC_BWD_FN(float, 4); } break; }
+        case 5: { if (bf) { MHC_BWD_FN(bf16_t, 5); } else { MHC_BWD_FN(float, 5); } break; }
+        case 6: { if (bf) { MHC_BWD_FN(bf16_t, 6); } else { MHC_BWD_FN(float, 6); } break; }
+        case 7: { if (bf) { MHC_BWD_FN(bf16_t, 7); } else { MHC_BWD_FN(float, 7); } break; }
         case 8: { if (bf) { MHC_BWD_FN(bf16_t, 8); } else { MHC_BWD_FN(float, 8); } break; }
         default: break;
     }
@@ -977,8 +989,20 @@ static bool use_prefetch(const RowTiling& t) { return t.threads <= 256; }
 // chunk that fits their row state; everything else runs the channel-loop
 // kernels of wide.hip.
 static RowTiling fwd_tiling(int64_t C, int n) {
-    if (n > 8 || generic_layer_n(n)) return RowTiling{0, 0};
+    if (n > 8 || (generic_layer_n(n) && !odd_row_n(n))) return RowTiling{0, 0};
     return choose_row_tiling(C, kLayerWC, n, 512);
+}
+
+// The row kernels a launch runs on, from its register tiling (vpt 0: none
+// fits) and the alignment of its arrays.  n = 3, 5, 6, 7 ran on the generic
+// kernels, which walk the row 2-4 times with the mixing staged through LDS:
+// n = 6, 2047 x 1040, dynamic with bf16 x (fp32 rows in the backward): forward
+// 40.6 -> 16.0 us, backward with its dM kernel 249 -> 49.4 us on register rows.
+enum class RowPath { kRegs, kWide, kGen };
+static RowPath row_path(const RowTiling& t, int n, int64_t C, bool aligned) {
+    if (t.vpt > 0 && (aligned || !odd_row_n(n))) return RowPath::kRegs;
+    if (odd_row_n(n)) return wide_supported(n, C) ? RowPath::kWide : RowPath::kGen;
+    return generic_layer_n(n) ? RowPath::kGen : RowPath::kWide;
 }
 
 bool layer_fwd_is_wide(int n, int64_t C) { return fwd_tiling(C, n).vpt <= 0; }
@@ -987,10 +1011,11 @@ hipError_t launch_layer_fwd(int x_dtype, int n, const void* x, const float* w, c
                             int64_t coef_stride, void* out, int out_dtype, float* rms_out, int64_t B, int64_t C,
                             float eps, hipStream_t s, int64_t rms_scratch) {
     if (B == 0) return hipSuccess;
-    if (generic_layer_n(n))
-        return launch_gen_layer_fwd(x_dtype, out_dtype, n, x, w, coef, coef_stride, out, rms_out, B, C, eps, s);
     const RowTiling t = fwd_tiling(C, n);
-    if (t.vpt <= 0)
+    const RowPath path = row_path(t, n, C, rows_aligned(n, {x, w, out}));
+    if (path == RowPath::kGen)
+        return launch_gen_layer_fwd(x_dtype, out_dtype, n, x, w, coef, coef_stride, out, rms_out, B, C, eps, s);
+    if (path == RowPath::kWide)
         return launch_wide_fwd(x_dtype, out_dtype, n, x, w, coef, coef_stride, out, rms_out, B, C, eps, s, rms_scratch);
     const void* fn = pick_fwd(x_dtype, out_dtype, n, t.vpt);
     if (!fn) return hipErrorInvalidValue;
@@ -1019,7 +1044,7 @@ hipError_t launch_layer_static_fwd(int x_dtype, int n, const void* x, const void
                                    int iters, float sk_eps, float* out, float* rms_out, int64_t B, int64_t C,
                                    float eps, hipStream_t s) {
     const RowTiling t = fwd_tiling(C, n);
-    if (t.vpt <= 0 || n > 8) return hipErrorInvalidValue;
+    if (t.vpt <= 0 || n > 8 || !rows_aligned(n, {x, weight, saved, out})) return hipErrorInvalidValue;
     if (B == 0) {
         // no tokens: the saved state alone (the backward still needs it)
         return launch_static_coef(n, h_pre, h_post, h_res, weight, w_dtype, C, saved, iters, sk_eps, s);
@@ -1040,7 +1065,11 @@ hipError_t launch_layer_static_fwd(int x_dtype, int n, const void* x, const void
     }
     switch (n) {
         case 2: { MHC_SF_N(2); break; }
+        case 3: { MHC_SF_N(3); break; }
         case 4: { MHC_SF_N(4); break; }
+        case 5: { MHC_SF_N(5); break; }
+        case 6: { MHC_SF_N(6); break; }
+        case 7: { MHC_SF_N(7); break; }
         case 8: { MHC_SF_N(8); break; }
         default: break;
     }
@@ -1065,7 +1094,7 @@ hipError_t launch_layer_static_fwd(int x_dtype, int n, const void* x, const void
 // 512-lane form had been the faster one).
 static RowTiling bwd_tiling(int64_t C, int n, int x_dtype = kF32) {
     (void)x_dtype;
-    if (n > 8 || generic_layer_n(n)) return RowTiling{0, 0};
+    if (n > 8 || (generic_layer_n(n) && !odd_row_n(n))) return RowTiling{0, 0};
     return with_min_threads(choose_row_tiling(C, kLayerWC, 2 * n, 256), 2 + n * n + 3 * n);
 }
 
@@ -1076,31 +1105,34 @@ int layer_bwd_part_groups(int x_dtype, int n, int64_t C) {
     return t.vpt > 0 ? t.threads / 32 : 0;
 }
 
-int layer_bwd_grid(int x_dtype, int n, int64_t B, int64_t C) {
-    if (generic_layer_n(n)) return gen_layer_bwd_grid(B);
+int layer_bwd_grid(int x_dtype, int n, int64_t B, int64_t C, bool aligned) {
     const RowTiling t = bwd_tiling(C, n, x_dtype);
-    if (t.vpt <= 0) return wide_bwd_grid(x_dtype, n, B, C);
+    const RowPath path = row_path(t, n, C, aligned);
+    if (path == RowPath::kGen) return gen_layer_bwd_grid(B);
+    if (path == RowPath::kWide) return wide_bwd_grid(x_dtype, n, B, C);
     return persistent_grid(pick_bwd(x_dtype, n, t.vpt, 0, use_prefetch(t)), t.threads, B);
 }
 
-size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C) {
-    if (generic_layer_n(n)) return gen_layer_bwd_scratch_bytes(B, C);
-    return bwd_tiling(C, n, x_dtype).vpt <= 0 ? wide_bwd_scratch_bytes(n, B, C) : 0;
+size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C, bool aligned) {
+    const RowPath path = row_path(bwd_tiling(C, n, x_dtype), n, C, aligned);
+    if (path == RowPath::kGen) return gen_layer_bwd_scratch_bytes(B, C);
+    return path == RowPath::kWide ? wide_bwd_scratch_bytes(n, B, C) : 0;
 }
 
 hipError_t launch_layer_bwd(int x_dtype, int n, int mode, const float* g, const void* x, const float* w,
                             const float* coef, int64_t coef_stride, void* dx, float* dw_part, float* scal_out,
                             int grid, int64_t B, int64_t C, float eps, float* scratch, hipStream_t s,
-                            int32_t* dx_scale) {
-    if (generic_layer_n(n)) {
+                            int32_t* dx_scale, bool aligned) {
+    const RowTiling t = bwd_tiling(C, n, x_dtype);
+    const RowPath path = row_path(t, n, C, aligned);
+    if (path == RowPath::kGen) {
         // the generic kernels write a full-precision stream part only for
         // fp32 x; the dynamic entries send bf16 x through fp32 accumulation
         if (mode == 1 && x_dtype == kBF16) return hipErrorInvalidValue;
         return launch_gen_layer_bwd(x_dtype, n, mode, g, x, w, coef, coef_stride, dx, dw_part, scal_out, grid, B, C,
                                     eps, scratch, s);
     }
-    const RowTiling t = bwd_tiling(C, n, x_dtype);
-    if (t.vpt <= 0) {
+    if (path == RowPath::kWide) {
         // the channel-loop kernels write a bf16 stream part; the dynamic
         // entries send bf16 x there through fp32 accumulation instead
         if (mode == 1 && x_dtype == kBF16) return hipErrorInvalidValue;
@@ -1189,7 +1221,7 @@ hipError_t launch_column_finalize(int n, int w_dtype, const float* part, int row
                                   void* dw, const float* scal_part, int scal_rows, const float* h_pre,
                                   const float* h_post, const float* h_res, float* d_h_pre, float* d_h_post,
                                   float* d_h_res, int iters, float sk_eps, hipStream_t s, float* sk_hist) {
-    if (n > 0 && generic_layer_n(n)) {
+    if (n > 0 && generic_layer_n(n) && !odd_row_n(n)) {
         hipError_t e = launch_column_finalize(0, w_dtype, part, rows, cols, stage, dw, nullptr, 0, nullptr, nullptr,
                                               nullptr, nullptr, nullptr, nullptr, 0, 0.f, s);
         if (e != hipSuccess) return e;

@@ -8,6 +8,7 @@
 #endif
 #include <stdint.h>
 #include <stddef.h>
+#include <initializer_list>
 
 namespace mhc {
 
@@ -76,12 +77,24 @@ inline hipError_t mhc_launch_kernel(const void* fn, dim3 grid, dim3 block, void*
 
 // ---- generic.hip -----------------------------------------------------------
 // Expansion rates without a compiled instantiation (n <= kGenMaxN): the
-// layer's are n outside {2, 4, 8, 16, 32}, the stream operators' n outside
-// {1, 2, 4, 8, 16, 32}.  The layer launchers of layer.hip and dynamic.hip
+// layer's are n outside {2, 4, 8, 16, 32} (odd_row_n below: not at every
+// shape), the stream operators' n outside {1..8, 16, 32}.  The layer launchers of layer.hip and dynamic.hip
 // and the operator launchers of ops.hip route these n here themselves.
 constexpr int kGenMaxN = 64;
 bool generic_layer_n(int n);
 bool generic_ops_n(int n);
+// n = 3, 5, 6, 7 have the fixed-n row kernels too (register rows, and the
+// channel-loop rows up to kWideMaxC channels).  The register rows are taken
+// on 16-byte aligned arrays only; the channel-loop and generic kernels are
+// element-wise and take any alignment.
+inline bool odd_row_n(int n) { return n == 3 || (n >= 5 && n <= 7); }
+inline bool rows_aligned(int n, std::initializer_list<const void*> ps) {
+    if (!odd_row_n(n)) return true;
+    for (const void* p : ps) {
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+    }
+    return true;
+}
 hipError_t launch_gen_static_coef(int n, const float* h_pre, const float* h_post, const float* h_res,
                                   const void* weight, int w_dtype, int64_t C, float* saved, int iters, float sk_eps,
                                   hipStream_t s);
@@ -145,12 +158,13 @@ hipError_t launch_layer_fwd(int x_dtype, int n, const void* x, const float* w, c
 hipError_t launch_layer_bwd(int x_dtype, int n, int mode, const float* g, const void* x, const float* w,
                             const float* coef, int64_t coef_stride, void* dx, float* dw_part, float* scal_out,
                             int grid, int64_t B, int64_t C, float eps, float* scratch, hipStream_t s,
-                            int32_t* dx_scale = nullptr);
-int layer_bwd_grid(int x_dtype, int n, int64_t B, int64_t C);
+                            int32_t* dx_scale = nullptr, bool aligned = true);
+// aligned: rows_aligned(n, {g, x, dx}) of the launch that the grid (scratch) is for.
+int layer_bwd_grid(int x_dtype, int n, int64_t B, int64_t C, bool aligned = true);
 // Scale groups per token row of the mode-1 stream part (one per half
 // wave of the register-row kernel; 0 when the channel-loop kernels run).
 int layer_bwd_part_groups(int x_dtype, int n, int64_t C);
-size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C);
+size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C, bool aligned = true);
 // Whether the layer forward / backward of (n, C) runs the channel-loop
 // kernels of wide.hip rather than the register rows.
 bool layer_fwd_is_wide(int n, int64_t C);
@@ -183,7 +197,7 @@ hipError_t launch_column_finalize(int n, int w_dtype, const float* part, int row
                                   float* d_h_res, int iters, float sk_eps, hipStream_t s, float* sk_hist = nullptr);
 
 // ---- wide.hip --------------------------------------------------------------
-// Channel-loop layer kernels (any C up to kWideMaxC; n in {2, 4, 8, 16, 32}):
+// Channel-loop layer kernels (any C up to kWideMaxC; n in {2..8, 16, 32}):
 // used for n > 8 and where the register rows do not fit C.  The backward's
 // dw partial of a workgroup sits in LDS (C floats).
 constexpr int kWideMaxC = 12288;

@@ -440,10 +440,23 @@ hipError_t launch_compute_rms(int dt, const void* x, float* rms, int64_t B, int6
     switch (n) {                                                 \
         case 1: { constexpr int N_ = 1; __VA_ARGS__; break; }    \
         case 2: { constexpr int N_ = 2; __VA_ARGS__; break; }    \
+        case 3: { constexpr int N_ = 3; __VA_ARGS__; break; }    \
         case 4: { constexpr int N_ = 4; __VA_ARGS__; break; }    \
+        case 5: { constexpr int N_ = 5; __VA_ARGS__; break; }    \
+        case 6: { constexpr int N_ = 6; __VA_ARGS__; break; }    \
+        case 7: { constexpr int N_ = 7; __VA_ARGS__; break; }    \
         case 8: { constexpr int N_ = 8; __VA_ARGS__; break; }    \
         default: return hipErrorInvalidValue;                    \
     }
+
+// The stream operators' register rows (vpt 0: the channel-loop kernels run):
+// n <= 8, rows that fit, and for n = 3, 5, 6, 7 aligned arrays
+// (rows_aligned).  A row per workgroup in registers against the generic
+// kernels' staged mixing, n = 6, 2047 x 1040 bf16: MEASURED_OPS_N6.
+static RowTiling ops_tiling(int dt, int n, int64_t C, int arrays, int pref, std::initializer_list<const void*> ps) {
+    if (n > 8 || !rows_aligned(n, ps)) return RowTiling{0, 0};
+    return choose_row_tiling(C, dt == kBF16 ? 8 : 4, arrays, pref);
+}
 
 hipError_t launch_aggregate_fwd(int dt, int n, const void* x, const float* H, int64_t hs, void* out, float* h_act,
                                 int64_t B, int64_t C, hipStream_t s) {
@@ -454,7 +467,7 @@ hipError_t launch_aggregate_fwd(int dt, int n, const void* x, const float* H, in
         timing_end(tok, s);
         return e;
     }
-    const RowTiling t = n > 8 ? RowTiling{0, 0} : choose_row_tiling(C, dt == kBF16 ? 8 : 4, n + 1, 512);
+    const RowTiling t = ops_tiling(dt, n, C, n + 1, 512, {x, out});
     const int tok = timing_begin("aggregate_fwd", s);
     if (t.vpt <= 0) {
         const hipError_t e = launch_wide_aggregate_fwd(dt, n, x, H, hs, out, h_act, B, C, s);
@@ -485,7 +498,7 @@ hipError_t launch_aggregate_bwd(int dt, int n, const void* g, const void* x, con
         timing_end(tok, s);
         return e;
     }
-    const RowTiling t = n > 8 ? RowTiling{0, 0} : choose_row_tiling(C, dt == kBF16 ? 8 : 4, n + 1, 512);
+    const RowTiling t = ops_tiling(dt, n, C, n + 1, 512, {g, x, gx});
     const int tok = timing_begin("aggregate_bwd", s);
     if (t.vpt <= 0) {
         const hipError_t e = launch_wide_aggregate_bwd(dt, n, g, x, h_act, hs, gx, gh_act, gh_raw, B, C, s);
@@ -514,7 +527,7 @@ hipError_t launch_distribute_fwd(int dt, int n, const void* y, const float* H, i
                                  hipStream_t s) {
     if (B == 0) return hipSuccess;
     if (generic_ops_n(n)) return launch_gen_distribute_fwd(dt, n, y, H, hs, M, ms, x, out, h_act, B, C, s);
-    const RowTiling t = n > 8 ? RowTiling{0, 0} : choose_row_tiling(C, dt == kBF16 ? 8 : 4, n + 1, 512);
+    const RowTiling t = ops_tiling(dt, n, C, n + 1, 512, {y, x, out});
     const int tok = timing_begin("distribute_fwd", s);
     if (t.vpt <= 0) {
         const hipError_t e = launch_wide_distribute_fwd(dt, n, y, H, hs, M, ms, x, out, h_act, B, C, s);
@@ -536,8 +549,7 @@ hipError_t launch_distribute_bwd(int dt, int n, const float* g, const void* x, c
     if (generic_ops_n(n))
         return launch_gen_distribute_bwd(dt, n, g, x, y, M, ms, h_act, hs, gx, gy, gM, gh_act, gh_raw, B, C, s);
     // the block hands one of the n*n + n row sums to each thread
-    const RowTiling t =
-        n > 8 ? RowTiling{0, 0} : with_min_threads(choose_row_tiling(C, dt == kBF16 ? 8 : 4, 2 * n + 1), n * n + n);
+    const RowTiling t = with_min_threads(ops_tiling(dt, n, C, 2 * n + 1, 256, {g, x, y, gx, gy}), n * n + n);
     const int tok = timing_begin("distribute_bwd", s);
     if (t.vpt <= 0) {
         const hipError_t e =

@@ -952,7 +952,11 @@ __global__ __launch_bounds__(kWideThreads) void wide_distribute_bwd_kernel(
 #define MHC_WIDE_N(n, ...)                                        \
     switch (n) {                                                  \
         case 2: { constexpr int N_ = 2; __VA_ARGS__; break; }     \
+        case 3: { constexpr int N_ = 3; __VA_ARGS__; break; }     \
         case 4: { constexpr int N_ = 4; __VA_ARGS__; break; }     \
+        case 5: { constexpr int N_ = 5; __VA_ARGS__; break; }     \
+        case 6: { constexpr int N_ = 6; __VA_ARGS__; break; }     \
+        case 7: { constexpr int N_ = 7; __VA_ARGS__; break; }     \
         case 8: { constexpr int N_ = 8; __VA_ARGS__; break; }     \
         case 16: { constexpr int N_ = 16; __VA_ARGS__; break; }   \
         case 32: { constexpr int N_ = 32; __VA_ARGS__; break; }   \
@@ -960,7 +964,7 @@ __global__ __launch_bounds__(kWideThreads) void wide_distribute_bwd_kernel(
     }
 
 bool wide_supported(int n, int64_t C) {
-    return (n == 2 || n == 4 || n == 8 || n == 16 || n == 32) && C >= 1 && C <= kWideMaxC;
+    return ((n >= 2 && n <= 8) || n == 16 || n == 32) && C >= 1 && C <= kWideMaxC;
 }
 
 hipError_t launch_wide_fwd(int x_dtype, int out_dtype, int n, const void* x, const float* w, const float* coef,
@@ -1133,7 +1137,11 @@ hipError_t launch_wide_bwd(int x_dtype, int n, int mode, const float* g, const v
     switch (n) {                                                  \
         case 1: { constexpr int N_ = 1; __VA_ARGS__; break; }     \
         case 2: { constexpr int N_ = 2; __VA_ARGS__; break; }     \
+        case 3: { constexpr int N_ = 3; __VA_ARGS__; break; }     \
         case 4: { constexpr int N_ = 4; __VA_ARGS__; break; }     \
+        case 5: { constexpr int N_ = 5; __VA_ARGS__; break; }     \
+        case 6: { constexpr int N_ = 6; __VA_ARGS__; break; }     \
+        case 7: { constexpr int N_ = 7; __VA_ARGS__; break; }     \
         case 8: { constexpr int N_ = 8; __VA_ARGS__; break; }     \
         case 16: { constexpr int N_ = 16; __VA_ARGS__; break; }   \
         case 32: { constexpr int N_ = 32; __VA_ARGS__; break; }   \
