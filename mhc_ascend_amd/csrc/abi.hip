@@ -69,6 +69,38 @@ int device_cu_count() {
     return cache[dev];
 }
 
+// Resident workgroups of a kernel per CU, asked of the runtime once per
+// (device, kernel, launch shape): the entries size their grids and workspaces
+// with it several times per call.  At most kOccEntries are kept.
+int occupancy_per_cu(const void* fn, int threads, size_t lds) {
+    struct Entry {
+        int dev, threads;
+        const void* fn;
+        size_t lds;
+        int per_cu;
+    };
+    constexpr size_t kOccEntries = 512;
+    static std::mutex mu;
+    static std::vector<Entry> cache;
+    int dev = 0;
+    if (fn == nullptr || hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    std::lock_guard<std::mutex> lk(mu);
+    for (const Entry& e : cache) {
+        if (e.fn == fn && e.threads == threads && e.lds == lds && e.dev == dev) return e.per_cu;
+    }
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds) != hipSuccess || per_cu < 1) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    if (cache.size() >= kOccEntries) cache.clear();
+    cache.push_back(Entry{dev, threads, fn, lds, per_cu});
+    return per_cu;
+}
+
 // The row kernels are compiled with __launch_bounds__(512) and chunk counts
 // VPT in {1, 2, 4, 8}; at most kRowStateBudget floats of row state stay live
 // per thread so that a 512-lane workgroup fits in 256 VGPRs without spilling.  The

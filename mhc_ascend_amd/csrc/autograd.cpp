@@ -44,6 +44,18 @@ using torch::autograd::tensor_list;
     X(mhc_layer_dynamic_fwd)                  \
     X(mhc_layer_dynamic_bwd_workspace_size)   \
     X(mhc_layer_dynamic_bwd)                  \
+    X(mhc_layer_dynamic_packed_size)          \
+    X(mhc_layer_dynamic_infer_workspace_size) \
+    X(mhc_layer_dynamic_infer)                \
+    X(mhc_sinkhorn_knopp_fwd)                 \
+    X(mhc_sinkhorn_knopp_bwd)                 \
+    X(mhc_rmsnorm_fwd)                        \
+    X(mhc_rmsnorm_bwd_workspace_size)         \
+    X(mhc_rmsnorm_bwd)                        \
+    X(mhc_stream_aggregate_fwd)               \
+    X(mhc_stream_aggregate_bwd)               \
+    X(mhc_stream_distribute_mix_add_fwd)      \
+    X(mhc_stream_distribute_mix_add_bwd)      \
     X(mhc_wrapper_dynamic_saved_size)         \
     X(mhc_wrapper_dynamic_fwd_workspace_size_for) \
     X(mhc_wrapper_dynamic_fwd)                \
@@ -120,11 +132,49 @@ Tensor layer_x(const char* fn, const Tensor& x) {
 
 Tensor weight(const Tensor& w) { return (storage_dtype(w.scalar_type()) ? w : w.to(at::kFloat)).contiguous(); }
 
-Tensor f32c(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
+Tensor f32c(const Tensor& t) {
+    if (t.scalar_type() == at::kFloat && t.is_contiguous()) return t;
+    return t.to(at::kFloat).contiguous();
+}
 
-// alpha as a 1-element fp32 device tensor (a device pointer: no host sync)
+// alpha as a one-element fp32 device tensor of its own shape (a device
+// pointer: no host sync)
 Tensor scalar_param(const Tensor& a, c10::Device dev) {
-    return a.detach().to(dev, at::kFloat).reshape({1}).contiguous();
+    TORCH_CHECK(a.numel() == 1, "alpha must have one element, got shape ", a.sizes());
+    if (a.device() == dev) return f32c(a);
+    return a.detach().to(dev, at::kFloat).contiguous();
+}
+
+// A contiguous tensor of `sizes` over part of a contiguous buffer, from
+// element `offset` on.
+Tensor part_of(const Tensor& buf, at::IntArrayRef sizes, int64_t offset) {
+    c10::SmallVector<int64_t, 4> strides(sizes.size());
+    int64_t st = 1;
+    for (size_t i = sizes.size(); i-- > 0;) {
+        strides[i] = st;
+        st *= sizes[i] > 0 ? sizes[i] : 1;
+    }
+    return buf.as_strided(sizes, strides, offset);
+}
+
+// Appends the gradients of (phi_pre, phi_post, phi_res, alpha_pre, alpha_post,
+// alpha_res, b_pre, b_post, b_res), in the parameters' shapes, over the
+// entry's three gradient buffers.
+void push_param_grads(tensor_list& out, const at::IntArrayRef (&shapes)[9], int64_t n, const Tensor& gphi,
+                      const Tensor& galpha, const Tensor& gb) {
+    const Tensor* bufs[3] = {&gphi, &galpha, &gb};
+    const int64_t nC = gphi.size(1);
+    const int64_t want[3][3] = {{n * nC, n * nC, n * n * nC}, {1, 1, 1}, {n, n, n * n}};
+    for (int k = 0; k < 3; ++k) {
+        int64_t off = 0;
+        for (int i = 0; i < 3; ++i) {
+            const at::IntArrayRef shape = shapes[3 * k + i];
+            TORCH_CHECK(c10::multiply_integers(shape) == want[k][i], "dynamic layer: parameter of shape ", shape,
+                        " does not match n = ", n);
+            out.push_back(part_of(*bufs[k], shape, off));
+            off += want[k][i];
+        }
+    }
 }
 
 Tensor workspace(size_t nbytes, const Tensor& like) {
@@ -158,9 +208,6 @@ struct StaticLayer : public torch::autograd::Function<StaticLayer> {
               fn);
         ctx->save_for_backward({x, w, hp, hq, hr, saved});
         ctx->saved_data["x_dtype"] = (int64_t)x_in.scalar_type();
-        ctx->saved_data["hp_shape"] = hp_in.sizes().vec();
-        ctx->saved_data["hq_shape"] = hq_in.sizes().vec();
-        ctx->saved_data["hr_shape"] = hr_in.sizes().vec();
         ctx->saved_data["cfg"] = std::vector<double>{(double)iters, sk_eps, rms_eps};
         return out;
     }
@@ -178,7 +225,7 @@ struct StaticLayer : public torch::autograd::Function<StaticLayer> {
         const auto f32 = x.options().dtype(at::kFloat);
         Tensor grad_x = at::empty_like(x);
         Tensor gw = at::empty({C}, w.options());
-        Tensor ghp = at::empty({n}, f32), ghq = at::empty({n}, f32), ghr = at::empty({n, n}, f32);
+        Tensor ghp = at::empty(hp.sizes(), f32), ghq = at::empty(hq.sizes(), f32), ghr = at::empty(hr.sizes(), f32);
         const int xd = dtype_code(x.scalar_type());
         const size_t wsb = lib.mhc_layer_static_bwd_workspace_size(B, (int32_t)n, (int32_t)C, xd);
         Tensor ws = workspace(wsb, x);
@@ -188,14 +235,7 @@ struct StaticLayer : public torch::autograd::Function<StaticLayer> {
                                        (float)cfg[1], (float)cfg[2], stream()),
               fn);
         const auto x_dtype = (at::ScalarType)ctx->saved_data["x_dtype"].toInt();
-        return {grad_x.to(x_dtype),
-                gw,
-                ghp.view(ctx->saved_data["hp_shape"].toIntVector()),
-                ghq.view(ctx->saved_data["hq_shape"].toIntVector()),
-                ghr.view(ctx->saved_data["hr_shape"].toIntVector()),
-                Tensor(),
-                Tensor(),
-                Tensor()};
+        return {grad_x.to(x_dtype), gw, ghp, ghq, ghr, Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -239,12 +279,6 @@ struct DynamicLayer : public torch::autograd::Function<DynamicLayer> {
               fn);
         ctx->save_for_backward({x, w, saved, ph[0], ph[1], ph[2], ap, aq, ar, bp, bq, br});
         ctx->saved_data["x_dtype"] = (int64_t)x_in.scalar_type();
-        std::vector<int64_t> shapes;  // rank, then sizes, of each parameter in argument order
-        for (const Tensor* t : {&pp_in, &pq_in, &pr_in, &ap_in, &aq_in, &ar_in, &bp_in, &bq_in, &br_in}) {
-            shapes.push_back(t->dim());
-            for (int64_t s : t->sizes()) shapes.push_back(s);
-        }
-        ctx->saved_data["shapes"] = shapes;
         ctx->saved_data["cfg"] = std::vector<double>{(double)iters, sk_eps, rms_eps};
         return out;
     }
@@ -274,51 +308,21 @@ struct DynamicLayer : public torch::autograd::Function<DynamicLayer> {
                                         fp(galpha), fp(gb), ws.data_ptr(), wsb, B, (int32_t)n, (int32_t)C,
                                         (int32_t)cfg[0], (float)cfg[1], (float)cfg[2], stream()),
               fn);
-        const auto flat = ctx->saved_data["shapes"].toIntVector();
-        std::vector<std::vector<int64_t>> shp;
-        for (size_t i = 0; i < flat.size();) {
-            const int64_t r = flat[i++];
-            shp.emplace_back(flat.begin() + i, flat.begin() + i + r);
-            i += r;
-        }
         const auto x_dtype = (at::ScalarType)ctx->saved_data["x_dtype"].toInt();
-        return {grad_x.to(x_dtype),
-                gw,
-                gphi.narrow(0, 0, n).view(shp[0]),
-                gphi.narrow(0, n, n).view(shp[1]),
-                gphi.narrow(0, 2 * n, n * n).view(shp[2]),
-                galpha.narrow(0, 0, 1).view(shp[3]),
-                galpha.narrow(0, 1, 1).view(shp[4]),
-                galpha.narrow(0, 2, 1).view(shp[5]),
-                gb.narrow(0, 0, n).view(shp[6]),
-                gb.narrow(0, n, n).view(shp[7]),
-                gb.narrow(0, 2 * n, n * n).view(shp[8]),
-                Tensor(),
-                Tensor(),
-                Tensor()};
+        tensor_list out;
+        out.reserve(14);
+        out.push_back(grad_x.to(x_dtype));
+        out.push_back(gw);
+        push_param_grads(out,
+                         {sv[3].sizes(), sv[4].sizes(), sv[5].sizes(), sv[6].sizes(), sv[7].sizes(), sv[8].sizes(),
+                          sv[9].sizes(), sv[10].sizes(), sv[11].sizes()},
+                         n, gphi, galpha, gb);
+        out.resize(14);
+        return out;
     }
 };
 
 // ---- fused MHCResidualWrapper (layer.py:269-322) ----------------------------
-std::vector<int64_t> flat_shapes(std::initializer_list<const Tensor*> ts) {
-    std::vector<int64_t> v;  // rank, then sizes, of each tensor in order
-    for (const Tensor* t : ts) {
-        v.push_back(t->dim());
-        for (int64_t d : t->sizes()) v.push_back(d);
-    }
-    return v;
-}
-
-std::vector<std::vector<int64_t>> unflat_shapes(const std::vector<int64_t>& flat) {
-    std::vector<std::vector<int64_t>> out;
-    for (size_t i = 0; i < flat.size();) {
-        const int64_t r = flat[i++];
-        out.emplace_back(flat.begin() + i, flat.begin() + i + r);
-        i += r;
-    }
-    return out;
-}
-
 // residual / branch [tokens, hidden] as the kernels read them: residual in
 // fp32 or bf16 (others become fp32), branch in the residual's dtype.
 std::pair<Tensor, Tensor> wrapper_inputs(const char* fn, const Tensor& residual, const Tensor& branch) {
@@ -359,7 +363,6 @@ struct StaticWrapper : public torch::autograd::Function<StaticWrapper> {
               "mhc_wrapper_static_fwd");
         ctx->save_for_backward({r, b, w, hp, hq, hr, saved});
         ctx->saved_data["dtypes"] = std::vector<int64_t>{(int64_t)res_in.scalar_type(), (int64_t)br_in.scalar_type()};
-        ctx->saved_data["shapes"] = flat_shapes({&hp_in, &hq_in, &hr_in});
         ctx->saved_data["cfg"] = std::vector<double>{(double)mode, (double)n, (double)iters, sk_eps, rms_eps};
         return out;
     }
@@ -378,7 +381,8 @@ struct StaticWrapper : public torch::autograd::Function<StaticWrapper> {
         const auto f32 = r.options().dtype(at::kFloat);
         Tensor gr = at::empty_like(r), gb = at::empty_like(b);
         Tensor gw = at::empty({C}, w.options());
-        Tensor ghp = at::empty({n}, f32), ghq = at::empty({n}, f32), ghr = at::empty({n, n}, f32);
+        Tensor ghp = at::empty(sv[3].sizes(), f32), ghq = at::empty(sv[4].sizes(), f32),
+               ghr = at::empty(sv[5].sizes(), f32);
         const int dt = dtype_code(r.scalar_type());
         const size_t wsb = lib.mhc_wrapper_static_bwd_workspace_size(T, (int32_t)n, (int32_t)C, dt, mode);
         Tensor ws = workspace(wsb, r);
@@ -388,9 +392,8 @@ struct StaticWrapper : public torch::autograd::Function<StaticWrapper> {
                                          (int32_t)C, (int32_t)cfg[2], (float)cfg[3], (float)cfg[4], stream()),
               "mhc_wrapper_static_bwd");
         const auto dts = ctx->saved_data["dtypes"].toIntVector();
-        const auto shp = unflat_shapes(ctx->saved_data["shapes"].toIntVector());
-        return {gr.to((at::ScalarType)dts[0]), gb.to((at::ScalarType)dts[1]), gw, ghp.view(shp[0]), ghq.view(shp[1]),
-                ghr.view(shp[2]), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        return {gr.to((at::ScalarType)dts[0]), gb.to((at::ScalarType)dts[1]), gw, ghp, ghq, ghr, Tensor(), Tensor(),
+                Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -425,9 +428,10 @@ struct DynamicWrapper : public torch::autograd::Function<DynamicWrapper> {
                                           (float)sk_eps, (float)rms_eps, stream()),
               "mhc_wrapper_dynamic_fwd");
         ctx->save_for_backward({r, b, w, saved, ph[0], ph[1], ph[2], ap, aq, ar, bres});
+        // b_pre and b_post are not read by the backward: their shapes only
+        ctx->saved_data["b_pre"] = bp.sizes().vec();
+        ctx->saved_data["b_post"] = bq.sizes().vec();
         ctx->saved_data["dtypes"] = std::vector<int64_t>{(int64_t)res_in.scalar_type(), (int64_t)br_in.scalar_type()};
-        ctx->saved_data["shapes"] =
-            flat_shapes({&pp_in, &pq_in, &pr_in, &ap_in, &aq_in, &ar_in, &bp_in, &bq_in, &bres_in});
         ctx->saved_data["cfg"] = std::vector<double>{(double)mode, (double)n, (double)iters, sk_eps, rms_eps};
         return out;
     }
@@ -460,26 +464,247 @@ struct DynamicWrapper : public torch::autograd::Function<DynamicWrapper> {
                                           (int32_t)C, (int32_t)cfg[2], (float)cfg[3], (float)cfg[4], stream()),
               "mhc_wrapper_dynamic_bwd");
         const auto dts = ctx->saved_data["dtypes"].toIntVector();
-        const auto shp = unflat_shapes(ctx->saved_data["shapes"].toIntVector());
-        return {gr.to((at::ScalarType)dts[0]),
-                gb.to((at::ScalarType)dts[1]),
-                gw,
-                gphi.narrow(0, 0, n).view(shp[0]),
-                gphi.narrow(0, n, n).view(shp[1]),
-                gphi.narrow(0, 2 * n, n * n).view(shp[2]),
-                galpha.narrow(0, 0, 1).view(shp[3]),
-                galpha.narrow(0, 1, 1).view(shp[4]),
-                galpha.narrow(0, 2, 1).view(shp[5]),
-                gbias.narrow(0, 0, n).view(shp[6]),
-                gbias.narrow(0, n, n).view(shp[7]),
-                gbias.narrow(0, 2 * n, n * n).view(shp[8]),
-                Tensor(),
-                Tensor(),
-                Tensor(),
-                Tensor(),
-                Tensor()};
+        tensor_list out;
+        out.reserve(17);
+        out.push_back(gr.to((at::ScalarType)dts[0]));
+        out.push_back(gb.to((at::ScalarType)dts[1]));
+        out.push_back(gw);
+        const auto bp = ctx->saved_data["b_pre"].toIntVector(), bq = ctx->saved_data["b_post"].toIntVector();
+        push_param_grads(out,
+                         {sv[4].sizes(), sv[5].sizes(), sv[6].sizes(), sv[7].sizes(), sv[8].sizes(), sv[9].sizes(), bp,
+                          bq, sv[10].sizes()},
+                         n, gphi, galpha, gbias);
+        out.resize(17);
+        return out;
     }
 };
+
+// ---- forward-only dynamic layer (ops.py:337-380) ------------------------------
+Tensor dynamic_infer(const Tensor& x_in, const Tensor& packed, const Tensor& ap_in, const Tensor& aq_in,
+                     const Tensor& ar_in, const Tensor& bp_in, const Tensor& bq_in, const Tensor& br_in, int64_t iters,
+                     double sk_eps, double rms_eps, bool out_bf16) {
+    require_bound();
+    const char* fn = "mhc_layer_dynamic_infer";
+    const at::NoGradGuard no_grad;
+    check_device(fn, {&x_in, &packed, &bp_in, &bq_in, &br_in});
+    const at::DeviceGuard guard(x_in.device());
+    const Tensor x = layer_x(fn, x_in);
+    const int64_t B = x.size(0), n = x.size(1), C = x.size(2);
+    TORCH_CHECK(packed.scalar_type() == at::kByte &&
+                    (size_t)packed.numel() >= lib.mhc_layer_dynamic_packed_size((int32_t)n, (int32_t)C),
+                fn, ": packed parameters do not match x [B, n, C]");
+    const Tensor ap = scalar_param(ap_in, x.device()), aq = scalar_param(aq_in, x.device()),
+                 ar = scalar_param(ar_in, x.device());
+    const Tensor bp = f32c(bp_in), bq = f32c(bq_in), br = f32c(br_in);
+    TORCH_CHECK(bp.numel() == n && bq.numel() == n && br.numel() == n * n, fn,
+                ": b_pre/b_post must have n and b_res n*n elements");
+    Tensor out = at::empty({B, n, C}, x.options().dtype(out_bf16 ? at::kBFloat16 : at::kFloat));
+    const size_t wsb = lib.mhc_layer_dynamic_infer_workspace_size(B, (int32_t)n, (int32_t)C);
+    Tensor ws = workspace(wsb, x);
+    check(lib.mhc_layer_dynamic_infer(x.data_ptr(), dtype_code(x.scalar_type()), packed.data_ptr(), fp(ap), fp(aq),
+                                      fp(ar), fp(bp), fp(bq), fp(br), out.data_ptr(),
+                                      out_bf16 ? MHC_DTYPE_BF16 : MHC_DTYPE_F32, ws.data_ptr(), wsb, B, (int32_t)n,
+                                      (int32_t)C, (int32_t)iters, (float)sk_eps, (float)rms_eps, stream()),
+          fn);
+    return out;
+}
+
+// ---- standalone operators (ops.py:32-265) -------------------------------------
+// The same checks, dtypes and error text as the functions of
+// mhc_ascend_amd/native.py; the tensors saved are the caller's own.
+Tensor storage(const Tensor& t) { return (storage_dtype(t.scalar_type()) ? t : t.to(at::kFloat)).contiguous(); }
+
+// A per-token coefficient tensor as (fp32 tensor, batch stride): one that is
+// broadcast over the batch (stride 0) is passed once.
+std::pair<Tensor, int64_t> coef_view(const char* fn, const Tensor& t_in, int64_t B, int64_t per) {
+    const Tensor t = t_in.to(at::kFloat);
+    if (t.dim() >= 2 && t.size(0) == B && t.stride(0) == 0) {
+        const Tensor one = t.select(0, 0).contiguous();
+        TORCH_CHECK(one.numel() == per, fn, ": coefficient shape ", t.sizes(), " does not match n");
+        return {one, 0};
+    }
+    const Tensor c = t.contiguous();
+    TORCH_CHECK(c.numel() == B * per, fn, ": coefficient shape ", t.sizes(), " does not match [B=", B, ", ", per, "]");
+    return {c, per};
+}
+
+struct Sinkhorn : public torch::autograd::Function<Sinkhorn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& inp, int64_t iters, double eps) {
+        check_device("sinkhorn_knopp_fwd", {&inp});
+        const at::DeviceGuard guard(inp.device());
+        TORCH_CHECK(inp.dim() == 3, "Input must be 3D tensor [B, M, N]");
+        TORCH_CHECK(inp.size(1) == inp.size(2), "Sinkhorn-Knopp requires square matrices (M == N), got M=",
+                    inp.size(1), ", N=", inp.size(2));
+        TORCH_CHECK(inp.scalar_type() == at::kFloat, "inp must be float32");
+        const Tensor a = inp.contiguous();
+        Tensor out = at::empty_like(a);
+        check(lib.mhc_sinkhorn_knopp_fwd(fp(a), fp(out), a.size(0), (int32_t)a.size(1), (int32_t)iters, (float)eps,
+                                         stream()),
+              "mhc_sinkhorn_knopp_fwd");
+        ctx->save_for_backward({inp, out});
+        ctx->saved_data["iters"] = iters;
+        ctx->saved_data["eps"] = eps;
+        return out;
+    }
+
+    static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor g = f32c(grads[0]);
+        check_device("sinkhorn_knopp_bwd", {&g, &sv[0]});
+        const at::DeviceGuard guard(g.device());
+        TORCH_CHECK(g.sizes() == sv[0].sizes(), "grad_out shape must match inp");
+        const Tensor a = sv[0].contiguous();
+        Tensor gi = at::empty_like(a);
+        check(lib.mhc_sinkhorn_knopp_bwd(fp(g), fp(a), nullptr, fp(gi), a.size(0), (int32_t)a.size(1),
+                                         (int32_t)ctx->saved_data["iters"].toInt(),
+                                         (float)ctx->saved_data["eps"].toDouble(), stream()),
+              "mhc_sinkhorn_knopp_bwd");
+        return {gi, Tensor(), Tensor()};
+    }
+};
+
+struct RmsNorm : public torch::autograd::Function<RmsNorm> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& inp, const Tensor& w_in, double eps) {
+        check_device("rmsnorm_fwd", {&inp, &w_in});
+        const at::DeviceGuard guard(inp.device());
+        TORCH_CHECK(inp.dim() == 2, "Input must be 2D tensor [B, C]");
+        const Tensor x = storage(inp);
+        const int64_t B = x.size(0), C = x.size(1);
+        TORCH_CHECK(w_in.numel() == C, "weight must have C elements");
+        const Tensor w = f32c(w_in);
+        Tensor out = at::empty_like(x);
+        Tensor rms = at::empty({B}, x.options().dtype(at::kFloat));
+        check(lib.mhc_rmsnorm_fwd(x.data_ptr(), dtype_code(x.scalar_type()), fp(w), out.data_ptr(), fp(rms), B,
+                                  (int32_t)C, (float)eps, stream()),
+              "mhc_rmsnorm_fwd");
+        ctx->save_for_backward({inp, w_in, rms});
+        return out;
+    }
+
+    static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &inp = sv[0], &w_in = sv[1], &rms = sv[2];
+        check_device("rmsnorm_bwd", {&grads[0], &inp, &w_in, &rms});
+        const at::DeviceGuard guard(inp.device());
+        const Tensor x = storage(inp);
+        const int64_t B = x.size(0), C = x.size(1);
+        const Tensor g = grads[0].to(x.scalar_type()).contiguous();
+        TORCH_CHECK(g.sizes() == x.sizes(), "grad_out shape must match inp");
+        const Tensor w = f32c(w_in);
+        Tensor gx = at::empty_like(x);
+        Tensor gw = at::empty({C}, x.options().dtype(at::kFloat));
+        const int dt = dtype_code(x.scalar_type());
+        const size_t wsb = lib.mhc_rmsnorm_bwd_workspace_size(B, (int32_t)C, dt);
+        Tensor ws = workspace(wsb, x);
+        check(lib.mhc_rmsnorm_bwd(g.data_ptr(), x.data_ptr(), dt, fp(w), fp(rms), gx.data_ptr(), fp(gw), ws.data_ptr(),
+                                  wsb, B, (int32_t)C, stream()),
+              "mhc_rmsnorm_bwd");
+        return {gx.to(inp.scalar_type()), gw, Tensor()};
+    }
+};
+
+struct Aggregate : public torch::autograd::Function<Aggregate> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& inp, const Tensor& h_in) {
+        const char* fn = "stream_aggregate_fwd";
+        check_device(fn, {&inp, &h_in});
+        const at::DeviceGuard guard(inp.device());
+        TORCH_CHECK(inp.dim() == 3, "Input must be 3D tensor [B, n, C]");
+        const Tensor x = storage(inp);
+        const int64_t B = x.size(0), n = x.size(1), C = x.size(2);
+        const auto [h, hs] = coef_view(fn, h_in, B, n);
+        Tensor out = at::empty({B, C}, x.options());
+        Tensor act = at::empty({B, n}, x.options().dtype(at::kFloat));
+        check(lib.mhc_stream_aggregate_fwd(x.data_ptr(), dtype_code(x.scalar_type()), fp(h), hs, out.data_ptr(),
+                                           fp(act), B, (int32_t)n, (int32_t)C, stream()),
+              "mhc_stream_aggregate_fwd");
+        ctx->save_for_backward({inp, act});
+        return out;
+    }
+
+    static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &inp = sv[0], &act = sv[1];
+        check_device("stream_aggregate_bwd", {&grads[0], &inp, &act});
+        const at::DeviceGuard guard(inp.device());
+        const Tensor x = storage(inp);
+        const int64_t B = x.size(0), n = x.size(1), C = x.size(2);
+        const Tensor g = grads[0].to(x.scalar_type()).contiguous();
+        TORCH_CHECK(g.dim() == 2 && g.size(0) == B && g.size(1) == C, "grad_out must be [B, C]");
+        Tensor gx = at::empty_like(x);
+        Tensor graw = at::empty({B, n}, act.options());
+        check(lib.mhc_stream_aggregate_bwd(g.data_ptr(), x.data_ptr(), dtype_code(x.scalar_type()), fp(act), n,
+                                           gx.data_ptr(), nullptr, fp(graw), B, (int32_t)n, (int32_t)C, stream()),
+              "mhc_stream_aggregate_bwd");
+        return {gx.to(inp.scalar_type()), graw};
+    }
+};
+
+struct Distribute : public torch::autograd::Function<Distribute> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& y_in, const Tensor& h_in, const Tensor& m_in,
+                          const Tensor& x_in) {
+        const char* fn = "stream_distribute_mix_add_fwd";
+        check_device(fn, {&y_in, &h_in, &m_in, &x_in});
+        const at::DeviceGuard guard(x_in.device());
+        TORCH_CHECK(x_in.dim() == 3, "x_inp must be 3D tensor [B, n, C]");
+        const Tensor x = storage(x_in);
+        const int64_t B = x.size(0), n = x.size(1), C = x.size(2);
+        const Tensor y = y_in.to(x.scalar_type()).contiguous();
+        TORCH_CHECK(y.dim() == 2 && y.size(0) == B && y.size(1) == C, "y_norm must be [B, C]");
+        const auto [h, hs] = coef_view(fn, h_in, B, n);
+        const auto [m, ms] = coef_view(fn, m_in, B, n * n);
+        const auto f32 = x.options().dtype(at::kFloat);
+        Tensor out = at::empty({B, n, C}, f32);
+        Tensor act = at::empty({B, n}, f32);
+        check(lib.mhc_stream_distribute_mix_add_fwd(y.data_ptr(), fp(h), hs, fp(m), ms, x.data_ptr(),
+                                                    dtype_code(x.scalar_type()), fp(out), fp(act), B, (int32_t)n,
+                                                    (int32_t)C, stream()),
+              "mhc_stream_distribute_mix_add_fwd");
+        ctx->save_for_backward({x_in, y_in, m_in, act});
+        return out;
+    }
+
+    static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+        const char* fn = "stream_distribute_mix_add_bwd";
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &x_in = sv[0], &y_in = sv[1], &m_in = sv[2], &act = sv[3];
+        check_device(fn, {&grads[0], &x_in, &y_in, &m_in, &act});
+        const at::DeviceGuard guard(x_in.device());
+        const Tensor x = storage(x_in);
+        const int64_t B = x.size(0), n = x.size(1), C = x.size(2);
+        const Tensor y = y_in.to(x.scalar_type()).contiguous();
+        const Tensor g = f32c(grads[0]);
+        TORCH_CHECK(g.sizes() == x.sizes(), "grad_out shape must match x_inp");
+        const auto [m, ms] = coef_view(fn, m_in, B, n * n);
+        const auto f32 = x.options().dtype(at::kFloat);
+        Tensor gx = at::empty_like(x), gy = at::empty({B, C}, x.options());
+        Tensor gm = at::empty({B, n, n}, f32), graw = at::empty({B, n}, f32);
+        check(lib.mhc_stream_distribute_mix_add_bwd(fp(g), x.data_ptr(), y.data_ptr(), dtype_code(x.scalar_type()),
+                                                    fp(m), ms, fp(act), n, gx.data_ptr(), gy.data_ptr(), fp(gm),
+                                                    nullptr, fp(graw), B, (int32_t)n, (int32_t)C, stream()),
+              "mhc_stream_distribute_mix_add_bwd");
+        return {gy.to(y_in.scalar_type()), graw, gm, gx.to(x_in.scalar_type())};
+    }
+};
+
+Tensor sinkhorn_knopp(const Tensor& inp, int64_t iters, double eps) {
+    require_bound();
+    return Sinkhorn::apply(inp, iters, eps);
+}
+
+Tensor rmsnorm(const Tensor& inp, const Tensor& w, double eps) {
+    require_bound();
+    return RmsNorm::apply(inp, w, eps);
+}
+
+Tensor stream_aggregate(const Tensor& inp, const Tensor& h) {
+    require_bound();
+    return Aggregate::apply(inp, h);
+}
+
+Tensor stream_distribute_mix_add(const Tensor& y, const Tensor& h, const Tensor& m, const Tensor& x) {
+    require_bound();
+    return Distribute::apply(y, h, m, x);
+}
 
 Tensor static_layer(const Tensor& x, const Tensor& w, const Tensor& hp, const Tensor& hq, const Tensor& hr,
                     int64_t iters, double sk_eps, double rms_eps) {
@@ -515,7 +740,7 @@ Tensor dynamic_wrapper(const Tensor& residual, const Tensor& branch, const Tenso
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-    m.doc() = "C++ autograd nodes of the fused mHC layers over libmhc_hip's C ABI";
+    m.doc() = "C++ autograd nodes of the fused mHC layers and the standalone operators over libmhc_hip's C ABI";
     m.def("entry_names", &entry_names, "C-ABI entry points bind() needs");
     m.def("bind", &bind, "set the C-ABI entry points from {name: address}");
     m.def("static_layer", &static_layer,
@@ -531,4 +756,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "fused dynamic-H MHCResidualWrapper with autograd: (residual, branch, weight, phi_pre, phi_post, phi_res, "
           "alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res, residual_mode, n, num_iters, sinkhorn_eps, "
           "rmsnorm_eps) -> fp32 [tokens, C]");
+    m.def("dynamic_infer", &dynamic_infer,
+          "forward-only dynamic-H layer: (x, packed, alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res, "
+          "num_iters, sinkhorn_eps, rmsnorm_eps, out_bf16) -> [B, n, C]");
+    m.def("sinkhorn_knopp", &sinkhorn_knopp, "(inp [B, n, n] fp32, num_iters, eps) with autograd");
+    m.def("rmsnorm", &rmsnorm, "(inp [B, C], weight, eps) with autograd");
+    m.def("stream_aggregate", &stream_aggregate, "(inp [B, n, C], H_pre_raw [B, n]) with autograd");
+    m.def("stream_distribute_mix_add", &stream_distribute_mix_add,
+          "(y_norm [B, C], H_post_raw [B, n], M [B, n, n], x_inp [B, n, C]) -> fp32 [B, n, C] with autograd");
 }

@@ -2015,12 +2015,7 @@ bool proj_stream_path(int np) { return np > kStreamOB; }
 static int proj_stream_ksplit(int64_t B, int64_t K, int np) {
     const int mt = proj_stream_mt(B);
     const int64_t groups0 = ((B + 16 * mt - 1) / (16 * mt)) * ((np + kStreamOB - 1) / kStreamOB);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, proj_stream_fn<3, 0>(mt), 256, 0) != hipSuccess ||
-        per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(proj_stream_fn<3, 0>(mt), 256, 0);
     // rounded down: a last partial round would leave most CUs idle while it
     // runs; splits x tokens at most 4096 (the partials the coefficient
     // kernel adds per token: 32 splits at 128 tokens, 128 at 32)
@@ -3156,11 +3151,7 @@ int proj_bwd_tiles(int x_dtype, int64_t B, int64_t K) {
     const int64_t gx = (K + cb - 1) / cb;
     const void* fn = x_dtype == kBF16 ? reinterpret_cast<const void*>(&proj_bwd_mfma_kernel<bf16_t, true, true>)
                                       : reinterpret_cast<const void*>(&proj_bwd_mfma_kernel<float, true, true>);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 2 * cb, 0) != hipSuccess || per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(fn, 2 * cb, 0);
     int64_t tiles = 2 * (int64_t)device_cu_count() * per_cu / gx;
     const int64_t blocks = (B + 31) / 32;
     if (tiles > blocks) tiles = blocks;

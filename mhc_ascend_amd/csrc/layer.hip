@@ -970,12 +970,7 @@ static const void* pick_bwd(int x_dtype, int n, int vpt, int mode, bool pf) {
 }
 
 static int persistent_grid(const void* fn, int threads, int64_t B) {
-    int per_cu = 0;
-    if (fn == nullptr || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0) != hipSuccess ||
-        per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(fn, threads, 0);
     int64_t g = (int64_t)device_cu_count() * per_cu;
     if (g > B) g = B;
     if (g < 1) g = 1;

@@ -35,6 +35,10 @@ inline RowTiling with_min_threads(RowTiling t, int need) {
 // Number of compute units of the current device (cached per device).
 int device_cu_count();
 
+// Resident workgroups per CU of `fn` on the current device (cached; 1 when
+// the runtime cannot tell).
+int occupancy_per_cu(const void* fn, int threads, size_t lds);
+
 // Per-kernel timing, compiled in only for the benchmark's build of the
 // library (MHC_KERNEL_TIMING, libmhc_hip_timed.so; include/mhc_hip_timing.h).
 // timing_begin(name) opens a scope (returning a token for timing_end) in

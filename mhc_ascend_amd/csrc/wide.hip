@@ -1045,13 +1045,7 @@ int wide_bwd_grid(int x_dtype, int n, int64_t B, int64_t C) {
         return hipSuccess;
     };
     if (pick() != hipSuccess || !fn) return 1;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kWideThreads, (size_t)C * sizeof(float)) !=
-            hipSuccess ||
-        per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(fn, kWideThreads, (size_t)C * sizeof(float));
     int64_t grid = (int64_t)device_cu_count() * per_cu;
     if (grid > B) grid = B;
     return (int)(grid < 1 ? 1 : grid);
@@ -1171,13 +1165,7 @@ int wide_rmsnorm_bwd_grid(int dt, int64_t B, int64_t C) {
     if (B <= 0 || C < 1 || C > kWideMaxC) return 1;
     const void* fn = dt == kBF16 ? reinterpret_cast<const void*>(&wide_rmsnorm_bwd_kernel<bf16_t>)
                                  : reinterpret_cast<const void*>(&wide_rmsnorm_bwd_kernel<float>);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kWideThreads, (size_t)C * sizeof(float)) !=
-            hipSuccess ||
-        per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(fn, kWideThreads, (size_t)C * sizeof(float));
     int64_t grid = (int64_t)device_cu_count() * per_cu;
     if (grid > B) grid = B;
     return (int)(grid < 1 ? 1 : grid);

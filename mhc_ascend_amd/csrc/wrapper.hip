@@ -1578,12 +1578,7 @@ static const void* wrap_bwd_fn() {
 }
 
 static int wrap_grid(const void* fn, int threads, int64_t B) {
-    int per_cu = 0;
-    if (fn == nullptr || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0) != hipSuccess ||
-        per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(fn, threads, 0);
     int64_t g = (int64_t)device_cu_count() * per_cu;
     if (g > B) g = B;
     if (g < 1) g = 1;
@@ -1755,11 +1750,7 @@ int wrap_proj_bwd_tiles(int dt, int64_t B, int64_t C) {
     const int64_t gx = (C + kWpbCols - 1) / kWpbCols;
     const void* fn = dt == kBF16 ? reinterpret_cast<const void*>(&wrap_proj_bwd_kernel<bf16_t, 4, true, true>)
                                  : reinterpret_cast<const void*>(&wrap_proj_bwd_kernel<float, 4, true, true>);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kWpbThreads, 0) != hipSuccess || per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
+    const int per_cu = occupancy_per_cu(fn, kWpbThreads, 0);
     int64_t tiles = 2 * (int64_t)device_cu_count() * per_cu / gx;
     const int64_t blocks = (B + 31) / 32;
     if (tiles > blocks) tiles = blocks;

@@ -1,5 +1,8 @@
 """Autograd functions over the HIP kernels (mirror of src/python/mhc/ops.py).
 
+The autograd nodes of the layers, the wrapper and the stand-alone operators
+are C++ (csrc/autograd.cpp); the projection's is the one Python Function.
+
 Public functional ops keep the reference's names, arguments and defaults.
 Documented differences from the Ascend implementation (all toward the
 PyTorch reference math, which is the contract):
@@ -28,22 +31,12 @@ _STREAM_PROJ_ROWS = 128
 # Sinkhorn-Knopp (ops.py:32-80)
 # =============================================================================
 
-class SinkhornKnoppFunction(torch.autograd.Function):
+class SinkhornKnoppFunction:
     """Sinkhorn-Knopp doubly stochastic normalisation of [B, n, n]."""
 
     @staticmethod
-    def forward(ctx, inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) -> torch.Tensor:
-        out = native.sinkhorn_knopp_fwd(inp, num_iters, eps)
-        ctx.save_for_backward(inp, out)
-        ctx.num_iters = num_iters
-        ctx.eps = eps
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out: torch.Tensor):
-        inp, out = ctx.saved_tensors
-        grad_inp = native.sinkhorn_knopp_bwd(grad_out.float().contiguous(), inp, out, ctx.num_iters, ctx.eps)
-        return grad_inp, None, None
+    def apply(inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) -> torch.Tensor:
+        return _lib.autograd().sinkhorn_knopp(inp, int(num_iters), float(eps))
 
 
 def sinkhorn_knopp(inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) -> torch.Tensor:
@@ -55,21 +48,12 @@ def sinkhorn_knopp(inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) ->
 # RMSNorm (ops.py:87-136)
 # =============================================================================
 
-class RMSNormFunction(torch.autograd.Function):
+class RMSNormFunction:
     """Root Mean Square normalisation of [B, C] rows."""
 
     @staticmethod
-    def forward(ctx, inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
-        out, rms = native.rmsnorm_fwd(inp, weight, eps)
-        ctx.save_for_backward(inp, weight, rms)
-        ctx.eps = eps
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out: torch.Tensor):
-        inp, weight, rms = ctx.saved_tensors
-        grad_inp, grad_weight = native.rmsnorm_bwd(grad_out, inp, weight, rms)
-        return grad_inp.to(inp.dtype), grad_weight, None
+    def apply(inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
+        return _lib.autograd().rmsnorm(inp, weight, float(eps))
 
 
 def rmsnorm(inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
@@ -81,20 +65,12 @@ def rmsnorm(inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch
 # Stream aggregate (ops.py:143-188)
 # =============================================================================
 
-class StreamAggregateFunction(torch.autograd.Function):
+class StreamAggregateFunction:
     """out = sum_i sigmoid(H_pre_raw[:, i]) * inp[:, i]."""
 
     @staticmethod
-    def forward(ctx, inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor:
-        out, h_act = native.stream_aggregate_fwd(inp, H_pre_raw)
-        ctx.save_for_backward(inp, h_act)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out: torch.Tensor):
-        inp, h_act = ctx.saved_tensors
-        gx, _, graw = native._aggregate_bwd(grad_out, inp, h_act, True)
-        return gx.to(inp.dtype), graw
+    def apply(inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor:
+        return _lib.autograd().stream_aggregate(inp, H_pre_raw)
 
 
 def stream_aggregate(inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor:
@@ -106,20 +82,12 @@ def stream_aggregate(inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor
 # Stream distribute-mix-add (ops.py:195-265)
 # =============================================================================
 
-class StreamDistributeMixAddFunction(torch.autograd.Function):
+class StreamDistributeMixAddFunction:
     """out[:, i] = 2 sigmoid(H_post_raw[:, i]) * y_norm + sum_j M[:, i, j] x[:, j]."""
 
     @staticmethod
-    def forward(ctx, y_norm, H_post_raw, M, x_inp):
-        out, h_act = native.stream_distribute_mix_add_fwd(y_norm, H_post_raw, M, x_inp)
-        ctx.save_for_backward(x_inp, y_norm, M, h_act)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        x_inp, y_norm, M, h_act = ctx.saved_tensors
-        gx, gy, gM, _, graw = native._distribute_bwd(grad_out, x_inp, y_norm, M, h_act, True)
-        return gy.to(y_norm.dtype), graw, gM, gx.to(x_inp.dtype)
+    def apply(y_norm: torch.Tensor, H_post_raw: torch.Tensor, M: torch.Tensor, x_inp: torch.Tensor) -> torch.Tensor:
+        return _lib.autograd().stream_distribute_mix_add(y_norm, H_post_raw, M, x_inp)
 
 
 def stream_distribute_mix_add(y_norm: torch.Tensor, H_post_raw: torch.Tensor, M: torch.Tensor,
@@ -197,6 +165,11 @@ def mhc_layer_fused_dynamic_inference(x_expanded, rmsnorm_weight, phi_pre, phi_p
                                                 alpha_post, alpha_res, b_pre, b_post, b_res, sinkhorn_iters,
                                                 sinkhorn_eps, rmsnorm_eps)[0]
         packed = native.mhc_layer_dynamic_pack(rmsnorm_weight, phi_pre, phi_post, phi_res)
+    if (out_dtype in (torch.float32, torch.bfloat16) and torch.is_tensor(alpha_pre) and torch.is_tensor(alpha_post)
+            and torch.is_tensor(alpha_res)):
+        return _lib.autograd().dynamic_infer(x_expanded, packed, alpha_pre, alpha_post, alpha_res, b_pre, b_post,
+                                             b_res, int(sinkhorn_iters), float(sinkhorn_eps), float(rmsnorm_eps),
+                                             out_dtype == torch.bfloat16)
     return native.mhc_layer_dynamic_infer(x_expanded, packed, alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res,
                                           sinkhorn_iters, sinkhorn_eps, rmsnorm_eps, out_dtype)
 
