@@ -1346,15 +1346,14 @@ size_t mhc_wrapper_dynamic_saved_size(int64_t tokens, int32_t n, int32_t hidden)
 static bool wrap_res_grad_vanishes(int32_t num_iters, float sinkhorn_eps);
 
 // ---- run-time-n wrapper (wrapper_gen.hip) ---------------------------------------
-// The row passes rebuild the streams from r and b; with dynamic H the
-// layer's projection kernels (forward and backward) take the stream rows
-// X [tokens, n*C] from wgen_synth_kernel, and the backward folds their dX
-// over the streams.
+// The row passes rebuild the streams from r and b, and so does the forward
+// projection where hidden % 8 == 0; otherwise, and in the backward's general
+// case, the layer's projection kernels take the stream rows X [tokens, n*C]
+// from wgen_synth_kernel, and the backward folds their dX over the streams.
 //
-// dynamic forward workspace: [the layer projection's workspace (proj_fwd_ws)
-// | X], X only where the projection does not rebuild the streams itself
-// (wgen_fwd_direct); the all-dtypes size query reserves X at 4 bytes per
-// element.
+// dynamic forward workspace: the folded projection's (wfold_ws), or, for
+// hidden sizes it does not take (hidden % 8 != 0), [the layer projection's
+// workspace (proj_fwd_ws) | X].
 struct WgenFwdWs {
     ProjFwdWs p;
     size_t x_off, total;
@@ -1369,15 +1368,27 @@ static WgenFwdWs wgen_fwd_ws(int64_t tokens, int32_t n, int32_t hidden) {
     return w;
 }
 
-// bf16 rows of whole 64-channel stages, more than 32 projection rows and
-// at least 1024 tokens: the streaming projection reads residual and branch
-// and rebuilds the streams itself
-static bool wgen_fwd_direct(int32_t dtype, int32_t n, int32_t hidden, int64_t tokens) {
-    return proj_one_pass(dtype, 2 * n + n * n, tokens) && hidden % 64 == 0;
+// The projection folded onto r and b (wrapper_proj.hip): [packed Phi | P
+// partials | sum X^2 partials | aligned copies of r and b, for rows at an
+// address that is not 16-byte aligned].
+struct WfoldWs {
+    int ks;
+    size_t p_off, ss_off, copy_off, total;
+};
+
+static WfoldWs wfold_ws(int32_t dtype, int64_t tokens, int32_t n, int32_t hidden) {
+    WfoldWs w{};
+    const int np = 2 * n + n * n;
+    w.ks = tokens > 0 ? wfold_ksplit(dtype, tokens, hidden, np) : 1;
+    w.p_off = align256(wfold_pack_bytes(dtype, n, hidden, np));
+    w.ss_off = w.p_off + align256((size_t)proj_tiles(np) * w.ks * tokens * kProjTile * sizeof(float));
+    w.copy_off = w.ss_off + align256((size_t)w.ks * tokens * sizeof(float));
+    w.total = w.copy_off + 2 * align256((size_t)tokens * hidden * dtype_size(dtype));
+    return w;
 }
 
 static size_t wgen_fwd_need(const WgenFwdWs& w, int32_t dtype, int32_t n, int32_t hidden, int64_t tokens) {
-    if (wgen_fwd_direct(dtype, n, hidden, tokens)) return w.p.total;
+    if (wfold_ok(n, hidden)) return wfold_ws(dtype, tokens, n, hidden).total;
     return w.x_off + align256((size_t)tokens * n * hidden * dtype_size(dtype));
 }
 
@@ -1469,7 +1480,9 @@ static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dt
                             int32_t num_iters, float sinkhorn_eps, float rmsnorm_eps, hipStream_t s) {
     const DynSaved d = dyn_saved(tokens, n, hidden);
     float* w32 = saved + d.w_off;
-    hipError_t e = launch_weight_f32(weight, weight_dtype, hidden, w32, s);
+    const bool wfold = tokens > 0 && wfold_ok(n, hidden);
+    // the weight's fp32 copy: its own launch, or inside the folded pack's
+    hipError_t e = wfold ? hipSuccess : launch_weight_f32(weight, weight_dtype, hidden, w32, s);
     if (e != hipSuccess || tokens == 0) return hip_status(e);
     const WgenFwdWs w = wgen_fwd_ws(tokens, n, hidden);
     if (!workspace || workspace_bytes < wgen_fwd_need(w, dtype, n, hidden, tokens))
@@ -1482,10 +1495,23 @@ static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dt
     float* pp = (float*)(pw + w.p.p_off);
     float* ss = (float*)(pw + w.p.ss_off);
     bf16_raw_t* phib = (bf16_raw_t*)(pw + w.p.phib_off);
-    if (wgen_fwd_direct(dtype, n, hidden, tokens)) {
-        e = launch_phi_split(phi_pre, phi_post, phi_res, n, np, K, phib, s);
+    int ks = w.p.ks;
+    if (wfold) {
+        const WfoldWs f = wfold_ws(dtype, tokens, n, hidden);
+        const void *pres = residual, *pbr = branch;
+        if ((uintptr_t)residual % 16 != 0 || (uintptr_t)branch % 16 != 0) {
+            char* c = pw + f.copy_off;
+            char* c2 = c + align256((size_t)tokens * hidden * dtype_size(dtype));
+            e = launch_wfold_copy(dtype, residual, c, branch, c2, tokens * hidden, s);
+            pres = c;
+            pbr = c2;
+        }
+        ks = f.ks;
+        pp = (float*)(pw + f.p_off);
+        ss = (float*)(pw + f.ss_off);
         if (e == hipSuccess)
-            e = launch_proj_stream_wrap(decay, residual, branch, hidden, phib, np, pp, ss, tokens, K, w.p.ks, s);
+            e = launch_wfold_proj(dtype, n, decay, pres, pbr, phi_pre, phi_post, phi_res, weight, weight_dtype, w32, pw,
+                                  pp, ss, tokens, hidden, ks, s);
     } else {
         e = launch_wgen_synth(dtype, dtype, n, decay, residual, branch, X, tokens, hidden, s);
         if (e == hipSuccess && w.p.stream) {
@@ -1501,7 +1527,7 @@ static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dt
         }
     }
     if (e == hipSuccess)
-        e = launch_dyn_coef_fwd(n, pp, ss, w.p.ks, tokens, K, alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res,
+        e = launch_dyn_coef_fwd(n, pp, ss, ks, tokens, K, alpha_pre, alpha_post, alpha_res, b_pre, b_post, b_res,
                                 saved + d.coef_off, saved + d.p_off, saved + d.rh_off, num_iters, sinkhorn_eps,
                                 rmsnorm_eps, s);
     if (e == hipSuccess)
@@ -1663,7 +1689,11 @@ static WrapFwdWs wrap_fwd_ws(int64_t tokens, int32_t n, int32_t hidden) {
 
 size_t mhc_wrapper_dynamic_fwd_workspace_size(int64_t tokens, int32_t n, int32_t hidden) {
     if (tokens < 0 || n < 1 || hidden < 1) return 0;
-    if (!wrap_fused4(n, hidden, true)) return wgen_fwd_ws(tokens, n, hidden).total;
+    if (!wrap_fused4(n, hidden, true)) {
+        const WgenFwdWs w = wgen_fwd_ws(tokens, n, hidden);
+        const size_t a = wgen_fwd_need(w, kF32, n, hidden, tokens), b = wgen_fwd_need(w, kBF16, n, hidden, tokens);
+        return a > b ? a : b;
+    }
     return wrap_fwd_ws(tokens, n, hidden).total;
 }
 

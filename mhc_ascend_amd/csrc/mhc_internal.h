@@ -297,14 +297,6 @@ constexpr size_t proj_xplanes_bytes(int64_t B, int64_t K) { return (size_t)(3 * 
 hipError_t launch_proj_stream(int x_dtype, const void* x, bf16_raw_t* xplanes, const float* phi_pre,
                               const float* phi_post, const float* phi_res, int n_pre, const bf16_raw_t* phib, int np,
                               float* p_part, float* ss_part, int64_t B, int64_t K, int ks, hipStream_t s);
-// The streaming projection of the MHCResidualWrapper's stream rows with
-// bf16 storage, read from residual / branch ([B][Cw] each, Cw % 64 == 0)
-// instead of a stream tensor (decay: streams j >= 2 are bf16(r 0.1^(j-1)),
-// else 0); Phi as the planes of launch_phi_split; p_part / ss_part as
-// launch_proj_mfma.
-hipError_t launch_proj_stream_wrap(bool decay, const void* res, const void* br, int64_t Cw, const bf16_raw_t* phib,
-                                   int np, float* p_part, float* ss_part, int64_t B, int64_t K, int ks,
-                                   hipStream_t s);
 hipError_t launch_proj_reduce(const float* p_part, int ks, int64_t B, int np, float* out, hipStream_t s);
 #ifdef MHC_KERNEL_TIMING
 // The benchmark build's VALU projection (A/B against launch_proj_mfma): Phi
@@ -502,5 +494,19 @@ hipError_t launch_sinkhorn_fwd(int n, const float* inp, float* out, int64_t batc
                                hipStream_t s);
 hipError_t launch_sinkhorn_bwd(int n, const float* grad_out, const float* inp, float* grad_inp, int64_t batch,
                                int iters, float eps, hipStream_t s);
+
+// ---- wrapper_proj.hip --------------------------------------------------------
+// The wrapper's forward projection over r and b (hidden % 8 == 0, 16-byte
+// aligned rows): P and sum X^2 partials of wfold_ksplit splits in
+// launch_proj_mfma's layout, Phi packed into `pack` (wfold_pack_bytes, both
+// residual modes) and the RMSNorm weight's fp32 copy into w32 on the way.
+bool wfold_ok(int n, int64_t C);
+int wfold_ksplit(int dt, int64_t B, int64_t C, int np);
+size_t wfold_pack_bytes(int dt, int n, int64_t C, int np);
+hipError_t launch_wfold_copy(int dt, const void* res, void* res_out, const void* br, void* br_out, int64_t elems,
+                             hipStream_t s);
+hipError_t launch_wfold_proj(int dt, int n, bool decay, const void* res, const void* br, const float* phi_pre,
+                             const float* phi_post, const float* phi_res, const void* weight, int w_dtype, float* w32,
+                             void* pack, float* p_part, float* ss_part, int64_t B, int64_t C, int ks, hipStream_t s);
 
 }  // namespace mhc

@@ -452,7 +452,8 @@ hipError_t launch_compute_rms(int dt, const void* x, float* rms, int64_t B, int6
 // The stream operators' register rows (vpt 0: the channel-loop kernels run):
 // n <= 8, rows that fit, and for n = 3, 5, 6, 7 aligned arrays
 // (rows_aligned).  A row per workgroup in registers against the generic
-// kernels' staged mixing, n = 6, 2047 x 1040 bf16: MEASURED_OPS_N6.
+// kernels' staged mixing, n = 6, 2047 x 1040 bf16: aggregate 12.7 / 16.5 ->
+// 10.6 / 14.2 us forward / backward, distribute 39.2 / 114 -> 28.3 / 28.0 us.
 static RowTiling ops_tiling(int dt, int n, int64_t C, int arrays, int pref, std::initializer_list<const void*> ps) {
     if (n > 8 || !rows_aligned(n, ps)) return RowTiling{0, 0};
     return choose_row_tiling(C, dt == kBF16 ? 8 : 4, arrays, pref);
