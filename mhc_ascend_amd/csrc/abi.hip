@@ -1392,6 +1392,16 @@ static size_t wgen_fwd_need(const WgenFwdWs& w, int32_t dtype, int32_t n, int32_
     return w.x_off + align256((size_t)tokens * n * hidden * dtype_size(dtype));
 }
 
+// The size queries' answer.  They keep the relation that callers dividing one
+// buffer between storage types count on: fp32 rows, and bf16 rows that the
+// streaming projection could not rebuild (up to 32 projection rows, fewer than
+// 1024 tokens, hidden % 64 != 0), reserve the stream rows in their own dtype.
+static size_t wgen_fwd_size(const WgenFwdWs& w, int32_t dtype, int32_t n, int32_t hidden, int64_t tokens) {
+    const size_t need = wgen_fwd_need(w, dtype, n, hidden, tokens);
+    if (!wfold_ok(n, hidden) || (proj_one_pass(dtype, 2 * n + n * n, tokens) && hidden % 64 == 0)) return need;
+    return need + align256((size_t)tokens * n * hidden * dtype_size(dtype));
+}
+
 // backward workspace: [per-token factors | dw partials | dw stage | ...]
 //   static:  [scalar rows per wave | their sum | Sinkhorn history
 //            (static_sk_hist)]
@@ -1691,7 +1701,7 @@ size_t mhc_wrapper_dynamic_fwd_workspace_size(int64_t tokens, int32_t n, int32_t
     if (tokens < 0 || n < 1 || hidden < 1) return 0;
     if (!wrap_fused4(n, hidden, true)) {
         const WgenFwdWs w = wgen_fwd_ws(tokens, n, hidden);
-        const size_t a = wgen_fwd_need(w, kF32, n, hidden, tokens), b = wgen_fwd_need(w, kBF16, n, hidden, tokens);
+        const size_t a = wgen_fwd_size(w, kF32, n, hidden, tokens), b = wgen_fwd_size(w, kBF16, n, hidden, tokens);
         return a > b ? a : b;
     }
     return wrap_fwd_ws(tokens, n, hidden).total;
@@ -1700,7 +1710,7 @@ size_t mhc_wrapper_dynamic_fwd_workspace_size(int64_t tokens, int32_t n, int32_t
 size_t mhc_wrapper_dynamic_fwd_workspace_size_for(int64_t tokens, int32_t n, int32_t hidden, int32_t dtype) {
     if (tokens < 0 || n < 1 || hidden < 1 || !valid_dtype(dtype)) return 0;
     if (!wrap_fused4(n, hidden, true))
-        return wgen_fwd_need(wgen_fwd_ws(tokens, n, hidden), dtype, n, hidden, tokens);
+        return wgen_fwd_size(wgen_fwd_ws(tokens, n, hidden), dtype, n, hidden, tokens);
     return wrap_fwd_ws(tokens, n, hidden).total;
 }
 
