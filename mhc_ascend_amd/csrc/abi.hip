@@ -1426,9 +1426,9 @@ static bool wgen_fold_ok(int32_t n, int32_t hidden) {
 }
 
 struct WgenBwdWs {
-    int cblocks, ptiles, dtiles, qtiles, ftiles, srows;
+    int cblocks, ptiles, dtiles, qtiles, ftiles, wtiles, srows;
     size_t ep_off, dw_off, stw_off, scal_off, ssum_off, hist_off, dp_off, s_off, cpart_off, x_off, dx_off, part_off,
-        stp_off, total;
+        stp_off, phif_off, total;
 };
 
 static WgenBwdWs wgen_bwd_ws(int64_t tokens, int32_t n, int32_t hidden, bool dynamic) {
@@ -1439,7 +1439,9 @@ static WgenBwdWs wgen_bwd_ws(int64_t tokens, int32_t n, int32_t hidden, bool dyn
     size_t o = 0;
     w.dtiles = tokens > 0 ? wgen_dx_tiles(tokens, hidden) : 1;
     w.ftiles = tokens > 0 ? wgen_fold_tiles(tokens, hidden) : 1;
-    const int dw_rows = dynamic && w.ftiles > w.dtiles ? w.ftiles : w.dtiles;
+    w.wtiles = dynamic && tokens > 0 ? wbwd_tiles(n, tokens, hidden) : 1;
+    int dw_rows = dynamic && w.ftiles > w.dtiles ? w.ftiles : w.dtiles;
+    if (w.wtiles > dw_rows) dw_rows = w.wtiles;
     w.ep_off = o; o += align256((size_t)tokens * kWgEp * 4);
     w.dw_off = o; o += align256((size_t)dw_rows * hidden * 4);
     w.stw_off = o; o += align256(column_sums_stage_floats(hidden) * 4);
@@ -1466,8 +1468,11 @@ static WgenBwdWs wgen_bwd_ws(int64_t tokens, int32_t n, int32_t hidden, bool dyn
     if (np <= kProjTile && (size_t)w.ptiles * np > part) part = (size_t)w.ptiles * np;
     if (!wgen_fold_ok(n, hidden) && 2 * n <= kProjTile && (size_t)w.ptiles * 2 * n > part)
         part = (size_t)w.ptiles * 2 * n;
+    // wbwd_kernel's: 2n rows of each stream that it forms
+    const size_t wpart = (size_t)w.wtiles * 2 * n * (n <= 8 ? n : 2) * hidden;
     const int64_t srows = np <= kProjTile ? np : 2 * n;
-    w.part_off = o; o += align256(part * K * 4);
+    w.part_off = o; o += align256((part * K > wpart ? part * K : wpart) * 4);
+    w.phif_off = o; o += align256(wbwd_fold_bytes(n, hidden));
     w.stp_off = o; o += align256(column_sums_stage_floats(srows * K) * 4);
     w.x_off = o; o += align256((size_t)tokens * K * 4);
     w.dx_off = o; o += align256((size_t)tokens * K * 4);
@@ -1581,6 +1586,13 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
     const int64_t K = (int64_t)n * hidden;
     // the fold kernels' shapes carry the pre / post rows without stream rows
     const bool fold = rows < np && wgen_fold_ok(n, hidden);
+    // wbwd_kernel takes whole 16-byte pieces of aligned rows; bf16 'decay' past
+    // n = 8, C % 8 != 0 and unaligned rows keep the kernels below.  dPhi, d r and
+    // d b at n = 8 (65,536 x 7168 bf16): 1.30 ms against 3.2; fp32 n = 16 (4096 x
+    // 2048): 50 us against 905
+    const bool one = tokens > 0 && rows < np && wbwd_shape_ok(dtype, n, decay, hidden) &&
+                     ((uintptr_t)grad_out | (uintptr_t)residual | (uintptr_t)branch | (uintptr_t)grad_residual |
+                      (uintptr_t)grad_branch) % 16 == 0;
     hipError_t e = hipSuccess;
     int rows_w = fold ? w.ftiles : w.dtiles, rows_c = w.cblocks;
     if (tokens == 0) {
@@ -1597,7 +1609,22 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
             e = launch_dyn_coef_bwd(n, scal, saved + d.coef_off, saved + d.p_off, saved + d.rh_off, tokens, K,
                                     alpha_pre, alpha_post, alpha_res, b_res, dp, stok, cpart, num_iters, sinkhorn_eps,
                                     nullptr, s, rows == np);
-        if (fold) {
+        if (one) {
+            if (e == hipSuccess)
+                e = launch_wbwd(dtype, n, decay, grad_out, residual, branch, w32, ep, dp, dp_stride(np), stok, phi_pre,
+                                phi_post, (float*)(ws + w.phif_off), grad_residual, grad_branch, dw_part, part,
+                                w.wtiles, tokens, hidden, s);
+            const int nst = wbwd_streams(dtype, n, decay);
+            const bool few = w.cblocks <= kWrapSumsMaxRows;
+            if (e == hipSuccess)
+                e = launch_wrap_sums(WrapSums{part, (int64_t)nst * rows * hidden, (int64_t)rows * hidden, hidden,
+                                              w.wtiles, nst, rows, n, np, hidden, decay, grad_phi, dw_part, w.wtiles,
+                                              weight_dtype == kBF16, grad_weight, few ? cpart : nullptr,
+                                              few ? w.cblocks : 0, grad_b, grad_alpha, 0},
+                                     s);
+            if (few || e != hipSuccess) return hip_status(e);
+        }
+        if (!one && fold) {
             if (e == hipSuccess)
                 e = launch_wgen_dphi(dtype, n, decay, residual, branch, dp, dp_stride(np), rows, part, w.qtiles, tokens,
                                      hidden, s);
@@ -1609,8 +1636,9 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
                                         dp, dp_stride(np), rows, stok, phi_pre, phi_post, grad_residual,
                                         grad_branch, dw_part, w.ftiles, tokens, hidden, s);
         }
-        if (!fold && e == hipSuccess) e = launch_wgen_synth(dtype, kF32, n, decay, residual, branch, X, tokens, hidden, s);
-        if (!fold && e == hipSuccess) {
+        const bool full = !one && !fold;
+        if (full && e == hipSuccess) e = launch_wgen_synth(dtype, kF32, n, decay, residual, branch, X, tokens, hidden, s);
+        if (full && e == hipSuccess) {
             if (rows > kProjTile) {  // X and dX once for all output tiles
                 e = launch_proj_bwd_small(X, dp, dp_stride(np), nullptr, phi_pre, phi_post, phi_res, n, rows, dX,
                                           false, grad_phi, tokens, K, s);
@@ -1622,11 +1650,11 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
                                                nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0.f, s);
             }
         }
-        if (!fold && e == hipSuccess)
+        if (full && e == hipSuccess)
             e = launch_wgen_dx(dtype, n, decay, grad_out, residual, branch, w32, saved + d.coef_off, np, ep, dX, stok,
                                grad_residual, grad_branch, dw_part, w.dtiles, tokens, hidden, s);
     }
-    if (e == hipSuccess)
+    if (!one && e == hipSuccess)
         e = launch_column_finalize(0, weight_dtype, dw_part, rows_w, hidden, stw, grad_weight, nullptr, 0, nullptr,
                                    nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0.f, s);
     if (e == hipSuccess) e = launch_small_column_sum(cpart, rows_c, np + 3, grad_b, grad_alpha, np, s);
@@ -1890,6 +1918,15 @@ int mhc_wrapper_dynamic_bwd(const float* grad_out, const void* residual, const v
             e = launch_wrap_proj_bwd(dtype, n, decay, grad_out, residual, branch, w32, ep, dp, stok, phi_pre,
                                      phi_post, phi_res, grad_residual, grad_branch, dw_part, phip, w.tiles, tokens,
                                      hidden, res_rows, s);
+        // one launch instead of four: the sums of small calls were 15 us of gaps
+        if (!res_rows && rows_c <= kWrapSumsMaxRows) {
+            if (e == hipSuccess)
+                e = launch_wrap_sums(WrapSums{phip, (int64_t)npo * K, hidden, K, w.tiles, n, npo, n, np, hidden, decay,
+                                              grad_phi, dw_part, w.tiles, weight_dtype == kBF16, grad_weight, cpart,
+                                              rows_c, grad_b, grad_alpha, 0},
+                                     s);
+            return hip_status(e);
+        }
     }
     if (e == hipSuccess)
         e = launch_column_finalize(0, weight_dtype, dw_part, rows_p, hidden, stw, grad_weight, nullptr, 0, nullptr,

@@ -33,7 +33,8 @@ AUTOGRAD_NAME = "_mhc_autograd"
 AUTOGRAD_PATH = os.path.join(PKG, AUTOGRAD_NAME + ".so")
 
 SOURCES = ["abi.hip", "compat.hip", "dynamic.hip", "generic.hip", "layer.hip", "ops.hip", "sinkhorn.hip", "wide.hip",
-           "wrapper.hip", "wrapper_gen.hip", "wrapper_proj.hip"]
+           "wrapper.hip", "wrapper_gen.hip", "wrapper_proj.hip",
+           "wrapper_bwd.hip"]
 
 ARCH = os.environ.get("MHC_OFFLOAD_ARCH", "gfx950")
 

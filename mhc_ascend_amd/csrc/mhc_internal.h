@@ -509,4 +509,40 @@ hipError_t launch_wfold_proj(int dt, int n, bool decay, const void* res, const v
                              const float* phi_post, const float* phi_res, const void* weight, int w_dtype, float* w32,
                              void* pack, float* p_part, float* ss_part, int64_t B, int64_t C, int ks, hipStream_t s);
 
+// ---- wrapper_bwd.hip ---------------------------------------------------------
+// The wrapper's dynamic-H backward after wgen_red / the coefficients, with the
+// H_res rows of dP zero: d r, d b, dw_part[tiles][C] and
+// dphi_part[tiles][wbwd_streams][2n][C] (wbwd_shape_ok; 16-byte aligned rows;
+// tiles from wbwd_tiles; fold: wbwd_fold_bytes of scratch).
+bool wbwd_shape_ok(int dt, int n, bool decay, int64_t C);
+int wbwd_streams(int dt, int n, bool decay);
+int wbwd_tiles(int n, int64_t B, int64_t C);
+size_t wbwd_fold_bytes(int n, int64_t C);
+hipError_t launch_wbwd(int dt, int n, bool decay, const float* g, const void* res, const void* br, const float* w,
+                       const float* ep, const float* dP, int dp_stride, const float* s_tok, const float* phi_pre,
+                       const float* phi_post, float* fold, void* dres, void* dbr, float* dw_part, float* dphi_part,
+                       int tiles, int64_t B, int64_t C, hipStream_t s);
+// The wrapper's parameter gradients from its backward's partials:
+// phi_part[t tile_stride + j stream_stride + o row_stride + c] over `tiles`
+// tiles, nst streams and `rows` rows into grad_phi[o][n][C] (streams past nst
+// are stream 0's multiples by 0.1^(j-1), or zeros without `decay`);
+// dw_part[dw_rows][C] into grad_w; and, with crows > 0, cpart[crows][np + 3]
+// into grad_b / grad_alpha and the zeros of the H_res rows.
+// (crows <= kWrapSumsMaxRows: every zeroing workgroup sums the alpha columns)
+constexpr int kWrapSumsMaxRows = 1024;
+struct WrapSums {
+    const float* phi_part;
+    int64_t tile_stride, stream_stride, row_stride;
+    int tiles, nst, rows, n, np, C, decay;
+    float* grad_phi;
+    const float* dw_part;
+    int dw_rows, w_bf16;
+    void* grad_w;
+    const float* cpart;
+    int crows;
+    float *grad_b, *grad_alpha;
+    int phases;  // set by launch_wrap_sums
+};
+hipError_t launch_wrap_sums(WrapSums a, hipStream_t s);
+
 }  // namespace mhc

@@ -225,10 +225,10 @@ __global__ __launch_bounds__(256) void wgen_fwd_kernel(const TX* __restrict__ re
 // every lane: sum dh_post_act), since dM_ij does not depend on i, and
 // spread over the n*n+2n slots once per wave.  Both write the per-token
 // factors of d r / d b, ep_out[b][kWgEp]:
-//   [A_r, B_r hs/r, A_b, B_b hs/r, hs/r, -B_r k2, -B_b k2, 0, h_pre_0..7]
+//   [A_r, B_r hs/r, A_b, B_b hs/r, hs/r, -B_r k2, -B_b k2, B_r, h_pre_0..7]
 // with A_r = sum_j w_j cm_j, B_r = sum_j w_j h_pre_j, A_b = cm_1,
 // B_b = h_pre_1, so that d r = A_r G + B_r gxa and d b = A_b G + B_b gxa
-// (h_pre only up to capacity 8: the wider kernels read it from coef).
+// (wgen_dx / wgen_dx_fold read h_pre past capacity 8 from coef).
 // ---------------------------------------------------------------------------
 template <typename TX, int NM, bool DECAY, bool STATIC>
 __global__ __launch_bounds__(256) void wgen_red_kernel(const float* __restrict__ g, const TX* __restrict__ res,
@@ -354,9 +354,9 @@ __global__ __launch_bounds__(256) void wgen_red_kernel(const float* __restrict__
         rec[4] = hsi;
         rec[5] = -b_r * k2;
         rec[6] = -b_b * k2;
-        rec[7] = 0.f;
+        rec[7] = b_r;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) rec[8 + j] = NM <= 8 && j < NM ? hp[j < NM ? j : 0] : 0.f;
+        for (int j = 0; j < 8; ++j) rec[8 + j] = j < NM ? hp[j < NM ? j : 0] : 0.f;
         float ev = 0.f;
 #pragma unroll
         for (int k = 0; k < kWgEp; ++k) ev = (lane == k) ? rec[k] : ev;
