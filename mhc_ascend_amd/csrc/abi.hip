@@ -1546,7 +1546,7 @@ static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dt
                                 saved + d.coef_off, saved + d.p_off, saved + d.rh_off, num_iters, sinkhorn_eps,
                                 rmsnorm_eps, s);
     if (e == hipSuccess)
-        e = launch_wgen_fwd(dtype, n, decay, residual, branch, w32, saved + d.coef_off, np, out, tokens, hidden,
+        e = launch_wrow_fwd(dtype, n, decay, residual, branch, w32, saved + d.coef_off, np, out, tokens, hidden,
                             rmsnorm_eps, s);
     return hip_status(e);
 }
@@ -1601,8 +1601,12 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
         if (e == hipSuccess) e = launch_fill_zero(cpart, np + 3, s);
         if (e == hipSuccess) e = launch_fill_zero(grad_phi, (int64_t)rows * K, s);
     } else {
-        e = launch_wgen_red(dtype, n, decay, false, grad_out, residual, branch, w32, saved + d.coef_off, np, scal, ep,
-                            tokens, hidden, rmsnorm_eps, s);
+        if (rows < np && wrow_red_ok(dtype, n, decay, hidden))
+            e = launch_wrow_red(dtype, n, decay, grad_out, residual, branch, w32, saved + d.coef_off, np, scal, ep,
+                                tokens, hidden, rmsnorm_eps, s);
+        else
+            e = launch_wgen_red(dtype, n, decay, false, grad_out, residual, branch, w32, saved + d.coef_off, np, scal,
+                                ep, tokens, hidden, rmsnorm_eps, s);
         // with the H_res rows vanishing no Sinkhorn adjoint runs (their dP,
         // db and dalpha are zeros, overwritten with the NaN carry below)
         if (e == hipSuccess)
@@ -1782,7 +1786,7 @@ int mhc_wrapper_dynamic_fwd(const void* residual, const void* branch, int32_t dt
                                 saved + d.coef_off, saved + d.p_off, saved + d.rh_off, num_iters, sinkhorn_eps,
                                 rmsnorm_eps, s);
     if (e == hipSuccess)
-        e = launch_wrap_fwd(dtype, n, decay, residual, branch, w32, saved + d.coef_off, np, out, tokens, hidden,
+        e = launch_wrow_fwd(dtype, n, decay, residual, branch, w32, saved + d.coef_off, np, out, tokens, hidden,
                             rmsnorm_eps, s);
     return hip_status(e);
 }
@@ -1957,9 +1961,9 @@ int mhc_wrapper_static_fwd(const void* residual, const void* branch, int32_t dty
                                       sinkhorn_eps, s);
     if (e != hipSuccess) return hip_status(e);
     if (!wrap_fused4(n, hidden, false))
-        return hip_status(launch_wgen_fwd(dtype, n, residual_mode == MHC_WRAPPER_DECAY, residual, branch,
+        return hip_status(launch_wrow_fwd(dtype, n, residual_mode == MHC_WRAPPER_DECAY, residual, branch,
                                           saved + saved_w_offset(n), saved, 0, out, tokens, hidden, rmsnorm_eps, s));
-    return hip_status(launch_wrap_fwd(dtype, n, residual_mode == MHC_WRAPPER_DECAY, residual, branch,
+    return hip_status(launch_wrow_fwd(dtype, n, residual_mode == MHC_WRAPPER_DECAY, residual, branch,
                                       saved + saved_w_offset(n), saved, 0, out, tokens, hidden, rmsnorm_eps, s));
 }
 

@@ -34,7 +34,7 @@ AUTOGRAD_PATH = os.path.join(PKG, AUTOGRAD_NAME + ".so")
 
 SOURCES = ["abi.hip", "compat.hip", "dynamic.hip", "generic.hip", "layer.hip", "ops.hip", "sinkhorn.hip", "wide.hip",
            "wrapper.hip", "wrapper_gen.hip", "wrapper_proj.hip",
-           "wrapper_bwd.hip"]
+           "wrapper_bwd.hip", "wrapper_row.hip"]
 
 ARCH = os.environ.get("MHC_OFFLOAD_ARCH", "gfx950")
 

@@ -392,9 +392,6 @@ hipError_t launch_weight_f32(const void* w, int w_dtype, int64_t C, float* out, 
 // Floats per token of the dynamic backward's stream-part factors
 // (cm_0..3, h_pre_0..3, hs, 1/r, k2, one spare slot).
 constexpr int kWrapEp = 12;
-hipError_t launch_wrap_fwd(int dt, int n, bool decay, const void* res, const void* br, const float* w,
-                           const float* coef, int64_t coef_stride, float* out, int64_t B, int64_t C, float eps,
-                           hipStream_t s);
 int wrap_bwd_grid(int dt, int n, bool decay, int64_t B, int64_t C);
 // Static-H backward: per-workgroup sums of [dM, dh_post_act, dh_pre_act] in
 // scal_out[grid][n*n+2n], d r / d b and the dw partials dw_part[grid][C].
@@ -431,15 +428,24 @@ hipError_t launch_wrap_proj_bwd(int dt, int n, bool decay, const float* g, const
 // kernels above do not take); hidden % 4 == 0.  The dPhi / fold kernels
 // (the dynamic-H backward without stream rows) take n <= kWgFoldMaxN.
 constexpr int kWgMaxN = 32;
+constexpr double wrap_pow01(int e) { return e <= 0 ? 1.0 : 0.1 * wrap_pow01(e - 1); }
+
+// Decay multiplier of stream j >= 2: Python's 0.1 ** (j - 1) as fp32 (the
+// product r * m is formed in fp32 by the reference's mul; the double
+// repeated product rounds to the same fp32 value as 0.1 ** e for e <= 63).
+#define MHC_WRAP_M(e) (float)wrap_pow01(e)
+constexpr float kWrapMult[kWgMaxN] = {
+    1.f,          0.f,          MHC_WRAP_M(1),  MHC_WRAP_M(2),  MHC_WRAP_M(3),  MHC_WRAP_M(4),  MHC_WRAP_M(5),  MHC_WRAP_M(6),
+    MHC_WRAP_M(7),  MHC_WRAP_M(8),  MHC_WRAP_M(9),  MHC_WRAP_M(10), MHC_WRAP_M(11), MHC_WRAP_M(12), MHC_WRAP_M(13), MHC_WRAP_M(14),
+    MHC_WRAP_M(15), MHC_WRAP_M(16), MHC_WRAP_M(17), MHC_WRAP_M(18), MHC_WRAP_M(19), MHC_WRAP_M(20), MHC_WRAP_M(21), MHC_WRAP_M(22),
+    MHC_WRAP_M(23), MHC_WRAP_M(24), MHC_WRAP_M(25), MHC_WRAP_M(26), MHC_WRAP_M(27), MHC_WRAP_M(28), MHC_WRAP_M(29), MHC_WRAP_M(30)};
+#undef MHC_WRAP_M
+
 constexpr int kWgFoldMaxN = 16;
 // Floats per token of the per-token factors of d r / d b (and h_pre up to
 // capacity 8).
 constexpr int kWgEp = 16;
 bool wgen_supported(int n, int64_t C);
-hipError_t launch_wgen_fwd(int dt, int n, bool decay, const void* res, const void* br, const float* w,
-                           const float* coef, int64_t coef_stride, float* out, int64_t B, int64_t C, float eps,
-                           hipStream_t s);
-// Waves of the static-H row sums (rows of its scal_out) are 4 x this grid.
 int wgen_red_static_grid(int64_t B);
 // Row sums of the backward: stat = false: scal_out[B][n*n+2n+2] per token;
 // stat = true: scal_out[4 * wgen_red_static_grid(B)][n*n+2n] per wave.
@@ -508,6 +514,18 @@ hipError_t launch_wfold_copy(int dt, const void* res, void* res_out, const void*
 hipError_t launch_wfold_proj(int dt, int n, bool decay, const void* res, const void* br, const float* phi_pre,
                              const float* phi_post, const float* phi_res, const void* weight, int w_dtype, float* w32,
                              void* pack, float* p_part, float* ss_part, int64_t B, int64_t C, int ks, hipStream_t s);
+
+// ---- wrapper_row.hip ---------------------------------------------------------
+// The wrapper's forward row pass at run-time n (coef: [h_pre | h_post | M] at
+// coef + b * coef_stride), C % 4 == 0, wgen_supported.
+hipError_t launch_wrow_fwd(int dt, int n, bool decay, const void* res, const void* br, const float* w,
+                           const float* coef, int64_t coef_stride, float* out, int64_t B, int64_t C, float eps,
+                           hipStream_t s);
+// launch_wgen_red's dynamic-H outputs except dM, for H_res gradients that vanish.
+bool wrow_red_ok(int dt, int n, bool decay, int64_t C);
+hipError_t launch_wrow_red(int dt, int n, bool decay, const float* g, const void* res, const void* br, const float* w,
+                           const float* coef, int64_t coef_stride, float* scal_out, float* ep_out, int64_t B,
+                           int64_t C, float eps, hipStream_t s);
 
 // ---- wrapper_bwd.hip ---------------------------------------------------------
 // The wrapper's dynamic-H backward after wgen_red / the coefficients, with the

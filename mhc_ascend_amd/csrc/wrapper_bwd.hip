@@ -43,11 +43,6 @@ __device__ __forceinline__ vf32x4_t vmfma(vu32x4_t a, vu32x4_t b, vf32x4_t c) {
                                                    c, 0, 0, 0);
 }
 
-constexpr double vb_pow01(int e) { return e <= 0 ? 1.0 : 0.1 * vb_pow01(e - 1); }
-// 0.1^(j-1) in fp32 (wrapper_gen.hip's kWgMult), j = 2..8
-constexpr float kVbMult[9] = {1.f, 0.f, (float)vb_pow01(1), (float)vb_pow01(2), (float)vb_pow01(3), (float)vb_pow01(4),
-                              (float)vb_pow01(5), (float)vb_pow01(6), (float)vb_pow01(7)};
-
 // 8 fp32 -> bf16 parts in operand order
 __device__ __forceinline__ void vsplit8(const float (&v)[8], vu32x4_t& hi, vu32x4_t& mid) {
 #pragma unroll
@@ -207,7 +202,7 @@ __global__ __launch_bounds__(kVbThreads) __attribute__((amdgpu_waves_per_eu(2)))
                         if (decay) {
 #pragma unroll
                             for (int j = 2; j < 8; ++j) {
-                                if (j < n) r = fmaf(kVbMult[j], rowp[(int64_t)j * C], r);
+                                if (j < n) r = fmaf(kWrapMult[j], rowp[(int64_t)j * C], r);
                             }
                         }
                     }
@@ -375,8 +370,8 @@ __global__ __launch_bounds__(kVbThreads) __attribute__((amdgpu_waves_per_eu(2)))
                     vu32x4_t x;
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        x[e] = pack_bf16x2(__uint_as_float(rr[2 * e] << 16) * kVbMult[j],
-                                           __uint_as_float(rr[2 * e + 1] << 16) * kVbMult[j]);
+                        x[e] = pack_bf16x2(__uint_as_float(rr[2 * e] << 16) * kWrapMult[j],
+                                           __uint_as_float(rr[2 * e + 1] << 16) * kWrapMult[j]);
                     acc[j][0] = vmfma(ah[0], x, acc[j][0]);
                     acc[j][0] = vmfma(al[0], x, acc[j][0]);
                 }
@@ -440,7 +435,7 @@ __global__ __launch_bounds__(kVbThreads) __attribute__((amdgpu_waves_per_eu(2)))
             // xa = cr r + h_1 b (+ the rounded streams): without them every
             // stream of r is a multiple of it (e1.w = sum_j w_j h_j); with them
             // stream 7 (1e-6 r) joins the multiple
-            const float cr = XS ? (NST > 7 ? fmaf(hp[7], kVbMult[7], hp[0]) : hp[0]) : e1.w;
+            const float cr = XS ? (NST > 7 ? fmaf(hp[7], kWrapMult[7], hp[0]) : hp[0]) : e1.w;
             const int col = wc0 + 4 * lg;
             const int boff = t * PITCH + col * (int)sizeof(TX);
             float rv[4], bv[4];
@@ -459,13 +454,13 @@ __global__ __launch_bounds__(kVbThreads) __attribute__((amdgpu_waves_per_eu(2)))
                 for (int j = 2; j < (NST < 7 ? NST : 7); ++j) {
 #pragma unroll
                     for (int i = 0; i < 4; i += 2) {
-                        const uint32_t x2 = pack_bf16x2(rv[i] * kVbMult[j], rv[i + 1] * kVbMult[j]);
+                        const uint32_t x2 = pack_bf16x2(rv[i] * kWrapMult[j], rv[i + 1] * kWrapMult[j]);
                         const float x0 = __uint_as_float(x2 << 16), x1 = __uint_as_float(x2 & 0xffff0000u);
                         xav[i] = fmaf(hp[j], x0, xav[i]);
                         xav[i + 1] = fmaf(hp[j], x1, xav[i + 1]);
                         if (j < 4) {  // wsq holds the streams past the fourth
-                            sxv[i] = fmaf(kVbMult[j], x0, sxv[i]);
-                            sxv[i + 1] = fmaf(kVbMult[j], x1, sxv[i + 1]);
+                            sxv[i] = fmaf(kWrapMult[j], x0, sxv[i]);
+                            sxv[i + 1] = fmaf(kWrapMult[j], x1, sxv[i + 1]);
                         }
                     }
                 }

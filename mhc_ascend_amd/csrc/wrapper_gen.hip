@@ -18,46 +18,33 @@
 //             w_j = 1, 0, 0.1, 0.01, ... (0 past stream 1 in 'zero' mode),
 //             dw = sum_tokens hs G xa / r.
 // Kernels:
-//   wgen_fwd_kernel    forward row pass, one wave per token
 //   wgen_red_kernel    backward row sums, one wave per token: the
-//                      coefficient backward's scalars per token (dynamic H)
-//                      or summed per wave (static H), and the per-token
-//                      factors of d r / d b
+//                      coefficient backward's scalars per token (dynamic H,
+//                      where wrapper_row.hip's sums do not do) or summed per
+//                      wave (static H), and the per-token factors of d r / d b
 //   wgen_dx_kernel     d r, d b (rounded once) and the dw partials:
 //                      workgroups of 1024 channels x one token tile; with
 //                      dynamic H it adds the layer projection backward's dX
 //                      folded over the streams (Sinkhorn settings where the
 //                      H_res rows of dP do not vanish, and shapes the fold
 //                      kernels do not take)
-//   wgen_dphi_mfma_kernel  dynamic H, H_res rows of dP vanishing, n <= 8, or
-//                      n <= 16 on rows of 2048 channels or more:
-//                      dPhi of the 2n pre / post rows from the rebuilt
-//                      streams (bf16 MFMA)
+//   wgen_dphi_mfma_kernel  dynamic H, H_res rows of dP vanishing, rows that
+//                      wrapper_bwd.hip does not take, n <= 8, or n <= 16 on
+//                      rows of 2048 channels or more: dPhi of the 2n pre /
+//                      post rows from the rebuilt streams (bf16 MFMA)
 //   wgen_dx_fold_kernel  the same case: d r, d b with dP . Phi folded over
 //                      the streams, and the dw partials
 //   wgen_synth_kernel  the stream rows [tokens, n*C] as the operand of the
 //                      layer's projection kernels (dynamic H: the forward's
-//                      in the storage dtype; the backward's in fp32 when the
-//                      fold kernels do not run)
+//                      in the storage dtype on rows that wrapper_proj.hip does
+//                      not take; the backward's in fp32 when none of the
+//                      kernels above run)
 #include "mhc_device.h"
 #include "mhc_internal.h"
 
 namespace mhc {
 
 namespace {
-
-constexpr double wg_pow01(int e) { return e <= 0 ? 1.0 : 0.1 * wg_pow01(e - 1); }
-
-// Decay multiplier of stream j >= 2: Python's 0.1 ** (j - 1) as fp32 (the
-// product r * m is formed in fp32 by the reference's mul; the double
-// repeated product rounds to the same fp32 value as 0.1 ** e for e <= 63).
-#define MHC_WG_M(e) (float)wg_pow01(e)
-constexpr float kWgMult[kWgMaxN] = {
-    1.f,          0.f,          MHC_WG_M(1),  MHC_WG_M(2),  MHC_WG_M(3),  MHC_WG_M(4),  MHC_WG_M(5),  MHC_WG_M(6),
-    MHC_WG_M(7),  MHC_WG_M(8),  MHC_WG_M(9),  MHC_WG_M(10), MHC_WG_M(11), MHC_WG_M(12), MHC_WG_M(13), MHC_WG_M(14),
-    MHC_WG_M(15), MHC_WG_M(16), MHC_WG_M(17), MHC_WG_M(18), MHC_WG_M(19), MHC_WG_M(20), MHC_WG_M(21), MHC_WG_M(22),
-    MHC_WG_M(23), MHC_WG_M(24), MHC_WG_M(25), MHC_WG_M(26), MHC_WG_M(27), MHC_WG_M(28), MHC_WG_M(29), MHC_WG_M(30)};
-#undef MHC_WG_M
 
 template <typename TX>
 __device__ __forceinline__ float wg_round(float v) {
@@ -73,13 +60,13 @@ template <typename TX, bool DECAY>
 __device__ __forceinline__ float wg_stream(int j, float r, float b) {
     if (j == 0) return r;
     if (j == 1) return b;
-    return DECAY ? wg_round<TX>(r * kWgMult[j]) : 0.f;
+    return DECAY ? wg_round<TX>(r * kWrapMult[j]) : 0.f;
 }
 
 // d r weight of stream j.
 template <bool DECAY>
 __device__ __forceinline__ float wg_rweight(int j) {
-    return j == 0 ? 1.f : (j == 1 ? 0.f : (DECAY ? kWgMult[j] : 0.f));
+    return j == 0 ? 1.f : (j == 1 ? 0.f : (DECAY ? kWrapMult[j] : 0.f));
 }
 
 // h_pre, cm = (1/n) column sums of M and hs = (1/n) sum h_post of one token
@@ -140,79 +127,6 @@ __device__ __forceinline__ float wg_xa(float r, float b, const float (&hp)[NM], 
 constexpr int kWgU = 4;  // 4-channel chunks per lane in flight
 
 }  // namespace
-
-// ---------------------------------------------------------------------------
-// Forward row pass: one wave per token, 4-channel chunks (lane l takes
-// chunks l, l + 64, ...).  Pass 1 forms sum xa^2 (r and b read through the
-// cache), pass 2 reads them again (last use) with the weight and stores the
-// fp32 output.
-// ---------------------------------------------------------------------------
-template <typename TX, int NM, bool DECAY>
-__global__ __launch_bounds__(256) void wgen_fwd_kernel(const TX* __restrict__ res, const TX* __restrict__ br,
-                                                       const float* __restrict__ w, const float* __restrict__ coef,
-                                                       int64_t coef_stride, float* __restrict__ out, int64_t B, int C,
-                                                       int n, float eps) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t b = (int64_t)blockIdx.x * (blockDim.x / kWave) + (int64_t)wave_uniform(threadIdx.x / kWave);
-    if (b >= B) return;
-    float hp[NM], cm[NM], hs;
-    wg_coefs<NM>(coef + b * coef_stride, n, hp, cm, hs);
-    const TX* rb = res + b * (int64_t)C;
-    const TX* bb = br + b * (int64_t)C;
-    const int nq = C / 4;
-    float ss = 0.f;
-    for (int q0 = 0; q0 < nq; q0 += kWgU * kWave) {
-        float rv[kWgU][4], bv[kWgU][4];
-#pragma unroll
-        for (int u = 0; u < kWgU; ++u) {
-            const int q = q0 + u * kWave + lane;
-            const int c0 = (q < nq ? q : 0) * 4;
-            load_run<TX, 4>(rb + c0, rv[u]);
-            load_run<TX, 4>(bb + c0, bv[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kWgU; ++u) {
-            if (q0 + u * kWave + lane >= nq) continue;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float xa = wg_xa<TX, NM, DECAY>(rv[u][e], bv[u][e], hp, n);
-                ss += xa * xa;
-            }
-        }
-    }
-    float t[1] = {ss};
-    wave_sum<1>(t);
-    const float inv = 1.f / sqrtf(t[0] / (float)C + eps);
-    float* ob = out + b * (int64_t)C;
-    for (int q0 = 0; q0 < nq; q0 += kWgU * kWave) {
-        float rv[kWgU][4], bv[kWgU][4], wv[kWgU][4];
-#pragma unroll
-        for (int u = 0; u < kWgU; ++u) {
-            const int q = q0 + u * kWave + lane;
-            const int c0 = (q < nq ? q : 0) * 4;
-            load_run_nt<TX, 4>(rb + c0, rv[u]);
-            load_run_nt<TX, 4>(bb + c0, bv[u]);
-            load_run<float, 4>(w + c0, wv[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kWgU; ++u) {
-            const int q = q0 + u * kWave + lane;
-            if (q >= nq) continue;
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float r = rv[u][e], bvv = bv[u][e];
-                float s = hs * (wg_xa<TX, NM, DECAY>(r, bvv, hp, n) * inv * wv[u][e]);
-#pragma unroll
-                for (int j = 0; j < NM; ++j) {
-                    if (j < n) s += cm[j] * wg_stream<TX, DECAY>(j, r, bvv);
-                }
-                o[e] = s;
-            }
-            store_run_nt<float, 4>(ob + q * 4, o);
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Backward row sums, one wave per token: ss = sum xa^2, gwx = sum w G xa,
@@ -434,7 +348,7 @@ __global__ __launch_bounds__(256) void wgen_dx_kernel(const float* __restrict__ 
                 a += dx[0][q] + sv * rv[q];
 #pragma unroll
                 for (int j = 2; j < NM; ++j) {
-                    if (j < n && DECAY) a += kWgMult[j] * (dx[j][q] + sv * wg_stream<TX, DECAY>(j, rv[q], bv[q]));
+                    if (j < n && DECAY) a += kWrapMult[j] * (dx[j][q] + sv * wg_stream<TX, DECAY>(j, rv[q], bv[q]));
                 }
                 c += dx[1][q] + sv * bv[q];
             }
@@ -659,7 +573,7 @@ __global__ __launch_bounds__(256) void wgen_dx_fold_kernel(
                 vr = row[c0 + e];
 #pragma unroll
                 for (int j = 2; j < NM; ++j) {
-                    if (j < n && DECAY) vr += kWgMult[j] * row[(int64_t)j * C + c0 + e];
+                    if (j < n && DECAY) vr += kWrapMult[j] * row[(int64_t)j * C + c0 + e];
                 }
                 vb = row[C + c0 + e];
             }
@@ -708,7 +622,7 @@ __global__ __launch_bounds__(256) void wgen_dx_fold_kernel(
             float xs = rv[q];
 #pragma unroll
             for (int j = 2; j < NM; ++j) {
-                if (j < n && DECAY) xs += kWgMult[j] * wg_stream<TX, DECAY>(j, rv[q], bv[q]);
+                if (j < n && DECAY) xs += kWrapMult[j] * wg_stream<TX, DECAY>(j, rv[q], bv[q]);
             }
             dr[q] = e0 * gq + e1 * wg + e5 * xa + pa + sv * xs;
             db[q] = e2 * gq + e3 * wg + e6 * xa + pc + sv * bv[q];
@@ -795,22 +709,6 @@ bool wgen_supported(int n, int64_t C) { return n >= 2 && n <= kWgMaxN && C >= 4 
     }
 #define MHC_WG_DISPATCH(dt, decay, n, ...) MHC_WG_DISPATCH_BY(MHC_WG_NM, dt, decay, n, __VA_ARGS__)
 #define MHC_WG_DISPATCH_WIDE(dt, decay, n, ...) MHC_WG_DISPATCH_BY(MHC_WG_NM_WIDE, dt, decay, n, __VA_ARGS__)
-
-hipError_t launch_wgen_fwd(int dt, int n, bool decay, const void* res, const void* br, const float* w,
-                           const float* coef, int64_t coef_stride, float* out, int64_t B, int64_t C, float eps,
-                           hipStream_t s) {
-    if (B == 0) return hipSuccess;
-    if (!wgen_supported(n, C)) return hipErrorInvalidValue;
-    const int64_t blocks = (B + 3) / 4;  // one token per wave
-    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    const int Ci = (int)C;
-    const int tok = timing_begin("wrap_fwd", s);
-    MHC_WG_DISPATCH_WIDE(dt, decay, n,
-                    MHC_LAUNCH_GGL((wgen_fwd_kernel<TX_, NM_, D_>), dim3((unsigned)blocks), dim3(256), 0, s,
-                                   (const TX_*)res, (const TX_*)br, w, coef, coef_stride, out, B, Ci, n, eps));
-    timing_end(tok, s);
-    return hipGetLastError();
-}
 
 int wgen_red_static_grid(int64_t B) {
     int64_t g = (B + 3) / 4;

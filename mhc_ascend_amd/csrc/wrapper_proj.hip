@@ -59,7 +59,7 @@ __device__ __forceinline__ float wdot2(uint32_t a, uint32_t b, float c) {
 __device__ __forceinline__ float wlo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float whi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// 0.1^(j-1) as Python's product gives it in fp32 (wrapper_gen.hip's kWgMult)
+// 0.1^(j-1) as Python's product gives it in fp32
 constexpr double wp_pow01(int e) { return e <= 0 ? 1.0 : 0.1 * wp_pow01(e - 1); }
 constexpr float kWpMult[7] = {1.f, 0.f, (float)wp_pow01(1), (float)wp_pow01(2), (float)wp_pow01(3),
                               (float)wp_pow01(4), (float)wp_pow01(5)};
