@@ -42,11 +42,12 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) { return pack_
 // fp32 -> three bf16 terms: v = hi + mid + lo exactly up to the last bit
 // for normal values (3 x 8 significant bits = the fp32 mantissa).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void split3(float v, float& h, float& m, float& l) {
-    h = bf16_to_f32(f32_to_bf16(v));
-    const float r = v - h;
-    m = bf16_to_f32(f32_to_bf16(r));
-    l = r - m;
+// Two values at a time, each term packed as it is rounded.
+__device__ __forceinline__ void split3(float v0, float v1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = pack_bf16(v0, v1);
+    const float r0 = v0 - __uint_as_float(h << 16), r1 = v1 - __uint_as_float(h & 0xffff0000u);
+    m = pack_bf16(r0, r1);
+    l = pack_bf16(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
 }
 
 // Phi -> bf16 planes in MFMA B-fragment order, p = hi / mid / lo:
@@ -87,12 +88,7 @@ __global__ __launch_bounds__(256) void phi_split_kernel(const float* __restrict_
         uint32_t w[3][4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            float h0, m0, l0, h1, m1, l1;
-            split3(v[2 * e], h0, m0, l0);
-            split3(v[2 * e + 1], h1, m1, l1);
-            w[0][e] = pack_bf16(h0, h1);
-            w[1][e] = pack_bf16(m0, m1);
-            w[2][e] = pack_bf16(l0, l1);
+            split3(v[2 * e], v[2 * e + 1], w[0][e], w[1][e], w[2][e]);
         }
 #pragma unroll
         for (int p = 0; p < 3; ++p)
@@ -238,12 +234,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     ss[mt] += v[2 * e] * v[2 * e] + v[2 * e + 1] * v[2 * e + 1];
-                    float h0, m0, l0, h1, m1, l1;
-                    split3(v[2 * e], h0, m0, l0);
-                    split3(v[2 * e + 1], h1, m1, l1);
-                    ah[e] = pack_bf16(h0, h1);
-                    am[e] = pack_bf16(m0, m1);
-                    al[e] = pack_bf16(l0, l1);
+                    uint32_t hh, mm, ll;
+                    split3(v[2 * e], v[2 * e + 1], hh, mm, ll);
+                    ah[e] = hh;
+                    am[e] = mm;
+                    al[e] = ll;
                 }
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
@@ -349,13 +344,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 // fragment-order planes of phi_split_kernel instead, as packed for the
 // forward-only entry).  Products as proj_mfma_kernel: bf16 x:
 // x.(hi + mid + lo); fp32 x: xh.(hi + mid + lo) + xm.(hi + mid) + xl.hi.
+// Bound by the split and the MFMAs, which one wave runs in turn (38% and 42% of
+// the cycles by the counters).
 // Partials p_part[tile][ks][B][32], the layout proj_mfma_kernel writes;
 // with bf16 x the workgroups of output block 0 also store ss_part[ks][B]
-// (fp32 x: proj_xsplit_kernel stores it).  Workgroups that stage the same x
-// (same token block and K range) get ids on one XCD.
+// (fp32 x: proj_xsplit_kernel stores it).
 // ---------------------------------------------------------------------------
 constexpr int kStreamOB = 128;                    // output rows per workgroup (32 per wave)
 constexpr int kStreamKS = 64;                     // k per LDS stage
+constexpr int kStreamTC = 4;                      // token blocks of a chunk (ids of one XCD)
 constexpr int kStreamPitch = kStreamKS * 2 + 16;  // bytes per staged row of one plane
 
 // fp32 x -> xp[3][B][K] bf16 (split3 per element) and ss_part[q][b] = sum
@@ -377,12 +374,7 @@ __global__ __launch_bounds__(256) void proj_xsplit_kernel(const float* __restric
         uint32_t w[3][4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            float h0, m0, l0, h1, m1, l1;
-            split3(v[2 * e], h0, m0, l0);
-            split3(v[2 * e + 1], h1, m1, l1);
-            w[0][e] = pack_bf16(h0, h1);
-            w[1][e] = pack_bf16(m0, m1);
-            w[2][e] = pack_bf16(l0, l1);
+            split3(v[2 * e], v[2 * e + 1], w[0][e], w[1][e], w[2][e]);
             ss[0] += v[2 * e] * v[2 * e] + v[2 * e + 1] * v[2 * e + 1];
         }
         const int64_t pc = (b * K + k) / 8;
@@ -397,7 +389,7 @@ template <int XPL, int MT, bool PHI_PLANES>
 __global__ __launch_bounds__(256) void proj_stream_kernel(
     const bf16_t* __restrict__ xpl, const float* __restrict__ phi_pre, const float* __restrict__ phi_post,
     const float* __restrict__ phi_res, int n_pre, const uint4* __restrict__ phif, int np, float* __restrict__ p_part,
-    float* __restrict__ ss_part, int64_t B, int64_t K, int64_t kchunk, int ks, int oblocks, int64_t groups) {
+    float* __restrict__ ss_part, int64_t B, int64_t K, int64_t kchunk, int ks, int oblocks, int64_t tblocks) {
     constexpr int TB = 16 * MT;
     constexpr int KS = kStreamKS;
     constexpr int PITCH = kStreamPitch;
@@ -409,15 +401,20 @@ __global__ __launch_bounds__(256) void proj_stream_kernel(
     const int wave = threadIdx.x >> 6;
     const int row = lane & 15;
     const int kg = lane >> 4;
-    // id = 8 (gq * oblocks + oi) + gx for group g = 8 gq + gx (token block
-    // x K range): one group's output blocks share an XCD
+    // XCD lin % 8 takes a run of the workgroups ordered by K range, then by
+    // chunk of kStreamTC token blocks, output block and token block: a chunk's
+    // workgroups share its x, and its Phi with the next output blocks' x, in L2
     const int64_t lin = blockIdx.x;
-    const int64_t rest = lin / 8;
-    const int oi = (int)(rest % oblocks);
-    const int64_t grp = (rest / oblocks) * 8 + lin % 8;
-    if (grp >= groups) return;
-    const int64_t tblk = grp / ks;
-    const int ksplit = (int)(grp % ks);
+    const int64_t per = gridDim.x / 8;
+    const int64_t unit = (lin % 8) * per + lin / 8;
+    if (unit >= ks * tblocks * oblocks) return;
+    const int ksplit = (int)(unit / (tblocks * oblocks));
+    const int64_t rem = unit % (tblocks * oblocks);
+    const int64_t chunk0 = rem / (kStreamTC * oblocks) * kStreamTC;
+    const int64_t in_chunk = tblocks - chunk0 < kStreamTC ? tblocks - chunk0 : kStreamTC;
+    const int64_t rem2 = rem - chunk0 * oblocks;
+    const int oi = (int)(rem2 / in_chunk);
+    const int64_t tblk = chunk0 + rem2 % in_chunk;
     const int64_t tok0 = tblk * TB;
     const int ow = oi * kStreamOB + 32 * wave;  // the wave's output tile: rows ow .. ow + 31
     const bool wave_on = ow < np;
@@ -518,12 +515,11 @@ __global__ __launch_bounds__(256) void proj_stream_kernel(
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                float h0, m0, l0, h1, m1, l1;
-                split3(ps.f[kk][nt][2 * e], h0, m0, l0);
-                split3(ps.f[kk][nt][2 * e + 1], h1, m1, l1);
-                h[e] = pack_bf16(h0, h1);
-                m[e] = pack_bf16(m0, m1);
-                l[e] = pack_bf16(l0, l1);
+                uint32_t hh, mm, ll;
+                split3(ps.f[kk][nt][2 * e], ps.f[kk][nt][2 * e + 1], hh, mm, ll);
+                h[e] = hh;
+                m[e] = mm;
+                l[e] = ll;
             }
         }
     };
@@ -1593,10 +1589,9 @@ __global__ __launch_bounds__(1024) void small_column_sum_kernel(const float* __r
 __device__ __forceinline__ void split_pack8(const float (&v)[8], u32x4_t& hi, u32x4_t& lo) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const float h0 = bf16_to_f32(f32_to_bf16(v[2 * e]));
-        const float h1 = bf16_to_f32(f32_to_bf16(v[2 * e + 1]));
-        hi[e] = pack_bf16(h0, h1);
-        lo[e] = pack_bf16(v[2 * e] - h0, v[2 * e + 1] - h1);
+        const uint32_t h = pack_bf16(v[2 * e], v[2 * e + 1]);
+        hi[e] = h;
+        lo[e] = pack_bf16(v[2 * e] - __uint_as_float(h << 16), v[2 * e + 1] - __uint_as_float(h & 0xffff0000u));
     }
 }
 
@@ -1962,23 +1957,30 @@ static const void* proj_stream_fn(int mt) {
 // x re-reads are few, is faster.
 bool proj_stream_path(int np) { return np > kStreamOB; }
 
-// K splits of the streaming projection: token blocks x output blocks x
-// splits fill two rounds of resident workgroups (occupancy of the fp32-x
-// kernel, whose LDS stage is the larger), at least two stages per split.
+// K splits of the streaming projection: the count whose rounds of resident
+// workgroups (occupancy of the fp32-x kernel, whose LDS stage is the larger)
+// take the fewest stages, three added per workgroup for its prologue and
+// stores; at least two stages per split, splits x tokens at most 4096 (the
+// partials the coefficient kernel adds per token).  n = 32, 128 tokens, C =
+// 1280: 28 splits are 504 workgroups, one round; 32, the cap, left 64 of 576 to
+// a second one (110 us, 88 with the workgroup order and the packed split below).
 static int proj_stream_ksplit(int64_t B, int64_t K, int np) {
     const int mt = proj_stream_mt(B);
     const int64_t groups0 = ((B + 16 * mt - 1) / (16 * mt)) * ((np + kStreamOB - 1) / kStreamOB);
     const int per_cu = occupancy_per_cu(proj_stream_fn<3, 0>(mt), 256, 0);
-    // rounded down: a last partial round would leave most CUs idle while it
-    // runs; splits x tokens at most 4096 (the partials the coefficient
-    // kernel adds per token: 32 splits at 128 tokens, 128 at 32)
-    int64_t ks = 2 * (int64_t)device_cu_count() * per_cu / groups0;
+    const int64_t slots = (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : 1);
+    const int64_t stages = (K + kStreamKS - 1) / kStreamKS;
     const int64_t kcap = B > 0 ? (4096 + B - 1) / B : 1;
-    if (ks > kcap) ks = kcap;
-    const int64_t kmax = (K + 2 * kStreamKS - 1) / (2 * kStreamKS);
-    if (ks > kmax) ks = kmax;
-    if (ks < 1) ks = 1;
-    return (int)ks;
+    const int64_t kmax = (stages + 1) / 2;
+    int64_t best = 1, best_cost = 0;
+    for (int64_t ks = 1; ks <= kcap && ks <= kmax; ++ks) {
+        const int64_t cost = (groups0 * ks + slots - 1) / slots * ((stages + ks - 1) / ks + 3);
+        if (ks == 1 || cost * 50 < best_cost * 49) {
+            best = ks;
+            best_cost = cost;
+        }
+    }
+    return (int)best;
 }
 
 // K splits so that token blocks x splits x output tiles fill about two
@@ -2029,8 +2031,7 @@ hipError_t launch_proj_stream(int x_dtype, const void* x, bf16_raw_t* xplanes, c
     const int mt = proj_stream_mt(B);
     const int64_t tb = (B + 16 * mt - 1) / (16 * mt);
     const int ob = (np + kStreamOB - 1) / kStreamOB;
-    const int64_t groups = tb * ks;
-    const dim3 grid((unsigned)(((groups + 7) / 8) * 8 * ob));
+    const dim3 grid((unsigned)((tb * ks * ob + 7) / 8 * 8));
     const int tok = timing_begin("proj", s);
     const bf16_t* xp = reinterpret_cast<const bf16_t*>(x);
     if (x_dtype == kF32) {
@@ -2042,10 +2043,10 @@ hipError_t launch_proj_stream(int x_dtype, const void* x, bf16_raw_t* xplanes, c
 #define MHC_STREAM(XPL_, MT_)                                                                                   \
     if (phib) {                                                                                                 \
         MHC_LAUNCH_GGL((proj_stream_kernel<XPL_, MT_, true>), grid, dim3(256), 0, s, xp, phi_pre, phi_post,   \
-                           phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, groups);                                                          \
+                           phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, tb);                                                          \
     } else {                                                                                                    \
         MHC_LAUNCH_GGL((proj_stream_kernel<XPL_, MT_, false>), grid, dim3(256), 0, s, xp, phi_pre, phi_post,  \
-                           phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, groups);                                                          \
+                           phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, tb);                                                          \
     }
 #define MHC_STREAM_MT(XPL_)                               \
     if (mt == 2) {                                        \
@@ -2400,7 +2401,7 @@ hipError_t launch_small_column_sum(const float* part, int rows, int cols, float*
 //     dx = dx_proj + (ACC ? dx : 0) + s x.
 //   dp_tsplit_kernel + x_tsplit_kernel + proj_bwd_dphi_kernel: dP and x
 //     split once into transposed hi / lo planes (tokens contiguous); one
-//     workgroup per 128 output rows x 128 columns walks all tokens,
+//     workgroup per 64 output rows x 128 columns walks all tokens,
 //     dPhi = dP^T x in MFMA registers, and stores its rows of dPhi directly
 //     (no partials, no column sums).  The row blocks of one column block get
 //     ids on one XCD, so they share those x columns through its L2.
@@ -2459,17 +2460,18 @@ __global__ __launch_bounds__(256) void proj_bwd_dx_small_kernel(
     // dP columns are read 8 at a time: a stride that is a multiple of 8
     // allows the aligned 16-byte loads (the layer's dP rows are)
     const bool dp_vec = (dp_stride % 8) == 0;
-    // A = Phi^T: Phi[o0 + 8 lg + e][column 16 ct + lr]; the next tile's
-    // values are loaded while the current tile is on the matrix cores
+    // A = Phi^T: Phi[o0 + 8 lg + e][column 2 lr + ct], both column tiles of a
+    // row from one 128-byte line; the next tile's values are loaded while the
+    // current tile is on the matrix cores
     float pv[2][8];
     auto load_phi = [&](int o0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int o = o0 + 8 * lg + e;
-                pv[ct][e] = o < np ? phi_row(phi_pre, phi_post, phi_res, n_pre, o, K)[kb0 + 16 * ct + lr] : 0.f;
-            }
+        for (int e = 0; e < 8; ++e) {
+            const int o = o0 + 8 * lg + e;
+            float2 q = make_float2(0.f, 0.f);
+            if (o < np) q = *reinterpret_cast<const float2*>(phi_row(phi_pre, phi_post, phi_res, n_pre, o, K) + kb0 + 2 * lr);
+            pv[0][e] = q.x;
+            pv[1][e] = q.y;
         }
     };
     load_phi(0);
@@ -2503,7 +2505,7 @@ __global__ __launch_bounds__(256) void proj_bwd_dx_small_kernel(
             }
         }
     }
-    // D[column 16 ct + 4 lg + i][token 16 tt + lr]: four consecutive columns of one token
+    // D[column 2 (4 lg + i) + ct][token 16 tt + lr]: eight consecutive columns of one token
 #pragma unroll
     for (int st = 0; st < TS; ++st) {
 #pragma unroll
@@ -2512,9 +2514,10 @@ __global__ __launch_bounds__(256) void proj_bwd_dx_small_kernel(
             if (t >= B) continue;
             const float sv = HAS_S ? s_tok[t] : 0.f;
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct) {
-                const int64_t off = t * K + kb0 + 16 * ct + 4 * lg;
-                float4 o = make_float4(d[st][tt][ct][0], d[st][tt][ct][1], d[st][tt][ct][2], d[st][tt][ct][3]);
+            for (int h = 0; h < 2; ++h) {
+                const int64_t off = t * K + kb0 + 8 * lg + 4 * h;
+                float4 o = make_float4(d[st][tt][0][2 * h], d[st][tt][1][2 * h], d[st][tt][0][2 * h + 1],
+                                       d[st][tt][1][2 * h + 1]);
                 if constexpr (ACC) {
                     const float4 a = *reinterpret_cast<const float4*>(dx + off);
                     o.x += a.x; o.y += a.y; o.z += a.z; o.w += a.w;
@@ -2567,18 +2570,19 @@ __global__ __launch_bounds__(256) void proj_bwd_dphi_small_kernel(const float* _
             }
             split_pack8(v, ah[ot], al[ot]);
         }
-        // B = x: tokens t0 + 8 lg + e, column 16 ct + lr
+        // B = x: tokens t0 + 8 lg + e, columns 2 lr + ct (whole 128-byte lines)
         u32x4_t xh[2], xl[2];
+        float v0[8], v1[8];
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int64_t t = t0 + 8 * lg + e;
-                v[e] = t < B ? x[t * K + kb0 + 16 * ct + lr] : 0.f;
-            }
-            split_pack8(v, xh[ct], xl[ct]);
+        for (int e = 0; e < 8; ++e) {
+            const int64_t t = t0 + 8 * lg + e;
+            float2 q = make_float2(0.f, 0.f);
+            if (t < B) q = *reinterpret_cast<const float2*>(x + t * K + kb0 + 2 * lr);
+            v0[e] = q.x;
+            v1[e] = q.y;
         }
+        split_pack8(v0, xh[0], xl[0]);
+        split_pack8(v1, xh[1], xl[1]);
 #pragma unroll
         for (int ot = 0; ot < OT; ++ot) {
 #pragma unroll
@@ -2589,15 +2593,15 @@ __global__ __launch_bounds__(256) void proj_bwd_dphi_small_kernel(const float* _
             }
         }
     }
-    // D[o 16 ot + 4 lg + i][column 16 ct + lr]
+    // D[o 16 ot + 4 lg + i][column 2 lr + ct]
 #pragma unroll
     for (int ot = 0; ot < OT; ++ot) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int o = o0 + 16 * ot + 4 * lg + i;
             if (o >= np) continue;
-#pragma unroll
-            for (int ct = 0; ct < 2; ++ct) dphi[(int64_t)o * K + kb0 + 16 * ct + lr] = acc[ot][ct][i];
+            *reinterpret_cast<float2*>(dphi + (int64_t)o * K + kb0 + 2 * lr) =
+                make_float2(acc[ot][0][i], acc[ot][1][i]);
         }
     }
 }
@@ -2630,7 +2634,10 @@ __global__ __launch_bounds__(256) void dp_split_kernel(const float* __restrict__
 // the four waves, double-buffered; the Phi fragments (A = Phi^T: 8 outputs
 // of one column per lane, two tiles) are loaded two output tiles ahead.
 // Products hi.hi + lo.hi + hi.lo (as proj_bwd_mfma_kernel); then
-// dx = dx_proj + (ACC ? dx : 0) + (HAS_S ? s x : 0).
+// dx = dx_proj + (ACC ? dx : 0) + (HAS_S ? s x : 0).  Bound by the vector work
+// of a CU with two workgroups (320 at K = 40960): row addresses from scalar
+// bases within phi_res and packed splits took 85 us to 76 at n = 32, 128 tokens
+// (300 tokens: 169 to 146); 16 columns a wave took 90, Phi through LDS 147.
 constexpr int kDx2Tok = 128;                 // tokens per workgroup
 constexpr int kDx2Pitch = 64 + 16;           // bytes per token row of one dP plane tile in LDS
 
@@ -2688,12 +2695,23 @@ __global__ __launch_bounds__(256) void proj_bwd_dx2_kernel(
             *reinterpret_cast<uint4*>(&dps[buf][pl][r * PITCH + 16 * c]) = f[u];
         }
     };
+    // element offset of the lane's columns in a tile's row 8 lg (24 K + K < 2^27)
+    const uint32_t res_off = (uint32_t)(8 * lg * K + (wave_on ? kb0 + lr : 0));
     // A = Phi^T fragments of output tile ot: Phi[32 ot + 8 lg + e][kb0 + 16 ct + lr]
     struct PhiTile {
         float v[2][8];
     };
     auto fetch_phi = [&](PhiTile& pt, int ot) __attribute__((always_inline)) {
         const int64_t col = wave_on ? kb0 + lr : 0;
+        if (32 * ot >= 2 * n_pre && 32 * ot + 32 <= np) {  // a tile of phi_res: scalar row bases
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float* base = phi_res + (int64_t)(32 * ot + e - 2 * n_pre) * K;
+                pt.v[0][e] = base[res_off];
+                pt.v[1][e] = base[res_off + 16];
+            }
+            return;
+        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int o = 32 * ot + 8 * lg + e;
@@ -2795,8 +2813,10 @@ __global__ __launch_bounds__(256) void dp_tsplit_kernel(const float* __restrict_
     tl[i] = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-//   xT[k][t] from x[t][k]: a 32-token x 64-column tile through LDS (loads
-//   along k, stores along t).
+//   x^T in MFMA fragment order, 16 columns x 32 tokens as 64 lanes' 16-byte
+//   pieces (lane 16 g + c: column c, tokens 8 g .. + 7), so that a fragment is
+//   1 KB contiguous and not 16 half cache lines: a 32-token x 64-column tile
+//   through LDS.
 constexpr int kXtCols = 64;
 __global__ __launch_bounds__(256) void x_tsplit_kernel(const float* __restrict__ x, int64_t B, int64_t K, int64_t Bp,
                                                        uint4* __restrict__ th, uint4* __restrict__ tl) {
@@ -2821,21 +2841,25 @@ __global__ __launch_bounds__(256) void x_tsplit_kernel(const float* __restrict__
     for (int e = 0; e < 8; ++e) v[e] = tile[8 * g + e][c];
     u32x4_t h, l;
     split_pack8(v, h, l);
-    const int64_t idx = (k * Bp + t0 + 8 * g) / 8;
+    const int64_t idx = ((k / 16) * (Bp / 32) + tb) * 64 + g * 16 + k % 16;
     th[idx] = make_uint4(h[0], h[1], h[2], h[3]);
     tl[idx] = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-// dPhi rows: one workgroup per 128 output rows x 128 columns walks all
+// dPhi rows: one workgroup per 64 output rows x 128 columns walks all
 // tokens, dPhi = hi.hi + lo.hi + hi.lo in MFMA registers, its rows stored
-// directly (non-temporal).  A = dP^T (the workgroup's 128 rows, shared by
-// its four waves)
+// directly (non-temporal).  Bound by its L2 reads (96 KB a workgroup for 32 KB
+// written): n = 32, 128 tokens, C = 1280: 48 us (178 MB written); 72 with x^T
+// column by column, whose fragments were 16 half lines, and the staging's loads
+// one at a time behind index divisions; 128 rows left two workgroups a CU, 51
+// for 41 us at n = 16, 600 tokens.
+// A = dP^T (the workgroup's 64 rows, shared by its four waves)
 // goes through LDS 128 tokens at a time; B = x^T fragments of the wave's
 // own 32 columns come straight from the transposed planes, the next 32
 // tokens' in flight while the current ones are on the matrix cores.  The
 // row blocks of one column block get ids on one XCD, sharing those x
 // columns through its L2.
-constexpr int kDphiRows = 128;                // output rows (four 32-row tiles) per dPhi workgroup
+constexpr int kDphiRows = 64;                 // output rows per dPhi workgroup
 constexpr int kDphiTok = 128;                 // tokens per LDS chunk of dP^T
 constexpr int kDphiPitch = kDphiTok * 2 + 16;  // bytes per row of one plane in LDS
 
@@ -2872,31 +2896,42 @@ __global__ __launch_bounds__(256) void proj_bwd_dphi_kernel(const uint4* __restr
         uint4 h[2], l[2];
     };
     auto load_b = [&](BFrag& f, int64_t t0) __attribute__((always_inline)) {
-        const int64_t tp = (t0 + 8 * lg) / 8;
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct) {
-            const int64_t r = (wave_on ? kb0 + 16 * ct + lr : 0) * rowp + tp;
+            const int64_t r = ((wave_on ? kb0 / 16 + ct : 0) * (Bp / 32) + t0 / 32) * 64 + lane;
             f.h[ct] = xth[r];
             f.l[ct] = xtl[r];
         }
     };
+    BFrag fa, fb;
     for (int64_t c0 = 0; c0 < Bp; c0 += kDphiTok) {
         const int tc = Bp - c0 < kDphiTok ? (int)(Bp - c0) : kDphiTok;  // a multiple of 32
-        // dP^T rows o0 .. o0 + 63, tokens c0 .. c0 + tc - 1, both planes:
+        // the first x fragments in flight while dP^T is staged
+        load_b(fa, c0);
+        if (tc > 32) load_b(fb, c0 + 32);
+        // dP^T rows o0 .. o0 + 63, tokens c0 .. c0 + tc - 1, both planes, all
+        // loads before the first write:
         // piece i = (plane, row, 16-byte column)
-        const int pieces = 2 * kDphiRows * (tc / 8);
-        for (int i = threadIdx.x; i < pieces; i += 256) {
-            const int pl = i / (kDphiRows * (tc / 8));
-            const int r = (i / (tc / 8)) % kDphiRows;
-            const int c = i % (tc / 8);
-            const uint4* src = pl == 0 ? dth : dtl;
-            *reinterpret_cast<uint4*>(&as[pl][r * PITCH + 16 * c]) = src[(int64_t)(o0 + r) * rowp + c0 / 8 + c];
+        constexpr int PR = kDphiTok / 8;  // pieces per row (those past tc stay unread)
+        constexpr int PPT = 2 * kDphiRows * PR / 256;
+        uint4 st[PPT];
+#pragma unroll
+        for (int u = 0; u < PPT; ++u) {
+            const int i = threadIdx.x + 256 * u;
+            const int r = (i / PR) % kDphiRows;
+            const int c = i % PR < tc / 8 ? i % PR : 0;
+            st[u] = (256 * u < kDphiRows * PR ? dth : dtl)[(int64_t)(o0 + r) * rowp + c0 / 8 + c];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < PPT; ++u) {
+            const int i = threadIdx.x + 256 * u;
+            *reinterpret_cast<uint4*>(&as[256 * u / (kDphiRows * PR)][(i / PR) % kDphiRows * PITCH + 16 * (i % PR)]) =
+                st[u];
         }
         __syncthreads();
         if (wave_on) {
-            BFrag fa, fb;
             int t = 0;
-            load_b(fa, c0);
             auto mma = [&](const BFrag& f, int tt) __attribute__((always_inline)) {
 #pragma unroll
                 for (int ot = 0; ot < OT; ++ot) {
@@ -2912,10 +2947,10 @@ __global__ __launch_bounds__(256) void proj_bwd_dphi_kernel(const uint4* __restr
                 }
             };
             for (; t + 64 <= tc; t += 64) {
-                load_b(fb, c0 + t + 32);
                 mma(fa, t);
                 if (t + 64 < tc) load_b(fa, c0 + t + 64);
                 mma(fb, t + 32);
+                if (t + 96 < tc) load_b(fb, c0 + t + 96);
             }
             if (t < tc) mma(fa, t);
         }
