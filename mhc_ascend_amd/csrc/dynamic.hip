@@ -58,7 +58,7 @@ __device__ __forceinline__ void split3(float v0, float v1, uint32_t& h, uint32_t
 // phif + t * 6 * (K / 32) * 64 holding rows 32 t .. 32 t + 31; rows past np
 // are zero.  Grid-stride over tiles * 2 * (K / 32) * 64 fragments.
 // With w32 not null the same launch also converts the RMSNorm weight (wdt:
-// F32 or BF16, C elements) to fp32 (as weight_f32_kernel).
+// F32 or BF16, C elements) to fp32 (as convert_kernel).
 __global__ __launch_bounds__(256) void phi_split_kernel(const float* __restrict__ pre, const float* __restrict__ post,
                                                         const float* __restrict__ res, int n, int np, int64_t K,
                                                         uint4* __restrict__ phif, const void* __restrict__ wsrc,
