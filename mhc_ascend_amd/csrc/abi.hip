@@ -1015,13 +1015,15 @@ static DynBwdWs dyn_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_d
     w.pscale_off = o; o += align256((size_t)batch * w.groups * 4);
     w.cpart_off = o; o += align256((size_t)w.cblocks * (np + 3) * 4);
     // projection partials (per-tile path) or dP planes (all-tiles path)
-    size_t phip = (size_t)w.tiles * tile_rows((int)np) * K * 4;
+    const bool all = batch > 0 && w.wdt == kF32 && proj_bwd_tiles_path((int)np, batch);
+    const int64_t prows = all ? np : tile_rows((int)np);
+    size_t phip = (size_t)w.tiles * prows * K * 4;
     if (batch > 0 && proj_bwd_wide_path(w.wdt, (int)np, batch) &&
         phip < proj_bwd_wide_scratch_bytes((int)np, batch, K))
         phip = proj_bwd_wide_scratch_bytes((int)np, batch, K);
     w.phip_off = o; o += align256(phip);
     w.stw_off = o; o += align256(column_sums_stage_floats(hidden) * 4);
-    w.stp_off = o; o += align256(column_sums_stage_floats((int64_t)tile_rows((int)np) * K) * 4);
+    w.stp_off = o; o += align256(column_sums_stage_floats(prows * K) * 4);
     const size_t acc = w.wdt != x_dtype ? (size_t)batch * K * 4 : 0;
     w.xw_off = o; o += align256(acc);
     w.dxw_off = o; o += align256(acc);
@@ -1123,10 +1125,23 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
         }
         return hip_status(e);
     }
-    if (e == hipSuccess)
-        e = proj_bwd_all(w.wdt, xk, dp, dp_stride(np), stok, phi_pre, phi_post, phi_res, n, np, dxk, true, phip,
-                         rows_p, stp, grad_phi, batch, K, s, pscale, w.groups);
-    if (e == hipSuccess && w.wdt != x_dtype) e = launch_cast_bf16(dxw, batch * K, grad_x, s);
+    if (batch > 0 && w.wdt == kF32 && proj_bwd_tiles_path(np, batch)) {
+        // bf16 rows in place of their fp32 copies where both take 16-byte pieces
+        const bool direct = w.wdt == x_dtype || ((uintptr_t)x | (uintptr_t)grad_x) % 16 == 0;
+        if (e == hipSuccess)
+            e = launch_proj_bwd_tiles(direct ? x_dtype : w.wdt, direct ? x : xk, dp, dp_stride(np), stok, phi_pre,
+                                      phi_post, phi_res, n, np, (const float*)dxk, direct ? grad_x : dxk, phip, rows_p,
+                                      batch, K, s);
+        if (e == hipSuccess && !direct) e = launch_cast_bf16(dxw, batch * K, grad_x, s);
+        if (e == hipSuccess)
+            e = launch_column_finalize(0, kF32, phip, rows_p, (int64_t)np * K, stp, grad_phi, nullptr, 0, nullptr,
+                                       nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0.f, s);
+    } else {
+        if (e == hipSuccess)
+            e = proj_bwd_all(w.wdt, xk, dp, dp_stride(np), stok, phi_pre, phi_post, phi_res, n, np, dxk, true, phip,
+                             rows_p, stp, grad_phi, batch, K, s, pscale, w.groups);
+        if (e == hipSuccess && w.wdt != x_dtype) e = launch_cast_bf16(dxw, batch * K, grad_x, s);
+    }
     if (e == hipSuccess)
         e = launch_column_finalize(0, weight_dtype, dw_part, rows_w, hidden, stw, grad_weight, nullptr, 0, nullptr, nullptr,
                                   nullptr, nullptr, nullptr, nullptr, 0, 0.f, s);

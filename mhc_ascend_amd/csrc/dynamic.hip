@@ -1928,6 +1928,263 @@ __global__ __launch_bounds__(64 * kPbNW<TX>()) __attribute__((amdgpu_waves_per_e
 }
 
 // ---------------------------------------------------------------------------
+// The projection backward over OT = 2 or 3 output tiles at once (33..96 rows:
+// n = 5..8, past the tokens of the small-np kernels): proj_bwd_mfma_kernel's
+// stages with every tile's dP in LDS and its Phi^T fragments and dPhi sums in
+// registers, so x and the stream part are read once and dx is written once, in
+// x's type (TX; the stream part dx_in is fp32).  Bound by its bytes, 6 B read
+// and 2 B written per element of bf16 x.  n = 6, 2047 x 1040 bf16: 37 us where
+// two fp32 passes and the conversion back took 76 + 15; n = 8, 4096 x 2048 bf16:
+// 128 us for 443 + 131, 4096 x 1024 fp32: 98 us for 216.
+// ---------------------------------------------------------------------------
+template <typename TX, int OT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void proj_bwd_tiles_kernel(
+    const TX* __restrict__ x, const float* __restrict__ dP, int dp_stride, const float* __restrict__ s_tok,
+    const float* __restrict__ phi_pre, const float* __restrict__ phi_post, const float* __restrict__ phi_res,
+    int n_pre, int np, const float* dx_in, TX* dx, float* __restrict__ dphi_part, int64_t B, int64_t K, int64_t tile) {
+    constexpr int TB = 32;                 // tokens per stage
+    constexpr int CB = 128;                // columns per workgroup, 32 per wave
+    constexpr int EPV = 16 / sizeof(TX);   // elements per 16-byte piece of x / dx
+    constexpr int VPR = CB / EPV;
+    constexpr int RPP = 256 / VPR;
+    constexpr int PASSES = TB / RPP;
+    constexpr int DVPR = CB / 4;           // pieces per row of the stream part
+    constexpr int DRPP = 256 / DVPR;
+    constexpr int DPASSES = TB / DRPP;
+    constexpr int XPITCH = pb_pitch<TX, CB>();
+    constexpr int DPITCH = CB * 4 + 16;
+    __shared__ __align__(16) char x_lds[TB * XPITCH];
+    __shared__ __align__(16) char dx_lds[2][TB * DPITCH];
+    __shared__ __align__(16) bf16_t dps_lds[OT][4][32 * kDpPitch];  // hi_row, lo_row, hi_col, lo_col
+    __shared__ float s_lds[TB];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int lr = lane & 15;
+    const int lg = lane >> 4;
+    const int64_t kb0 = (int64_t)blockIdx.x * CB;
+    const int wc0 = wave * 32;
+    const bool wave_on = kb0 + wc0 < K;  // K % 32 == 0: whole waves are in or out
+    const int lrow = tid / VPR, lvec = tid % VPR;
+    const int64_t lcol = kb0 + (int64_t)lvec * EPV;
+    const int drow = tid / DVPR, dvec = tid % DVPR;
+    const int64_t dcol = kb0 + (int64_t)dvec * 4;
+    const int dtk = tid >> 3;       // dP loaders: token tid / 8,
+    const int dpo = (tid & 7) * 4;  // outputs 32 ot + 4 (tid % 8) .. + 3
+
+    // Phi^T: Phi[32 ot + 8 lg + e][column 16 ct + lr]
+    u32x4_t phh[OT][2], phl[OT][2];
+#pragma unroll
+    for (int ot = 0; ot < OT; ++ot) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+            const int64_t k = kb0 + wc0 + 16 * ct + lr;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int o = 32 * ot + 8 * lg + e;
+                v[e] = (wave_on && o < np) ? phi_row(phi_pre, phi_post, phi_res, n_pre, o, K)[k] : 0.f;
+            }
+            split_pack8(v, phh[ot][ct], phl[ot][ct]);
+        }
+    }
+    f32x4_t accP[2 * OT][2];
+#pragma unroll
+    for (int ot = 0; ot < 2 * OT; ++ot) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) accP[ot][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+
+    const int64_t t_begin = (int64_t)blockIdx.y * tile;
+    const int64_t t_end = (t_begin + tile < B) ? t_begin + tile : B;
+    const int64_t nrows = t_end > t_begin ? t_end - t_begin : 0;
+    const int64_t tb0 = nrows > 0 ? t_begin : 0;
+    // (buffer resources as in proj_bwd_mfma_kernel: no access behind a branch)
+    const uint32_t xrow = (uint32_t)(K * (int64_t)sizeof(TX));
+    const uint32_t drow_b = (uint32_t)(K * 4);
+    const buf_rsrc_t rs_x = make_buf_rsrc(x + tb0 * K, (uint32_t)(nrows * xrow));
+    const buf_rsrc_t rs_d = make_buf_rsrc(dx_in + tb0 * K, (uint32_t)(nrows * drow_b));
+    const buf_rsrc_t rs_o = make_buf_rsrc(dx + tb0 * K, (uint32_t)(nrows * xrow));
+    const buf_rsrc_t rs_p = make_buf_rsrc(dP + tb0 * dp_stride, (uint32_t)(nrows * dp_stride * 4));
+    const buf_rsrc_t rs_s = make_buf_rsrc(s_tok + tb0, (uint32_t)(nrows * 4));
+    const uint32_t xo = lcol < K ? (uint32_t)lrow * xrow + (uint32_t)(lcol * (int64_t)sizeof(TX)) : kBufOff;
+    const uint32_t dof = dcol < K ? (uint32_t)drow * drow_b + (uint32_t)(dcol * 4) : kBufOff;
+    const uint32_t po = (uint32_t)(dtk * dp_stride + dpo) * 4u;
+    const uint32_t so = tid < TB ? (uint32_t)tid * 4u : kBufOff;
+
+    struct Fetched {
+        uint4 x[PASSES], d[DPASSES];
+    };
+    struct Small {
+        uint4 dp[OT];
+        uint32_t s;
+    };
+    Fetched f0, f1;
+    Small sm;
+    auto fetch = [&](Fetched& f, uint32_t rel) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) f.x[p] = buf_ld16<true>(rs_x, xo + (rel + p * RPP) * xrow, 0u);
+#pragma unroll
+        for (int p = 0; p < DPASSES; ++p) f.d[p] = buf_ld16<true>(rs_d, dof + (rel + p * DRPP) * drow_b, 0u);
+    };
+    auto fetch_small = [&](uint32_t rel) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot)
+            sm.dp[ot] = buf_ld16<false>(rs_p, po + rel * (uint32_t)dp_stride * 4u + 128u * ot, 0u);
+        sm.s = buf_ld4(rs_s, so + rel * 4u, 0u);
+    };
+    auto commit = [&](const Fetched& f, int buf) __attribute__((always_inline)) {
+        // (an unconditional use of s: see proj_bwd_mfma_kernel)
+        asm volatile("" ::"v"(sm.s));
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) {
+            uint2* px = reinterpret_cast<uint2*>(&x_lds[(lrow + p * RPP) * XPITCH + lvec * 16]);
+            px[0] = make_uint2(f.x[p].x, f.x[p].y);
+            px[1] = make_uint2(f.x[p].z, f.x[p].w);
+        }
+#pragma unroll
+        for (int p = 0; p < DPASSES; ++p)
+            *reinterpret_cast<uint4*>(&dx_lds[buf][(drow + p * DRPP) * DPITCH + dvec * 16]) = f.d[p];
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot) {
+            const uint32_t w4[4] = {sm.dp[ot].x, sm.dp[ot].y, sm.dp[ot].z, sm.dp[ot].w};
+            float v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = 32 * ot + dpo + q < np ? __uint_as_float(w4[q]) : 0.f;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const uint32_t p0 = pack_bf16(v[0], v[1]), p1 = pack_bf16(v[2], v[3]);
+                *reinterpret_cast<uint2*>(&dps_lds[ot][k][dtk * kDpPitch + dpo]) = make_uint2(p0, p1);
+                bf16_t* col = dps_lds[ot][2 + k];
+                col[(dpo + 0) * kDpPitch + dtk] = (bf16_t)(p0 & 0xffffu);
+                col[(dpo + 1) * kDpPitch + dtk] = (bf16_t)(p0 >> 16);
+                col[(dpo + 2) * kDpPitch + dtk] = (bf16_t)(p1 & 0xffffu);
+                col[(dpo + 3) * kDpPitch + dtk] = (bf16_t)(p1 >> 16);
+                v[0] -= __uint_as_float(p0 << 16);
+                v[1] -= __uint_as_float(p0 & 0xffff0000u);
+                v[2] -= __uint_as_float(p1 << 16);
+                v[3] -= __uint_as_float(p1 & 0xffff0000u);
+            }
+        }
+        if (tid < TB) s_lds[tid] = __uint_as_float(sm.s);
+    };
+    auto read16 = [&](const bf16_t* p) __attribute__((always_inline)) -> u32x4_t {
+        const uint4 q = *reinterpret_cast<const uint4*>(p);
+        return u32x4_t{q.x, q.y, q.z, q.w};
+    };
+    auto compute = [&](int cur) __attribute__((always_inline)) {
+        if (!wave_on) return;
+        char* dt = dx_lds[cur];
+        // dPhi: A = dP^T (row 16 ot + lr, tokens 8 lg .. + 7), B = x (same tokens, column 16 ct + lr)
+        u32x4_t xh[2], xl[2];
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+            const int c = wc0 + 16 * ct + lr;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = VecIO<TX>::scalar(reinterpret_cast<const TX*>(x_lds + (8 * lg + e) * XPITCH) + c);
+            if constexpr (sizeof(TX) == 2) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xh[ct][e] = pack_bf16(v[2 * e], v[2 * e + 1]);  // exact
+            } else {
+                split_pack8(v, xh[ct], xl[ct]);
+            }
+        }
+#pragma unroll
+        for (int ot = 0; ot < 2 * OT; ++ot) {
+            const u32x4_t ah = read16(&dps_lds[ot / 2][2][(16 * (ot & 1) + lr) * kDpPitch + 8 * lg]);
+            const u32x4_t al = read16(&dps_lds[ot / 2][3][(16 * (ot & 1) + lr) * kDpPitch + 8 * lg]);
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct) {
+                accP[ot][ct] = mfma16x16x32(ah, xh[ct], accP[ot][ct]);
+                accP[ot][ct] = mfma16x16x32(al, xh[ct], accP[ot][ct]);
+                if constexpr (sizeof(TX) == 4) accP[ot][ct] = mfma16x16x32(ah, xl[ct], accP[ot][ct]);
+            }
+        }
+        // dx^T: D[column 16 ct + 4 lg + i][token 16 tt + lr]
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const int t = 16 * tt + lr;
+            f32x4_t d[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ot = 0; ot < OT; ++ot) {
+                const u32x4_t bh = read16(&dps_lds[ot][0][t * kDpPitch + 8 * lg]);
+                const u32x4_t bl = read16(&dps_lds[ot][1][t * kDpPitch + 8 * lg]);
+#pragma unroll
+                for (int ct = 0; ct < 2; ++ct) {
+                    d[ct] = mfma16x16x32(phh[ot][ct], bh, d[ct]);
+                    d[ct] = mfma16x16x32(phl[ot][ct], bh, d[ct]);
+                    d[ct] = mfma16x16x32(phh[ot][ct], bl, d[ct]);
+                }
+            }
+            const float st = s_lds[t];
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct) {
+                const int c0 = wc0 + 16 * ct + 4 * lg;
+                float xv[4];
+                lds_get4<TX>(x_lds + t * XPITCH + c0 * (int)sizeof(TX), xv);
+                float4* q = reinterpret_cast<float4*>(dt + t * DPITCH + c0 * 4);
+                const float4 a = *q;
+                *q = make_float4(fmaf(st, xv[0], d[ct][0] + a.x), fmaf(st, xv[1], d[ct][1] + a.y),
+                                 fmaf(st, xv[2], d[ct][2] + a.z), fmaf(st, xv[3], d[ct][3] + a.w));
+            }
+        }
+    };
+    auto store = [&](uint32_t rel, int cur) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) {
+            const char* q = &dx_lds[cur][(lrow + p * RPP) * DPITCH + lvec * EPV * 4];
+            uint4 o;
+            if constexpr (sizeof(TX) == 2) {
+                const float4 a = *reinterpret_cast<const float4*>(q), b = *reinterpret_cast<const float4*>(q + 16);
+                o = make_uint4(pack_bf16(a.x, a.y), pack_bf16(a.z, a.w), pack_bf16(b.x, b.y), pack_bf16(b.z, b.w));
+            } else {
+                o = *reinterpret_cast<const uint4*>(q);
+            }
+            buf_st16<true>(rs_o, xo + (rel + p * RPP) * xrow, 0u, o);
+        }
+    };
+    // whole pairs of stages, as proj_bwd_mfma_kernel
+    const uint32_t nr = (uint32_t)nrows;
+    fetch_small(0u);
+    fetch(f0, 0u);
+    commit(f0, 0);
+    fetch(f1, TB);
+    __syncthreads();
+    for (uint32_t r0 = 0; r0 < nr; r0 += 2 * TB) {
+        fetch_small(r0 + TB);
+        fetch(f0, r0 + 2 * TB);
+        compute(0);
+        __syncthreads();
+        store(r0, 0);
+        commit(f1, 1);
+        __syncthreads();
+        fetch_small(r0 + 2 * TB);
+        fetch(f1, r0 + 3 * TB);
+        compute(1);
+        __syncthreads();
+        store(r0 + TB, 1);
+        commit(f0, 0);
+        __syncthreads();
+    }
+    if (!wave_on) return;
+    float* out = dphi_part + (int64_t)blockIdx.y * np * K;
+#pragma unroll
+    for (int ot = 0; ot < 2 * OT; ++ot) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int o = 16 * ot + 4 * lg + i;
+                if (o < np) out[(int64_t)o * K + kb0 + wc0 + 16 * ct + lr] = accP[ot][ct][i];
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
 hipError_t launch_phi_split(const float* pre, const float* post, const float* res, int n, int np, int64_t K,
@@ -3113,6 +3370,40 @@ int proj_bwd_tiles(int x_dtype, int64_t B, int64_t K) {
     const int64_t mt = proj_bwd_max_tile(x_dtype, K) / 64 * 64;
     if (mt >= 64 && (B + tiles - 1) / tiles > mt) tiles = (B + mt - 1) / mt;
     return (int)tiles;
+}
+
+// n = 5..8, more tokens than the small-np kernels take
+bool proj_bwd_tiles_path(int np, int64_t B) {
+    return np > kProjTile && np <= 3 * kProjTile && B > kProjWideMaxB;
+}
+
+hipError_t launch_proj_bwd_tiles(int x_dtype, const void* x, const float* dP, int dp_stride, const float* s_tok,
+                                 const float* phi_pre, const float* phi_post, const float* phi_res, int n_pre, int np,
+                                 const float* dx_in, void* dx, float* dphi_part, int tiles, int64_t B, int64_t K,
+                                 hipStream_t s) {
+    if (!proj_bwd_tiles_path(np, B) || K % 32 != 0 || tiles < 1 || !s_tok) return hipErrorInvalidValue;
+    int64_t tile = (B + tiles - 1) / tiles;
+    tile = ((tile + 63) / 64) * 64;
+    if (tile > proj_bwd_max_tile(kF32, K)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((K + 127) / 128), (unsigned)tiles);
+    const int tok = timing_begin("proj_bwd", s);
+#define MHC_PBT(TX_, OT_)                                                                                            \
+    MHC_LAUNCH_GGL((proj_bwd_tiles_kernel<TX_, OT_>), grid, dim3(256), 0, s, (const TX_*)x, dP, dp_stride, s_tok,    \
+                   phi_pre, phi_post, phi_res, n_pre, np, dx_in, (TX_*)dx, dphi_part, B, K, tile)
+    if (x_dtype == kBF16) {
+        if (np <= 2 * kProjTile) {
+            MHC_PBT(bf16_t, 2);
+        } else {
+            MHC_PBT(bf16_t, 3);
+        }
+    } else if (np <= 2 * kProjTile) {
+        MHC_PBT(float, 2);
+    } else {
+        MHC_PBT(float, 3);
+    }
+#undef MHC_PBT
+    timing_end(tok, s);
+    return hipGetLastError();
 }
 
 hipError_t launch_proj_bwd(int x_dtype, const void* x, const float* dP, int dp_stride, const float* s_tok,
