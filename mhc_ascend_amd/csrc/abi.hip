@@ -1083,7 +1083,14 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
     float* dxw = (float*)(ws + w.dxw_off);
     int32_t* pscale = w.wdt == kBF16 ? (int32_t*)(ws + w.pscale_off) : nullptr;
     // the tensors the row and projection kernels work on
-    const void* xk = w.wdt != x_dtype ? (const void*)xw : x;
+    // (direct: the pass over all output tiles and the row kernel read bf16 x
+    // itself, where x and dx take 16-byte pieces and the rows fit registers:
+    // n = 8, 4096 x 2048 bf16 583 us of kernels with the fp32 copy of x, 497
+    // without)
+    const bool all_tiles = batch > 0 && w.wdt == kF32 && proj_bwd_tiles_path(2 * n + n * n, batch);
+    const bool direct = all_tiles && (w.wdt == x_dtype || (((uintptr_t)x | (uintptr_t)grad_x) % 16 == 0 &&
+                                                           layer_bwd_f32_dx_ok(n, hidden, aligned)));
+    const void* xk = w.wdt != x_dtype && !direct ? (const void*)xw : x;
     void* dxk = w.wdt != x_dtype ? (void*)dxw : grad_x;
     const DynSaved d = dyn_saved(batch, n, hidden);
     const int np = 2 * n + n * n;
@@ -1096,9 +1103,9 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
         e = launch_fill_zero(dw_part, hidden, s);
         if (e == hipSuccess) e = launch_fill_zero(cpart, np + 3, s);
     } else {
-        if (w.wdt != x_dtype) e = launch_weight_f32(x, x_dtype, batch * K, xw, s);
+        if (w.wdt != x_dtype && !direct) e = launch_weight_f32(x, x_dtype, batch * K, xw, s);
         if (e == hipSuccess)
-            e = launch_layer_bwd(w.wdt, n, 1, grad_out, xk, w32, saved + d.coef_off, np, dxk, dw_part, scal, w.grid,
+            e = launch_layer_bwd(direct ? x_dtype : w.wdt, n, direct && x_dtype == kBF16 ? 2 : 1, grad_out, xk, w32, saved + d.coef_off, np, dxk, dw_part, scal, w.grid,
                                  batch, hidden, rmsnorm_eps, (float*)(ws + w.rows_off), s, pscale, aligned);
         if (e == hipSuccess)
             e = launch_dyn_coef_bwd(n, scal, saved + d.coef_off, saved + d.p_off, saved + d.rh_off, batch, K,
@@ -1125,11 +1132,9 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
         }
         return hip_status(e);
     }
-    if (batch > 0 && w.wdt == kF32 && proj_bwd_tiles_path(np, batch)) {
-        // bf16 rows in place of their fp32 copies where both take 16-byte pieces
-        const bool direct = w.wdt == x_dtype || ((uintptr_t)x | (uintptr_t)grad_x) % 16 == 0;
+    if (all_tiles) {
         if (e == hipSuccess)
-            e = launch_proj_bwd_tiles(direct ? x_dtype : w.wdt, direct ? x : xk, dp, dp_stride(np), stok, phi_pre,
+            e = launch_proj_bwd_tiles(direct ? x_dtype : w.wdt, xk, dp, dp_stride(np), stok, phi_pre,
                                       phi_post, phi_res, n, np, (const float*)dxk, direct ? grad_x : dxk, phip, rows_p,
                                       batch, K, s);
         if (e == hipSuccess && !direct) e = launch_cast_bf16(dxw, batch * K, grad_x, s);

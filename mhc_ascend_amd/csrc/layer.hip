@@ -19,6 +19,8 @@
 // identity above avoids a second pass over gxa).  Workgroups are persistent
 // over tokens and keep dw and the scalar sums in registers; per-workgroup
 // partials are reduced deterministically afterwards.
+#include <type_traits>
+
 #include "mhc_device.h"
 #include "mhc_internal.h"
 #include "mhc_rows.h"
@@ -291,16 +293,20 @@ __global__ MHC_ROW_BOUNDS(false) void layer_static_fwd_kernel(const TX* __restri
 // MODE 1 (dynamic H) writes them per token to scal_out[b][n*n+2n+2]; its dx
 // holds the stream terms only (sum_i M_ij G_i + h_pre_j gxa), and a later
 // kernel adds the terms that need the per-token Sinkhorn backward first (the
-// projection and r_h terms).  dw accumulates in registers and goes to
-// dw_part[blockIdx.x][C].
+// projection and r_h terms).  MODE 2 is MODE 1 with an fp32 dx of bf16 x.  dw
+// accumulates in registers and goes to dw_part[blockIdx.x][C].
 // ---------------------------------------------------------------------------
+// dx of a mode: the storage type, or fp32 with MODE 2
+template <typename TX, int MODE>
+using BwdDx = std::conditional_t<MODE == 2, float, TX>;
+
 template <typename TX, int N, int VPT, int MODE>
 __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ coef, int64_t coef_stride,
                                           const float (&wv)[VPT][kLayerWC],
                                           const float (&xv)[N][VPT][kLayerWC],
                                           const float (&gv)[N][VPT][kLayerWC],
-                                          float (&dwacc)[VPT][kLayerWC], float& sacc, TX* __restrict__ dx,
-                                          float* __restrict__ scal_out, int32_t* __restrict__ dx_scale, int C,
+                                          float (&dwacc)[VPT][kLayerWC], float& sacc,
+                                          BwdDx<TX, MODE>* __restrict__ dx, float* __restrict__ scal_out, int32_t* __restrict__ dx_scale, int C,
                                           float eps, float* red) {
     constexpr int WC = kLayerWC;
     constexpr int NC = coef_size<N>();
@@ -440,7 +446,8 @@ __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ c
         const buf_rsrc_t qrs = make_buf_rsrc(dx_scale + b * ng, (uint32_t)(ng * 4));
         buf_st4(qrs, (threadIdx.x & 31) == 0 ? (uint32_t)(threadIdx.x / 32) * 4u : kBufOff, 0u, __int_as_float(ks));
     } else {
-        const buf_rsrc_t drs = make_buf_rsrc(dx + b * (int64_t)N * C, (uint32_t)((int64_t)N * C * (int64_t)sizeof(TX)));
+        using TD = BwdDx<TX, MODE>;
+        const buf_rsrc_t drs = make_buf_rsrc(dx + b * (int64_t)N * C, (uint32_t)((int64_t)N * C * (int64_t)sizeof(TD)));
 #pragma unroll
         for (int k = 0; k < VPT; ++k) {
             const int c0 = (k * blockDim.x + threadIdx.x) * WC;
@@ -456,7 +463,7 @@ __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ c
                 gxa[e] = wv[k][e] * gy * inv - xa * k2;
                 dwacc[k][e] += gy * xa * inv;
             }
-            const uint32_t o0 = c0 < C ? (uint32_t)c0 * (uint32_t)sizeof(TX) : kBufOff;
+            const uint32_t o0 = c0 < C ? (uint32_t)c0 * (uint32_t)sizeof(TD) : kBufOff;
 #pragma unroll
             for (int j = 0; j < N; ++j) {
                 float d[WC];
@@ -467,9 +474,9 @@ __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ c
                     for (int i = 0; i < N; ++i) s += cfv[2 * N + i * N + j] * gv[i][k][e];
                     d[e] = s;
                 }
-                const uint32_t o = o0 + (uint32_t)(j * C * (int)sizeof(TX));
+                const uint32_t o = o0 + (uint32_t)(j * C * (int)sizeof(TD));
                 static_assert(WC == 4, "4-channel chunks: one 16-byte (fp32) or 8-byte (bf16) store");
-                if constexpr (sizeof(TX) == 4) {
+                if constexpr (sizeof(TD) == 4) {
                     buf_st16<true>(drs, o, 0u, make_uint4(__float_as_uint(d[0]), __float_as_uint(d[1]),
                                                           __float_as_uint(d[2]), __float_as_uint(d[3])));
                 } else {
@@ -483,7 +490,7 @@ __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ c
 template <typename TX, int N, int VPT, int MODE, bool PF>
 __global__ MHC_ROW_BOUNDS(PF) void layer_bwd_kernel(const float* __restrict__ g, const TX* __restrict__ x,
                                                     const float* __restrict__ w, const float* __restrict__ coef,
-                                                    int64_t coef_stride, TX* __restrict__ dx,
+                                                    int64_t coef_stride, BwdDx<TX, MODE>* __restrict__ dx,
                                                     float* __restrict__ dw_part, float* __restrict__ scal_out,
                                                     int32_t* __restrict__ dx_scale, int64_t B, int C, float eps) {
     constexpr int WC = kLayerWC;
@@ -995,6 +1002,21 @@ static const void* pick_bwd(int x_dtype, int n, int vpt, int mode, bool pf) {
     return fn;
 }
 
+// mode 2: bf16 x, fp32 dx (n = 5..8, whose projection backward adds to it)
+static const void* pick_bwd_f32_dx(int n, int vpt, bool pf) {
+    const void* fn = nullptr;
+#define MHC_BWD_FN2(N_) MHC_PICK_VPT(vpt, fn = pf ? bwd_fn<bf16_t, N_, V_, 2, true>() : bwd_fn<bf16_t, N_, V_, 2, false>())
+    switch (n) {
+        case 5: { MHC_BWD_FN2(5); break; }
+        case 6: { MHC_BWD_FN2(6); break; }
+        case 7: { MHC_BWD_FN2(7); break; }
+        case 8: { MHC_BWD_FN2(8); break; }
+        default: break;
+    }
+#undef MHC_BWD_FN2
+    return fn;
+}
+
 static int persistent_grid(const void* fn, int threads, int64_t B) {
     const int per_cu = occupancy_per_cu(fn, threads, 0);
     int64_t g = (int64_t)device_cu_count() * per_cu;
@@ -1121,6 +1143,10 @@ static RowTiling bwd_tiling(int64_t C, int n, int x_dtype = kF32) {
 
 bool layer_bwd_is_wide(int n, int64_t C) { return bwd_tiling(C, n).vpt <= 0; }
 
+bool layer_bwd_f32_dx_ok(int n, int64_t C, bool aligned) {
+    return n >= 5 && n <= 8 && row_path(bwd_tiling(C, n), n, C, aligned) == RowPath::kRegs;
+}
+
 int layer_bwd_part_groups(int x_dtype, int n, int64_t C) {
     const RowTiling t = bwd_tiling(C, n, x_dtype);
     return t.vpt > 0 ? t.threads / 32 : 0;
@@ -1146,6 +1172,7 @@ hipError_t launch_layer_bwd(int x_dtype, int n, int mode, const float* g, const 
                             int32_t* dx_scale, bool aligned) {
     const RowTiling t = bwd_tiling(C, n, x_dtype);
     const RowPath path = row_path(t, n, C, aligned);
+    if (mode == 2 && path != RowPath::kRegs) return hipErrorInvalidValue;
     if (path == RowPath::kGen) {
         // the generic kernels write a full-precision stream part only for
         // fp32 x; the dynamic entries send bf16 x through fp32 accumulation
@@ -1161,7 +1188,8 @@ hipError_t launch_layer_bwd(int x_dtype, int n, int mode, const float* g, const 
                                scratch, s);
     }
     if (mode == 1 && x_dtype == kBF16 && (dx_scale == nullptr || C % kPartGroup != 0)) return hipErrorInvalidValue;
-    const void* fn = pick_bwd(x_dtype, n, t.vpt, mode, use_prefetch(t));
+    const void* fn = mode == 2 ? (x_dtype == kBF16 ? pick_bwd_f32_dx(n, t.vpt, use_prefetch(t)) : nullptr)
+                               : pick_bwd(x_dtype, n, t.vpt, mode, use_prefetch(t));
     if (!fn) return hipErrorInvalidValue;
     int Ci = (int)C;
     void* args[] = {(void*)&g, (void*)&x, (void*)&w, (void*)&coef, (void*)&coef_stride, (void*)&dx,

@@ -173,6 +173,8 @@ size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C, bool al
 // kernels of wide.hip rather than the register rows.
 bool layer_fwd_is_wide(int n, int64_t C);
 bool layer_bwd_is_wide(int n, int64_t C);
+// launch_layer_bwd takes mode 2: mode 1 with bf16 x and an fp32 dx
+bool layer_bwd_f32_dx_ok(int n, int64_t C, bool aligned);
 hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t s);
 // p0[0, n0) and p1[0, n1) = +0 while c[0] + .. + c[nc - 1] is finite, NaN
 // otherwise (fill_zero_carry_kernel)
