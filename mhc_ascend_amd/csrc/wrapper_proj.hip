@@ -9,8 +9,8 @@
 // dropped with it; 'zero' has no further streams.  With bf16 storage |d_j| <=
 // 2^-9 w_j |r|, so each residual stream takes one bf16 plane of Phi_j (error
 // 2^-18 w_j of the r term) where a stream of its own took three; past w_j =
-// 1e-5 (stream 6) it is below the r term's fp32 rounding (2^-24) and is
-// dropped.  n = 8: 11 plane products instead of 24 for each element of r, and
+// 1e-4 (stream 5) it is below the r term's fp32 rounding (2^-9 1e-5 against
+// 2^-24) and is dropped.  n = 8: 10 plane products instead of 24 for each element of r, and
 // two streams' worth of 'k' instead of eight at any n.
 //
 // The products run on bf16 MFMA 16x16x32, D[output][token]: A = Phi planes, B
@@ -18,7 +18,7 @@
 // fp32 rows are split hi / mid / lo in registers and their products keep the
 // six terms of 2^-16 and above.
 //
-// What bounds it: the matrix cores (n = 8, 65,536 tokens x 7168 bf16: 8.3e14
+// What bounds it: the matrix cores (n = 8, 65,536 tokens x 7168 bf16: 7.5e14
 // flops; the rows themselves are 1.9 GB), so the layout spares them
 // everything else.  A wave owns 16 TW tokens and all RT output tiles of its
 // row block: each Phi fragment (1 KB of LDS) feeds TW MFMAs, and a token's d_j
@@ -31,8 +31,8 @@
 // Measured (n = 8, 65,536 tokens x 7168 bf16): 3532 us for the eight rebuilt
 // streams through the layer's streaming projection, 1392 us folded with four
 // waves of unrolled planes (376 registers, one wave per SIMD: the residual
-// arithmetic and the MFMAs took turns), 931 us with eight waves (890 TFLOP/s of
-// plane products).  Errors against float64 over 10 draws at 8192 x 2048: db,
+// arithmetic and the MFMAs took turns), 931-975 us with eight waves, 865 without
+// stream 6's rounding.  Errors against float64 over 10 draws at 8192 x 2048: db,
 // dalpha 0.4-0.9 of the unfolded form's, all else equal.
 #include "mhc_device.h"
 #include "mhc_internal.h"
@@ -77,7 +77,7 @@ __device__ __forceinline__ float wp_mult(int j) {
 // Phi still crosses LDS once per 512 tokens; four otherwise (fp32 rows' split
 // operands need more than 256 registers).
 constexpr int wp_waves(int dt_size, int tw) { return dt_size == 2 && tw == 4 ? 8 : 4; }
-constexpr int kWpMaxRes = 5;  // residual streams 2 .. 6 (bf16 'decay')
+constexpr int kWpMaxRes = 4;  // residual streams 2 .. 5 (bf16 'decay')
 
 // Planes of Phi of a step: r and b hi / mid / lo, then -Phi_j of each residual
 // stream (the kernel forms w r - X).
@@ -547,13 +547,12 @@ hipError_t launch_wfold_proj(int dt, int n, bool decay, const void* res, const v
         MHC_WF(bf16_t, 2, 2);
     } else if (nres == 3) {  // n = 5: 35 rows
         MHC_WF(bf16_t, 3, 3);
-    } else if (nres == 4) {  // n = 6: 48 rows
-        MHC_WF(bf16_t, 3, 4);
-    } else {  // n >= 7: 63 rows and more
+    } else {  // n >= 6: 48 rows and more
         switch (rt) {
-            case 4: MHC_WF(bf16_t, 4, 5); break;
-            case 5: MHC_WF(bf16_t, 5, 5); break;
-            default: MHC_WF(bf16_t, 6, 5); break;
+            case 3: MHC_WF(bf16_t, 3, 4); break;
+            case 4: MHC_WF(bf16_t, 4, 4); break;
+            case 5: MHC_WF(bf16_t, 5, 4); break;
+            default: MHC_WF(bf16_t, 6, 4); break;
         }
     }
 #undef MHC_WF_RT
