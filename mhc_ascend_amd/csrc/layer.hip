@@ -1135,10 +1135,20 @@ hipError_t launch_layer_static_fwd(int x_dtype, int n, const void* x, const void
 // MODE 1: 213 -> 182 us against 512 lanes with one token in registers, once
 // the prefetch was unconditional; with the prefetch behind a branch the
 // 512-lane form had been the faster one).
-static RowTiling bwd_tiling(int64_t C, int n, int x_dtype = kF32) {
-    (void)x_dtype;
+// From n = 5 a row of one chunk per lane on more than 256 lanes takes over 128
+// registers: one workgroup a CU, one token at a time.  Two chunks on half the
+// lanes run the prefetch variant, the next token's rows in flight, which pays
+// once the CUs walk several tokens (B) and not before.  Backward row pass, dynamic n = 6, 2047 x 1040 bf16:
+// 43 us for 49; n = 5, 4096 x 1600 bf16: 72 for 85; n = 8, 4096 x 1280 fp32: 138
+// for 142; static n = 7, 4096 x 1184 fp32: 98 for 118.
+static RowTiling bwd_tiling(int64_t C, int n, int64_t B = 0) {
     if (n > 8 || (generic_layer_n(n) && !odd_row_n(n))) return RowTiling{0, 0};
-    return with_min_threads(choose_row_tiling(C, kLayerWC, 2 * n, 256), 2 + n * n + 3 * n);
+    RowTiling t = choose_row_tiling(C, kLayerWC, 2 * n, 256);
+    if (n >= 5 && t.vpt == 1 && t.threads > 256 && B >= 4 * (int64_t)device_cu_count() && layer_row_fits(2 * n, 2)) {
+        t.vpt = 2;
+        t.threads = (int)((C / kLayerWC + 127) / 128 * 64);
+    }
+    return with_min_threads(t, 2 + n * n + 3 * n);
 }
 
 bool layer_bwd_is_wide(int n, int64_t C) { return bwd_tiling(C, n).vpt <= 0; }
@@ -1148,12 +1158,13 @@ bool layer_bwd_f32_dx_ok(int n, int64_t C, bool aligned) {
 }
 
 int layer_bwd_part_groups(int x_dtype, int n, int64_t C) {
-    const RowTiling t = bwd_tiling(C, n, x_dtype);
+    (void)x_dtype;  // the fp16 stream part is that of bf16 x at n <= 4
+    const RowTiling t = bwd_tiling(C, n);
     return t.vpt > 0 ? t.threads / 32 : 0;
 }
 
 int layer_bwd_grid(int x_dtype, int n, int64_t B, int64_t C, bool aligned) {
-    const RowTiling t = bwd_tiling(C, n, x_dtype);
+    const RowTiling t = bwd_tiling(C, n, B);
     const RowPath path = row_path(t, n, C, aligned);
     if (path == RowPath::kGen) return gen_layer_bwd_grid(B);
     if (path == RowPath::kWide) return wide_bwd_grid(x_dtype, n, B, C);
@@ -1161,7 +1172,7 @@ int layer_bwd_grid(int x_dtype, int n, int64_t B, int64_t C, bool aligned) {
 }
 
 size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C, bool aligned) {
-    const RowPath path = row_path(bwd_tiling(C, n, x_dtype), n, C, aligned);
+    const RowPath path = row_path(bwd_tiling(C, n, B), n, C, aligned);
     if (path == RowPath::kGen) return gen_layer_bwd_scratch_bytes(B, C);
     return path == RowPath::kWide ? wide_bwd_scratch_bytes(n, B, C) : 0;
 }
@@ -1170,7 +1181,7 @@ hipError_t launch_layer_bwd(int x_dtype, int n, int mode, const float* g, const 
                             const float* coef, int64_t coef_stride, void* dx, float* dw_part, float* scal_out,
                             int grid, int64_t B, int64_t C, float eps, float* scratch, hipStream_t s,
                             int32_t* dx_scale, bool aligned) {
-    const RowTiling t = bwd_tiling(C, n, x_dtype);
+    const RowTiling t = bwd_tiling(C, n, B);
     const RowPath path = row_path(t, n, C, aligned);
     if (mode == 2 && path != RowPath::kRegs) return hipErrorInvalidValue;
     if (path == RowPath::kGen) {
