@@ -1525,16 +1525,21 @@ __global__ __launch_bounds__(256) void dyn_coef_w16_bwd_kernel(
 
 // out[c] = sum_r part[r][c] for a few columns (db, dalpha); one workgroup
 // per 32 columns, as 32 columns x 32 row phases, each phase summing every
-// 32nd row in order and the phases added in order (deterministic).
+// 32nd row in order and the phases added in order (deterministic).  Bound by
+// the latency of its loads, so the sums run in double at no cost and are
+// rounded once: a serial fp32 sum over the phases grew with the number of
+// partial rows (dynamic n = 8, 300 tokens, 75 rows against the 10 of 32-token
+// partials: db's error against float64 1.2 times as large, 0.9-1.04 so; n = 5,
+// 6 on 700-1500 tokens 0.76-0.95, 0.64-0.74 so).
 __global__ __launch_bounds__(1024) void small_column_sum_kernel(const float* __restrict__ part, int rows, int cols,
                                                                 float* __restrict__ out_db, float* __restrict__ out_da,
                                                                 int np) {
-    __shared__ float red[32][33];
+    __shared__ double red[32][33];
     const int cl = threadIdx.x & 31;
     const int ph = threadIdx.x >> 5;
     for (int c0 = blockIdx.x * 32; c0 < cols; c0 += gridDim.x * 32) {
         const int col = c0 + cl;
-        float s = 0.f;
+        double s = 0.0;
         if (col < cols) {
             // the phase's rows in order, 8 loads in flight
             int q = ph;
@@ -1550,8 +1555,9 @@ __global__ __launch_bounds__(1024) void small_column_sum_kernel(const float* __r
         red[ph][cl] = s;
         __syncthreads();
         if (ph == 0 && col < cols) {
-            float t = 0.f;
-            for (int k = 0; k < 32; ++k) t += red[k][cl];
+            double tot = 0.0;
+            for (int k = 0; k < 32; ++k) tot += red[k][cl];
+            const float t = (float)tot;
             if (col < np) out_db[col] = t;
             else out_da[col - np] = t;
         }
