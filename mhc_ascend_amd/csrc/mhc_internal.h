@@ -513,7 +513,7 @@ hipError_t launch_sinkhorn_bwd(int n, const float* grad_out, const float* inp, f
 
 // ---- wrapper_proj.hip --------------------------------------------------------
 // The wrapper's forward projection over r and b (hidden % 8 == 0, 16-byte
-// aligned rows): P and sum X^2 partials of wfold_ksplit splits in
+// aligned rows): P and sum X^2 partials of ks = wfold_ksplit splits in
 // launch_proj_mfma's layout, Phi packed into `pack` (wfold_pack_bytes, both
 // residual modes) and the RMSNorm weight's fp32 copy into w32 on the way.
 bool wfold_ok(int n, int64_t C);

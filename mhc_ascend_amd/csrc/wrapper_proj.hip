@@ -36,6 +36,7 @@
 // dalpha 0.4-0.9 of the unfolded form's, all else equal.
 #include "mhc_device.h"
 #include "mhc_internal.h"
+#include "wrapper_plan.h"
 
 namespace mhc {
 
@@ -72,11 +73,6 @@ __device__ __forceinline__ float wp_mult(int j) {
     return j == 6 ? kWpMult[6] : m;
 }
 
-// Waves per workgroup: eight at 64 tokens a wave of bf16 rows, so that two
-// waves of a SIMD overlap one's residual arithmetic with the other's MFMAs while
-// Phi still crosses LDS once per 512 tokens; four otherwise (fp32 rows' split
-// operands need more than 256 registers).
-constexpr int wp_waves(int dt_size, int tw) { return dt_size == 2 && tw == 4 ? 8 : 4; }
 constexpr int kWpMaxRes = 4;  // residual streams 2 .. 5 (bf16 'decay')
 
 // Planes of Phi of a step: r and b hi / mid / lo, then -Phi_j of each residual
@@ -235,7 +231,7 @@ __global__ __launch_bounds__(64 * wp_waves(sizeof(TX), TW)) void wfold_proj_kern
     };
     wu32x4_t st[CPW];
     auto fetch_phi = [&](int hs) __attribute__((always_inline)) {
-        const int h = hs < h1 ? hs : h0;  // past the last step: any step's planes
+        const int h = hs < h1 ? hs : h0;  // past the split's last step: any step's planes (h0 < steps)
 #pragma unroll
         for (int k = 0; k < CPW; ++k) {
             const int c = wave + kWpWaves * k;
@@ -403,43 +399,13 @@ static int wfold_nres(int dt, int n, bool decay) {
     return n - 2 < kWpMaxRes ? n - 2 : kWpMaxRes;
 }
 
-// 16-row tiles of a row block: all of them up to six, else the count that
-// pads least (the larger on ties: fewer passes over the rows).
-static int wfold_rt(int np) {
-    const int tiles = (np + 15) / 16;
-    if (tiles <= 6) return tiles;
-    int best = 6;
-    for (int rt = 5; rt >= 4; --rt) {
-        if ((tiles + rt - 1) / rt * rt * (rt + 1) * best < (tiles + best - 1) / best * best * (best + 1) * rt) best = rt;
-    }
-    return best;
-}
-
-// Token tiles per wave: four (512 tokens a workgroup) where that still leaves
-// enough workgroups, fewer for few tokens (a workgroup's rows past the batch
-// are wasted, and every workgroup reads all of its Phi steps).
-static int wfold_tw(int64_t B) { return B >= 2048 ? 4 : (B >= 512 ? 2 : 1); }
-static int64_t wfold_tokens(int dt, int64_t B) {
-    const int tw = wfold_tw(B);
-    return (int64_t)16 * tw * wp_waves(dtype_size(dt), tw);
-}
-
-static int wfold_steps(int dt, int64_t C) { return dt == kBF16 ? 2 * (int)((C + 63) / 64) : (int)((C + 31) / 32); }
-
 int wfold_ksplit(int dt, int64_t B, int64_t C, int np) {
-    const int rt = wfold_rt(np);
-    const int64_t per = wfold_tokens(dt, B);
-    const int64_t blocks = ((B + per - 1) / per) * (((np + 15) / 16 + rt - 1) / rt);
-    int64_t ks = device_cu_count() / (blocks < 1 ? 1 : blocks);
-    const int64_t kmax = wfold_steps(dt, C) / 4;  // at least four steps a split
-    if (ks > kmax) ks = kmax;
-    return (int)(ks < 1 ? 1 : ks);
+    return wfold_split(dt == kBF16, B, C, np, device_cu_count()).ks;
 }
 
 size_t wfold_pack_bytes(int dt, int n, int64_t C, int np) {
-    const int rt = wfold_rt(np);
-    const int64_t rbs = ((np + 15) / 16 + rt - 1) / rt;
-    return (size_t)rbs * wfold_steps(dt, C) * wp_planes(wfold_nres(dt, n, true)) * rt * 1024;
+    return (size_t)wfold_row_blocks(np) * wfold_steps(dt == kBF16, C) * wp_planes(wfold_nres(dt, n, true)) *
+           wfold_rt(np) * 1024;
 }
 
 bool wfold_ok(int n, int64_t C) { return n >= 2 && n <= kWgMaxN && C >= 8 && C % 8 == 0 && C <= (int64_t(1) << 21); }
@@ -495,8 +461,11 @@ hipError_t launch_wfold_proj(int dt, int n, bool decay, const void* res, const v
         reinterpret_cast<uintptr_t>(br) % 16 != 0)
         return hipErrorInvalidValue;
     const int nres = wfold_nres(dt, n, decay), rt = wfold_rt(np);
-    const int rbs = ((np + 15) / 16 + rt - 1) / rt;
-    const int steps = wfold_steps(dt, C);
+    const int rbs = wfold_row_blocks(np);
+    const WfoldSplit sp = wfold_split(dt == kBF16, B, C, np, device_cu_count());
+    // (the kernel's prologue reads the first step of its split)
+    if (ks != sp.ks || (int64_t)(sp.ks - 1) * sp.chunk >= sp.steps) return hipErrorInvalidValue;
+    const int steps = sp.steps, schunk = sp.chunk;
     const int Ci = (int)C;
     const int64_t frags = (int64_t)rbs * steps * rt * 64;
     int64_t pblocks = (frags + 255) / 256;
@@ -509,9 +478,7 @@ hipError_t launch_wfold_proj(int dt, int n, bool decay, const void* res, const v
                        n, np, Ci, decay ? 1 : 0, nres, rt, rbs, steps, (uint4*)pack, weight, w_dtype, w32);
     }
     const int tw = wfold_tw(B);
-    int schunk = (steps + ks - 1) / ks;
-    if (dt == kBF16) schunk = (schunk + 1) / 2 * 2;
-    const int64_t per = wfold_tokens(dt, B);
+    const int64_t per = wfold_tokens(dt == kBF16, B);
     const int64_t gx = (B + per - 1) / per * rbs;
     if (gx > 0x7fffffff || ks > 65535) return hipErrorInvalidValue;
     const dim3 grid((unsigned)gx, (unsigned)ks);
