@@ -7,33 +7,38 @@
 //   Phi_r = Phi_0 + sum_{j >= 2} w_j Phi_j (fp32),   d_j = X_j - w_j r.
 // With fp32 storage d_j is below the fp32 rounding of the r term and is
 // dropped with it; 'zero' has no further streams.  With bf16 storage |d_j| <=
-// 2^-9 w_j |r|, so each residual stream takes one bf16 plane of Phi_j (error
-// 2^-18 w_j of the r term) where a stream of its own took three; past w_j =
-// 1e-4 (stream 5) it is below the r term's fp32 rounding (2^-9 1e-5 against
-// 2^-24) and is dropped.  n = 8: 10 plane products instead of 24 for each element of r, and
-// two streams' worth of 'k' instead of eight at any n.
+// 2^-9 w_j |r|, so a product of the bf16 parts of d_j and Phi_j, off by 2^-9 of
+// it, is below the r term's fp32 rounding (2^-24) from stream 3 on (2^-18 w_j,
+// w_3 = 0.01); stream 2 takes d_h Phi_h + d_h Phi_m + d_m Phi_h (2^-17 of it).
+// Past w_j = 1e-4 (stream 5) d_j itself is below (2^-9 1e-5) and is dropped.
+// n = 8: 12 plane products instead of 24 for each element of r, and two streams'
+// worth of 'k' instead of eight at any n.
 //
 // The products run on bf16 MFMA 16x16x32, D[output][token]: A = Phi planes, B
 // = the token rows.  Phi_r and Phi_1 are split hi / mid / lo (exact to fp32);
 // fp32 rows are split hi / mid / lo in registers and their products keep the
-// six terms of 2^-16 and above.
+// six terms of 2^-16 and above.  The products below hi . hi have an accumulator
+// of their own where the registers allow it (wp_two_acc).
 //
-// What bounds it: the matrix cores (n = 8, 65,536 tokens x 7168 bf16: 7.5e14
-// flops; the rows themselves are 1.9 GB), so the layout spares them
-// everything else.  A wave owns 16 TW tokens and all RT output tiles of its
-// row block: each Phi fragment (1 KB of LDS) feeds TW MFMAs, and a token's d_j
-// fragments are built once.  The rows go from memory straight to the fragment
-// registers: with bf16 a lane's k order is free as long as Phi is packed
-// alike, so lane group g of a 64-channel stage takes channels 16 g .. 16 g +
-// 15 of its token (two 16-byte loads, four groups a whole 128-byte line).
-// Phi planes go through LDS, one 32-channel step ahead of the MFMAs, packed so
-// that a step of a row block is one contiguous run.
-// Measured (n = 8, 65,536 tokens x 7168 bf16): 3532 us for the eight rebuilt
-// streams through the layer's streaming projection, 1392 us folded with four
-// waves of unrolled planes (376 registers, one wave per SIMD: the residual
-// arithmetic and the MFMAs took turns), 931-975 us with eight waves, 865 without
-// stream 6's rounding.  Errors against float64 over 10 draws at 8192 x 2048: db,
-// dalpha 0.4-0.9 of the unfolded form's, all else equal.
+// A wave owns 16 TW tokens and all RT output tiles of its row block: each Phi
+// fragment (1 KB of LDS) feeds TW MFMAs, and a token's d_j fragments are built
+// once.  The rows go from memory straight to the fragment registers: with bf16 a
+// lane's k order is free as long as Phi is packed alike, so lane group g of a
+// 64-channel stage takes channels 16 g .. 16 g + 15 of its token (two 16-byte
+// loads, four groups a whole 128-byte line).  Phi planes go through LDS, one
+// 32-channel step ahead of the MFMAs, packed so that a step of a row block is one
+// contiguous run.
+// Measured (n = 8, 65,536 tokens x 7168 bf16; the rows are 1.9 GB): 3532 us for
+// the eight rebuilt streams through the layer's streaming projection, 1392 us
+// folded with four waves of unrolled planes (376 registers, one wave per SIMD:
+// the residual arithmetic and the MFMAs took turns), 980 us with eight waves; with
+// the residual streams formed in each product of stream 2 1260.  It follows the vector
+// work of the residual streams as well as the MFMAs.
+// Error of P against float64 (rms, relative; 3 draws each): n = 3..32, 32 to
+// 2100 tokens, 64 to 7168 channels 0.65e-7 to 3.4e-7, 0.25 to 0.98 of that of the
+// unfolded form on the same inputs; with one accumulator and one plane for stream
+// 2, 865 us here, it was up to 2.5 times the unfolded form's (n = 3, 700 x 512:
+// 2.9e-7 for 1.2e-7, 1.0e-7 now).
 #include "mhc_device.h"
 #include "mhc_internal.h"
 #include "wrapper_plan.h"
@@ -76,8 +81,15 @@ __device__ __forceinline__ float wp_mult(int j) {
 constexpr int kWpMaxRes = 4;  // residual streams 2 .. 5 (bf16 'decay')
 
 // Planes of Phi of a step: r and b hi / mid / lo, then -Phi_j of each residual
-// stream (the kernel forms w r - X).
-constexpr int wp_planes(int nres) { return 6 + nres; }
+// stream (the kernel forms w r - X), the first of them hi / mid.
+constexpr int wp_planes(int nres) { return 6 + nres + (nres > 0 ? 1 : 0); }
+
+// Products of two hi parts and the smaller ones in accumulators of their own:
+// then a step rounds the large sum twice and not 6 to 13 times.  Where the
+// registers allow it (bf16 rows at 64 tokens a wave: 256 of them, up to three
+// row tiles; past that the long chains of the same tokens are no shorter in any
+// other form).
+constexpr bool wp_two_acc(bool bf16, int rt, int tw) { return !bf16 || rt * tw <= 12; }
 
 }  // namespace
 
@@ -148,7 +160,12 @@ __global__ __launch_bounds__(256) void wfold_pack_kernel(const float* __restrict
                 if (j - 2 < nres) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[e] = -v[e];
-                    put(6 + j - 2, v);
+                    put(j == 2 ? 6 : 5 + j, v);
+                    if (j == 2) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) v[e] -= bf16_to_f32(f32_to_bf16(v[e]));
+                        put(7, v);
+                    }
                 }
             }
         }
@@ -194,12 +211,24 @@ __global__ __launch_bounds__(64 * wp_waves(sizeof(TX), TW)) void wfold_proj_kern
     const buf_rsrc_t rs_b = make_buf_rsrc(br + tb * C, (uint32_t)nrows * rowb);
     const wu32x4_t* pw = reinterpret_cast<const wu32x4_t*>(phi) + ((int64_t)rb * steps) * CH * 64 + lane;
 
-    wf32x4_t acc[RT][TW];
+    constexpr bool TWO = wp_two_acc(BF, RT, TW);
+    wf32x4_t acc[RT][TW], accs[TWO ? RT : 1][TWO ? TW : 1];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-        for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wf32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int tt = 0; tt < TW; ++tt) {
+            acc[rt][tt] = wf32x4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (TWO) accs[rt][tt] = acc[rt][tt];
+        }
     }
+    // the accumulator of the products below hi . hi
+    auto small = [&](int rt, int tt) __attribute__((always_inline)) -> wf32x4_t& {
+        if constexpr (TWO) {
+            return accs[rt][tt];
+        } else {
+            return acc[rt][tt];
+        }
+    };
     // (-1, 0) and (0, -1), held in registers: as a literal operand of the dot
     // product the first becomes the inline constant -1.0, which the hardware
     // reads as its fp32 bits, (0, -1)
@@ -259,22 +288,34 @@ __global__ __launch_bounds__(64 * wp_waves(sizeof(TX), TW)) void wfold_proj_kern
             }
             // rolled loops: one plane's products at a time keep the wave within
             // 256 registers (two waves per SIMD)
-#pragma unroll 1
-            for (int p = 0; p < 3; ++p) {
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) {
-                    const wu32x4_t a = frag(buf, p, rt);
+            for (int rt = 0; rt < RT; ++rt) {
+                const wu32x4_t a = frag(buf, 0, rt);
 #pragma unroll
-                    for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wmfma(a, xr[tt], acc[rt][tt]);
-                }
+                for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wmfma(a, xr[tt], acc[rt][tt]);
             }
 #pragma unroll 1
-            for (int p = 3; p < 6; ++p) {
+            for (int p = 1; p < 3; ++p) {
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
                     const wu32x4_t a = frag(buf, p, rt);
 #pragma unroll
-                    for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wmfma(a, xb[tt], acc[rt][tt]);
+                    for (int tt = 0; tt < TW; ++tt) small(rt, tt) = wmfma(a, xr[tt], small(rt, tt));
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const wu32x4_t a = frag(buf, 3, rt);
+#pragma unroll
+                for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wmfma(a, xb[tt], acc[rt][tt]);
+            }
+#pragma unroll 1
+            for (int p = 4; p < 6; ++p) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const wu32x4_t a = frag(buf, p, rt);
+#pragma unroll
+                    for (int tt = 0; tt < TW; ++tt) small(rt, tt) = wmfma(a, xb[tt], small(rt, tt));
                 }
             }
 #pragma unroll
@@ -285,26 +326,70 @@ __global__ __launch_bounds__(64 * wp_waves(sizeof(TX), TW)) void wfold_proj_kern
                     ss[tt] = wdot2(xb[tt][e], xb[tt][e], ss[tt]);
                 }
             }
+            // w r - X of a stream, exact: -d_j (the packed planes are -Phi_j), and
+            // its bf16 part; X^2 into sq
+            auto resid = [&](uint32_t xw, float m, bool add, float& sq, float& d0, float& d1)
+                __attribute__((always_inline)) {
+                const float p0 = wlo(xw) * m, p1 = whi(xw) * m;
+                const uint32_t x = pack_bf16x2(p0, p1);  // the stored stream
+                const uint32_t xs = add ? x : 0u;
+                sq = wdot2(xs, xs, sq);
+                d0 = wdot2(x, neg_lo, p0);
+                d1 = wdot2(x, neg_hi, p1);
+                return pack_bf16x2(d0, d1);
+            };
+            // stream 2, whose rounding is the largest: -d_2 and Phi_2 hi + mid
+            constexpr bool ONE = NRES > 0 && RT * TW >= 24;
+            if constexpr (NRES > 0 && !ONE) {
+                wu32x4_t dh[TW], dm[TW];
+#pragma unroll
+                for (int tt = 0; tt < TW; ++tt) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float d0, d1;
+                        dh[tt][e] = resid(xr[tt][e], kWpMult[2], true, ss[tt], d0, d1);
+                        dm[tt][e] = pack_bf16x2(wdot2(dh[tt][e], neg_lo, d0), wdot2(dh[tt][e], neg_hi, d1));
+                    }
+                }
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const wu32x4_t a = frag(buf, 6, rt), am = frag(buf, 7, rt);
+#pragma unroll
+                    for (int tt = 0; tt < TW; ++tt) small(rt, tt) = wmfma(a, dh[tt], small(rt, tt));
+#pragma unroll
+                    for (int tt = 0; tt < TW; ++tt) small(rt, tt) = wmfma(am, dh[tt], small(rt, tt));
+#pragma unroll
+                    for (int tt = 0; tt < TW; ++tt) small(rt, tt) = wmfma(a, dm[tt], small(rt, tt));
+                }
+            }
+            // the others, one plane each; with six row tiles, where both parts of
+            // d_2 do not fit, its three products first (t = 0, 1, 2)
 #pragma unroll 1
-            for (int j = 0; j < NRES; ++j) {
-                const float m = wp_mult(j + 2);
+            for (int t = ONE ? 0 : 3; t < NRES + 2; ++t) {
+                const float m = t < 3 ? kWpMult[2] : wp_mult(t);
+                const bool low = ONE && t == 2, again = ONE && (t == 1 || t == 2);
                 wu32x4_t d[TW];
 #pragma unroll
                 for (int tt = 0; tt < TW; ++tt) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float p0 = wlo(xr[tt][e]) * m, p1 = whi(xr[tt][e]) * m;
-                        const uint32_t x = pack_bf16x2(p0, p1);  // the stored stream
-                        ss[tt] = wdot2(x, x, ss[tt]);
-                        // w r - X, exact: -d_j (the packed plane is -Phi_j)
-                        d[tt][e] = pack_bf16x2(wdot2(x, neg_lo, p0), wdot2(x, neg_hi, p1));
+                        float d0, d1;
+                        const uint32_t h = resid(xr[tt][e], m, !again, ss[tt], d0, d1);
+                        if constexpr (ONE) {
+                            d0 -= low ? wlo(h) : 0.f;
+                            d1 -= low ? whi(h) : 0.f;
+                            d[tt][e] = pack_bf16x2(d0, d1);
+                        } else {
+                            d[tt][e] = h;
+                        }
                     }
                 }
+                const int p = low ? 6 : (t < 3 ? 6 + t : 5 + t);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
-                    const wu32x4_t a = frag(buf, 6 + j, rt);
+                    const wu32x4_t a = frag(buf, p, rt);
 #pragma unroll
-                    for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wmfma(a, d[tt], acc[rt][tt]);
+                    for (int tt = 0; tt < TW; ++tt) small(rt, tt) = wmfma(a, d[tt], small(rt, tt));
                 }
             }
         } else {
@@ -340,7 +425,10 @@ __global__ __launch_bounds__(64 * wp_waves(sizeof(TX), TW)) void wfold_proj_kern
 #pragma unroll
                         for (int k = 0; k < 3 - p; ++k) {
 #pragma unroll
-                            for (int tt = 0; tt < TW; ++tt) acc[rt][tt] = wmfma(a, x3[k][tt], acc[rt][tt]);
+                            for (int tt = 0; tt < TW; ++tt) {
+                                wf32x4_t& c = p + k == 0 ? acc[rt][tt] : small(rt, tt);
+                                c = wmfma(a, x3[k][tt], c);
+                            }
                         }
                     }
                 }
@@ -371,6 +459,13 @@ __global__ __launch_bounds__(64 * wp_waves(sizeof(TX), TW)) void wfold_proj_kern
         __syncthreads();
     }
 
+    if constexpr (TWO) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int tt = 0; tt < TW; ++tt) acc[rt][tt] += accs[rt][tt];
+        }
+    }
     // lane: token lr of tile tt, outputs 4 g .. 4 g + 3 of row tile rt
     const int tiles = (np + kProjTile - 1) / kProjTile;
 #pragma unroll

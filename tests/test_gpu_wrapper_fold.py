@@ -93,12 +93,8 @@ def test_unaligned_rows(device, n, dtype):
     _run(device, n, 70, 64, dtype, "decay", seed=n, shift=1)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_projection_error(device, dtype):
-    """The folded P against float64, relative to its norm: 1e-6 (hi / mid / lo
-    planes of Phi, residual streams to 2^-18 of a tenth), at n = 8 over a long
-    row, from the forward's saved state."""
-    n, T, C = 8, 96, 4096
+def _projection_error(device, n, T, C, dtype, mode):
+    """|P - float64| / |float64| of the folded P, from the forward's saved state."""
     g = torch.Generator().manual_seed(5)
     r, b = torch.randn(T, C, generator=g).to(dtype), torch.randn(T, C, generator=g).to(dtype)
     layer = mhc.MHCLayer(C, n).to(device)
@@ -107,11 +103,28 @@ def test_projection_error(device, dtype):
             getattr(layer, nm).fill_(1.0)
     from mhc_ascend_amd import native
     ps = [getattr(layer, nm).detach() for nm in NAMES]
-    _, saved = native.wrapper_dynamic_fwd(r.to(device), b.to(device), "decay", n, *ps)
+    _, saved = native.wrapper_dynamic_fwd(r.to(device), b.to(device), mode, n, *ps)
     np_ = 2 * n + n * n
     off = (C + 63) // 64 * 64 + (T * np_ + 63) // 64 * 64
     P = saved.view(-1)[off:off + T * np_].view(T, np_).double().cpu()
-    X = R.build_wrapper_streams(r, b, n, "decay").double().reshape(T, -1)
+    X = R.build_wrapper_streams(r, b, n, mode).double().reshape(T, -1)
     phi = torch.cat([layer.phi_pre, layer.phi_post, layer.phi_res]).detach().double().cpu()
     ref = X @ phi.t()
-    assert float((P - ref).norm() / ref.norm()) < 1e-6
+    return float((P - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_projection_error(device, dtype):
+    """The folded P against float64, relative to its norm: 1e-6 (hi / mid / lo
+    planes of Phi, residual streams below 2^-24), at n = 8 over a long row."""
+    assert _projection_error(device, 8, 96, 4096, dtype, "decay") < 1e-6
+
+
+@pytest.mark.parametrize("mode", ["decay", "zero"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,T,C", [(3, 700, 512), (5, 700, 512), (8, 300, 64), (12, 300, 64)])
+def test_projection_error_of_short_rows(device, n, T, C, dtype, mode):
+    """Rows of few steps: three half-ulps of fp32 (3 x 2^-24), which a step's
+    products below hi . hi in the large sum's accumulator, or stream 2 of bf16
+    'decay' from single bf16 parts, exceed."""
+    assert _projection_error(device, n, T, C, dtype, mode) < 3 * 2.0 ** -24
