@@ -174,10 +174,10 @@ __device__ __forceinline__ void fwd_token(int64_t b, const float* __restrict__ c
             float o[WC];
 #pragma unroll
             for (int e = 0; e < WC; ++e) {
-                float s = cfv[N + i] * y[e];
+                float s = kTermLast<N> ? 0.f : cfv[N + i] * y[e];
 #pragma unroll
                 for (int j = 0; j < N; ++j) s += cfv[2 * N + i * N + j] * xv[j][k][e];
-                o[e] = s;
+                o[e] = kTermLast<N> ? s + cfv[N + i] * y[e] : s;
             }
             const uint32_t off = o0 + (uint32_t)(i * C * (int)sizeof(TO));
             if constexpr (sizeof(TO) == 4) {
@@ -409,9 +409,10 @@ __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ c
                 dwacc[k][e] += gy * xa * inv;
 #pragma unroll
                 for (int j = 0; j < N; ++j) {
-                    float s = cfv[j] * gxa;
+                    float s = kTermLast<N> ? 0.f : cfv[j] * gxa;
 #pragma unroll
                     for (int i = 0; i < N; ++i) s += cfv[2 * N + i * N + j] * gv[i][k][e];
+                    if (kTermLast<N>) s += cfv[j] * gxa;
                     a[j][k][e] = s;
                     m = fmaxf(m, fabsf(s));
                 }
@@ -469,10 +470,10 @@ __device__ __forceinline__ void bwd_token(int64_t b, const float* __restrict__ c
                 float d[WC];
 #pragma unroll
                 for (int e = 0; e < WC; ++e) {
-                    float s = cfv[j] * gxa[e];
+                    float s = kTermLast<N> ? 0.f : cfv[j] * gxa[e];
 #pragma unroll
                     for (int i = 0; i < N; ++i) s += cfv[2 * N + i * N + j] * gv[i][k][e];
-                    d[e] = s;
+                    d[e] = kTermLast<N> ? s + cfv[j] * gxa[e] : s;
                 }
                 const uint32_t o = o0 + (uint32_t)(j * C * (int)sizeof(TD));
                 static_assert(WC == 4, "4-channel chunks: one 16-byte (fp32) or 8-byte (bf16) store");

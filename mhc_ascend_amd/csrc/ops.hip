@@ -260,10 +260,10 @@ __global__ MHC_ROW_BOUNDS(false) void distribute_fwd_kernel(const T* __restrict_
         for (int k = 0; k < VPT; ++k) {
 #pragma unroll
             for (int e = 0; e < WC; ++e) {
-                float s = h[i] * yv[0][k][e];
+                float s = kTermLast<N> ? 0.f : h[i] * yv[0][k][e];
 #pragma unroll
                 for (int j = 0; j < N; ++j) s += m[i * N + j] * xv[j][k][e];
-                o[k][e] = s;
+                o[k][e] = kTermLast<N> ? s + h[i] * yv[0][k][e] : s;
             }
         }
         store_row1<float, VPT, WC, true>(ob + (int64_t)i * C, C, o);

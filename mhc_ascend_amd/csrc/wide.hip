@@ -120,9 +120,10 @@ __device__ __forceinline__ void wide_fwd_channel(const TX* __restrict__ xb, cons
     const float y = xa * inv * w[c];
 #pragma unroll 4
     for (int i = 0; i < N; ++i) {
-        float s = cfs[N + i] * y;
+        float s = kTermLast<N> ? 0.f : cfs[N + i] * y;
 #pragma unroll
         for (int j = 0; j < N; ++j) s += cfs[2 * N + i * N + j] * xv[j];
+        if (kTermLast<N>) s += cfs[N + i] * y;
         st_elem_nt(ob + (int64_t)i * C + c, s);
     }
 }
@@ -310,9 +311,10 @@ __device__ __forceinline__ float wide_bwd_dx(const float* __restrict__ cf, const
     const float gxa = w[c] * gy * inv - xa * k2;
 #pragma unroll 4
     for (int j = 0; j < N; ++j) {
-        float s = cf[j] * gxa;
+        float s = kTermLast<N> ? 0.f : cf[j] * gxa;
 #pragma unroll
         for (int i = 0; i < N; ++i) s += cf[2 * N + i * N + j] * gv[i];
+        if (kTermLast<N>) s += cf[j] * gxa;
         st_elem_nt(db + (int64_t)j * C + c, s);
     }
     return gy * xa * inv;
@@ -874,9 +876,10 @@ __global__ __launch_bounds__(kWideThreads) void wide_distribute_fwd_kernel(
         for (int j = 0; j < N; ++j) xv[j] = ld_elem_nt(xb + (int64_t)j * C + c);
         const float yv = ld_elem_nt(y + b * C + c);
         for (int i = 0; i < N; ++i) {
-            float s = h[i] * yv;
+            float s = kTermLast<N> ? 0.f : h[i] * yv;
 #pragma unroll
             for (int j = 0; j < N; ++j) s += mb[i * N + j] * xv[j];
+            if (kTermLast<N>) s += h[i] * yv;
             st_elem_nt(ob + (int64_t)i * C + c, s);
         }
     }

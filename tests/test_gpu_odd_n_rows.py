@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import mhc_ascend_amd as mhc
+from mhc_ascend_amd import native
 from oracle import reference as R
 from tests.conftest import assert_close, grad_atol
 from tests.test_gpu_dynamic import _check_dyn, _oracle_dyn
@@ -89,3 +90,47 @@ def test_operator_rows(device, n, B, C, shift, dtype):
     for nm, a, e in zip(("dy", "dh", "dM", "dx"), got, want):
         stored = nm in ("dy", "dx")
         assert_close(a, e, rtol if stored else 1e-3, grad_atol(e, frac if stored else 1e-4), f"distribute {nm}")
+
+
+def _f32(t):
+    return t.float().double()
+
+
+def _mix32(h, y, m, x, last):
+    """out_i = h_i y + sum_j m_ij x_j as fp32 fused products (exact in float64,
+    rounded to fp32 each), the y term after the others or before them."""
+    f = _f32
+    n = x.shape[1]
+    rows = []
+    for i in range(n):
+        s = torch.zeros_like(y) if last else f(h[i] * y)
+        for j in range(n):
+            s = f(s + m[i, j] * x[:, j])
+        rows.append(f(s + h[i] * y) if last else s)
+    return torch.stack(rows, 1)
+
+
+@pytest.mark.parametrize("C", [512, 509])
+@pytest.mark.parametrize("n", [3, 5, 6, 7])
+def test_error_of_the_mix(device, n, C):
+    """out of fp32 rows (register and channel-loop rows), from the coefficients that
+    the library formed: the rms error against float64 is that of fp32 products with
+    the term that is no stream's added after the mix, and not that with it rounded
+    along with every product: the line lies between the two, formed on the same data,
+    nearer to the second (r_h has its own rounding) (0.93 and 1.1 times 2^-24 at n = 3, 1.2 and 1.5 at n = 7)."""
+    d = R.static_layer_inputs(300, n, C, seed=n)
+    ps = [d[k].to(device) for k in ("weight", "H_pre", "H_post", "H_res")]
+    out, _, saved = native.mhc_layer_static_fwd(d["x"].to(device), *ps)
+    out, coef, x, w = out.cpu().double(), saved[:2 * n + n * n].cpu().double(), d["x"].double(), d["weight"].double()
+    hp, h, m = coef[:n], coef[n:2 * n], coef[2 * n:].view(n, n)
+    xa = (hp[:, None] * x).sum(1)
+    y = xa / torch.sqrt((xa * xa).mean(-1, keepdim=True) + 1e-5) * w
+    ref = torch.matmul(m, x) + h[:, None] * y[:, None]
+    xa = torch.zeros_like(xa)
+    for j in range(n):
+        xa = _f32(xa + hp[j] * x[:, j])
+    inv = _f32(1 / _f32(torch.sqrt((xa * xa).mean(-1, keepdim=True) + 1e-5)))
+    y = _f32(_f32(xa * inv) * w)
+    rel = lambda t: float((t - ref).norm() / ref.norm())
+    err_last, err_first = rel(_mix32(h, y, m, x, True)), rel(_mix32(h, y, m, x, False))
+    assert rel(out) < 0.25 * err_last + 0.75 * err_first, (rel(out), err_last, err_first)
