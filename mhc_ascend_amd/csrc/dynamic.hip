@@ -18,6 +18,7 @@
 //   proj_bwd_mfma_kernel dx += dP.Phi + s x_flat, dPhi partials (bf16 MFMA, split operands)
 #include "mhc_device.h"
 #include "mhc_internal.h"
+#include "proj_plan.h"
 #include "mhc_rows.h"
 
 namespace mhc {
@@ -385,8 +386,17 @@ __global__ __launch_bounds__(256) void proj_xsplit_kernel(const float* __restric
     if (threadIdx.x == 0) ss_part[(int64_t)q * B + b] = ss[0];
 }
 
+// TL (proj_stream_two_level): the large sum is rounded once or twice per k step
+// and not with each of its 3 or 6 products, for chains that few splits made
+// longer: the step's products are summed from the smallest on before they join
+// it, or, where a workgroup has the CU's registers to itself, the products below
+// hi . hi have a sum of their own.  P at n = 32 against float64 (rms): 128 x 1280
+// fp32 2.7e-7 for 7.2e-7, 1500 x 256 bf16 2.3e-7 for 7.0e-7.
 template <int XPL, int MT, bool PHI_PLANES>
-__global__ __launch_bounds__(256) void proj_stream_kernel(
+constexpr bool stream_one_wg() { return XPL == 3 && MT == 4 && PHI_PLANES; }
+
+template <int XPL, int MT, bool PHI_PLANES, bool TL>
+__global__ __launch_bounds__(256, (TL && !stream_one_wg<XPL, MT, PHI_PLANES>()) ? 2 : 1) void proj_stream_kernel(
     const bf16_t* __restrict__ xpl, const float* __restrict__ phi_pre, const float* __restrict__ phi_post,
     const float* __restrict__ phi_res, int n_pre, const uint4* __restrict__ phif, int np, float* __restrict__ p_part,
     float* __restrict__ ss_part, int64_t B, int64_t K, int64_t kchunk, int ks, int oblocks, int64_t tblocks) {
@@ -523,6 +533,14 @@ __global__ __launch_bounds__(256) void proj_stream_kernel(
             }
         }
     };
+    // the step's own sum
+    constexpr bool TWO = TL && stream_one_wg<XPL, MT, PHI_PLANES>();
+    const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t accs[TWO ? MT : 1][2];
+    if constexpr (TWO) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) accs[mt][0] = accs[mt][1] = zero;
+    }
     auto compute = [&](int buf, int kk, const u32x4_t (&ph)[2], const u32x4_t (&pm)[2], const u32x4_t (&pl)[2])
         __attribute__((always_inline)) {
 #pragma unroll
@@ -541,9 +559,16 @@ __global__ __launch_bounds__(256) void proj_stream_kernel(
                 }
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
-                    acc[mt][nt] = mfma16x16x32(a0, ph[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a0, pm[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a0, pl[nt], acc[mt][nt]);
+                    if constexpr (TL) {
+                        f32x4_t c = mfma16x16x32(a0, pl[nt], zero);
+                        c = mfma16x16x32(a0, pm[nt], c);
+                        c = mfma16x16x32(a0, ph[nt], c);
+                        acc[mt][nt] += c;
+                    } else {
+                        acc[mt][nt] = mfma16x16x32(a0, ph[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a0, pm[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a0, pl[nt], acc[mt][nt]);
+                    }
                 }
             } else {
                 const uint4 q1 = *reinterpret_cast<const uint4*>(base + TB * PITCH);
@@ -552,12 +577,29 @@ __global__ __launch_bounds__(256) void proj_stream_kernel(
                 const u32x4_t a2 = u32x4_t{q2.x, q2.y, q2.z, q2.w};
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
-                    acc[mt][nt] = mfma16x16x32(a0, ph[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a0, pm[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a1, ph[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a0, pl[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a1, pm[nt], acc[mt][nt]);
-                    acc[mt][nt] = mfma16x16x32(a2, ph[nt], acc[mt][nt]);
+                    if constexpr (TWO) {
+                        acc[mt][nt] = mfma16x16x32(a0, ph[nt], acc[mt][nt]);
+                        accs[mt][nt] = mfma16x16x32(a0, pm[nt], accs[mt][nt]);
+                        accs[mt][nt] = mfma16x16x32(a1, ph[nt], accs[mt][nt]);
+                        accs[mt][nt] = mfma16x16x32(a0, pl[nt], accs[mt][nt]);
+                        accs[mt][nt] = mfma16x16x32(a1, pm[nt], accs[mt][nt]);
+                        accs[mt][nt] = mfma16x16x32(a2, ph[nt], accs[mt][nt]);
+                    } else if constexpr (TL) {
+                        f32x4_t c = mfma16x16x32(a0, pl[nt], zero);
+                        c = mfma16x16x32(a1, pm[nt], c);
+                        c = mfma16x16x32(a2, ph[nt], c);
+                        c = mfma16x16x32(a0, pm[nt], c);
+                        c = mfma16x16x32(a1, ph[nt], c);
+                        c = mfma16x16x32(a0, ph[nt], c);
+                        acc[mt][nt] += c;
+                    } else {
+                        acc[mt][nt] = mfma16x16x32(a0, ph[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a0, pm[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a1, ph[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a0, pl[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a1, pm[nt], acc[mt][nt]);
+                        acc[mt][nt] = mfma16x16x32(a2, ph[nt], acc[mt][nt]);
+                    }
                 }
             }
         }
@@ -597,6 +639,13 @@ __global__ __launch_bounds__(256) void proj_stream_kernel(
         }
         if (st < nst) step(st, p0, p2);
         if (st + 1 < nst) step(st + 1, p1, p0);
+    }
+    if constexpr (TWO) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            acc[mt][0] += accs[mt][0];
+            acc[mt][1] += accs[mt][1];
+        }
     }
     if (wave_on) {
         // D[token 16 mt + 4 kg + i][output ow + 16 nt + row]
@@ -2211,8 +2260,8 @@ static int proj_stream_mt(int64_t B) { return B > 32 ? 4 : 2; }
 
 template <int XPL, int PHI>
 static const void* proj_stream_fn(int mt) {
-    if (mt == 2) return reinterpret_cast<const void*>(&proj_stream_kernel<XPL, 2, PHI != 0>);
-    return reinterpret_cast<const void*>(&proj_stream_kernel<XPL, 4, PHI != 0>);
+    if (mt == 2) return reinterpret_cast<const void*>(&proj_stream_kernel<XPL, 2, PHI != 0, false>);
+    return reinterpret_cast<const void*>(&proj_stream_kernel<XPL, 4, PHI != 0, false>);
 }
 
 // The streaming projection pays off where Phi outweighs x (np > 128, n >= 16:
@@ -2220,30 +2269,22 @@ static const void* proj_stream_fn(int mt) {
 // x re-reads are few, is faster.
 bool proj_stream_path(int np) { return np > kStreamOB; }
 
-// K splits of the streaming projection: the count whose rounds of resident
-// workgroups (occupancy of the fp32-x kernel, whose LDS stage is the larger)
-// take the fewest stages, three added per workgroup for its prologue and
-// stores; at least two stages per split, splits x tokens at most 4096 (the
-// partials the coefficient kernel adds per token).  n = 32, 128 tokens, C =
-// 1280: 28 splits are 504 workgroups, one round; 32, the cap, left 64 of 576 to
-// a second one (110 us, 88 with the workgroup order and the packed split below).
-static int proj_stream_ksplit(int64_t B, int64_t K, int np) {
+// (occupancy of the fp32-x kernel, whose LDS stage is the larger)
+static StreamFill stream_fill(int64_t B, int64_t K, int np) {
     const int mt = proj_stream_mt(B);
-    const int64_t groups0 = ((B + 16 * mt - 1) / (16 * mt)) * ((np + kStreamOB - 1) / kStreamOB);
     const int per_cu = occupancy_per_cu(proj_stream_fn<3, 0>(mt), 256, 0);
-    const int64_t slots = (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : 1);
-    const int64_t stages = (K + kStreamKS - 1) / kStreamKS;
-    const int64_t kcap = B > 0 ? (4096 + B - 1) / B : 1;
-    const int64_t kmax = (stages + 1) / 2;
-    int64_t best = 1, best_cost = 0;
-    for (int64_t ks = 1; ks <= kcap && ks <= kmax; ++ks) {
-        const int64_t cost = (groups0 * ks + slots - 1) / slots * ((stages + ks - 1) / ks + 3);
-        if (ks == 1 || cost * 50 < best_cost * 49) {
-            best = ks;
-            best_cost = cost;
-        }
-    }
-    return (int)best;
+    return stream_fill_of(B, K, np, mt, kStreamOB, kStreamKS, (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : 1));
+}
+
+// K splits of the streaming projection (proj_plan.h).
+static int proj_stream_ksplit(int64_t B, int64_t K, int np) { return stream_ksplit(stream_fill(B, K, np)); }
+
+// The splits that fill two rounds of workgroups (the last one part empty) give
+// shorter chains than `ks`: their sums are then taken in two levels.
+static bool proj_stream_two_level(int64_t B, int64_t K, int np, int ks) {
+    const StreamFill f = stream_fill(B, K, np);
+    const int64_t fill = stream_fill_splits(f);
+    return (f.stages + ks - 1) / ks > (f.stages + fill - 1) / fill;
 }
 
 // K splits so that token blocks x splits x output tiles fill about two
@@ -2303,13 +2344,19 @@ hipError_t launch_proj_stream(int x_dtype, const void* x, bf16_raw_t* xplanes, c
         xp = reinterpret_cast<const bf16_t*>(xplanes);
     }
     const uint4* phif = reinterpret_cast<const uint4*>(phib);
-#define MHC_STREAM(XPL_, MT_)                                                                                   \
-    if (phib) {                                                                                                 \
-        MHC_LAUNCH_GGL((proj_stream_kernel<XPL_, MT_, true>), grid, dim3(256), 0, s, xp, phi_pre, phi_post,   \
-                           phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, tb);                                                          \
-    } else {                                                                                                    \
-        MHC_LAUNCH_GGL((proj_stream_kernel<XPL_, MT_, false>), grid, dim3(256), 0, s, xp, phi_pre, phi_post,  \
-                           phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, tb);                                                          \
+    const bool tl = proj_stream_path(np) && proj_stream_two_level(B, K, np, ks);
+#define MHC_STREAM_(XPL_, MT_, PHI_, TL_)                                                                     \
+    MHC_LAUNCH_GGL((proj_stream_kernel<XPL_, MT_, PHI_, TL_>), grid, dim3(256), 0, s, xp, phi_pre, phi_post,  \
+                   phi_res, n_pre, phif, np, p_part, ss_part, B, K, kchunk, ks, ob, tb)
+#define MHC_STREAM(XPL_, MT_)                        \
+    if (phib && tl) {                                \
+        MHC_STREAM_(XPL_, MT_, true, true);          \
+    } else if (phib) {                               \
+        MHC_STREAM_(XPL_, MT_, true, false);         \
+    } else if (tl) {                                 \
+        MHC_STREAM_(XPL_, MT_, false, true);         \
+    } else {                                         \
+        MHC_STREAM_(XPL_, MT_, false, false);        \
     }
 #define MHC_STREAM_MT(XPL_)                               \
     if (mt == 2) {                                        \
@@ -2324,6 +2371,7 @@ hipError_t launch_proj_stream(int x_dtype, const void* x, bf16_raw_t* xplanes, c
     }
 #undef MHC_STREAM_MT
 #undef MHC_STREAM
+#undef MHC_STREAM_
     timing_end(tok, s);
     return hipGetLastError();
 }

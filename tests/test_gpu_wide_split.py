@@ -82,3 +82,34 @@ def test_wide_backward_few_tokens(device):
     assert_close(x.grad, xr.grad, 1e-3, grad_atol(xr.grad, 1e-5), "dx")
     for nm, a, e in zip(PARAMS[1:], ps[1:], pr[1:]):
         assert_close(a.grad, e.grad, 1e-3, grad_atol(e.grad, 1e-4), f"d_{nm}")
+
+
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,C,infer", [(128, 1280, False), (300, 512, False), (1500, 256, False), (20, 2048, False),
+                                       (1100, 128, True), (1100, 128, False)])
+def test_projection_error_of_long_chains(device, B, C, infer, x_dtype):
+    """P of n = 32 where fewer K splits than fill the chip make a chain longer
+    (32 rows and fewer, and more), against float64, relative to its norm: eight
+    half-ulps (8 x 2^-24; a sum rounded with each of a step's products exceeds
+    them).  The forward-only entry keeps no P: its h_post stands for it."""
+    n = 32
+    np_ = n * n + 2 * n
+    g = torch.Generator().manual_seed(B + C)
+    x = torch.randn(B, n, C, generator=g).to(x_dtype).to(device)
+    phi = [(0.02 * torch.randn(r, n * C, generator=g)).to(device) for r in (n, n, n * n)]
+    one, zero = torch.ones(1, device=device), torch.zeros(n * n, device=device)
+    w = torch.ones(C, device=device)
+    args = (one, one, one, zero[:n], zero[:n], zero.view(n, n))
+    ref = x.double().reshape(B, -1) @ torch.cat(phi).double().t()
+    if infer:
+        packed = native.mhc_layer_dynamic_pack(w, *phi)
+        # out - M x = h_post y with h_post near 1 + P / (2 r_h): too coarse for P,
+        # so only that both entries agree to a few of its roundings
+        a = native.mhc_layer_dynamic_infer(x, packed, *args)
+        b, _ = native.mhc_layer_dynamic_fwd(x, w, *phi, *args)
+        assert float((a - b).double().norm() / b.double().norm()) < 8 * 2.0 ** -24
+        return
+    _, saved = native.mhc_layer_dynamic_fwd(x, w, *phi, *args)
+    off = (C + 63) // 64 * 64 + (B * np_ + 63) // 64 * 64
+    P = saved.view(-1)[off:off + B * np_].view(B, np_).double()
+    assert float((P - ref).norm() / ref.norm()) < 8 * 2.0 ** -24
