@@ -38,14 +38,21 @@ inline int64_t stream_fill_splits(const StreamFill& f) {
 // takes 2% less.  n = 32, 128 tokens, C = 1280: 28 splits are 504 workgroups, one
 // round; 32, the cap, left 64 of 576 to a second one (110 us, 88 with the
 // workgroup order and the packed split of the kernel).
+// (Of the counts with the same stages per split the first has the fewest rounds:
+// the search steps from one to the next, some 2 sqrt(stages) of them.  It runs in
+// every size query and launch; each count in turn took 1024 steps for a single
+// token at n = 32, 4096 channels.)
 inline int stream_ksplit(const StreamFill& f) {
     int64_t best = 1, best_cost = 0;
-    for (int64_t ks = 1; ks <= f.kmax; ++ks) {
-        const int64_t cost = (f.groups * ks + f.slots - 1) / f.slots * ((f.stages + ks - 1) / ks + 3);
+    for (int64_t ks = 1; ks <= f.kmax;) {
+        const int64_t per = (f.stages + ks - 1) / ks;
+        const int64_t cost = (f.groups * ks + f.slots - 1) / f.slots * (per + 3);
         if (ks == 1 || cost * 50 < best_cost * 49) {
             best = ks;
             best_cost = cost;
         }
+        if (per <= 1) break;
+        ks = (f.stages + per - 2) / (per - 1);
     }
     return (int)best;
 }

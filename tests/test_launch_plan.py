@@ -1,6 +1,6 @@
-"""The wrapper's launch rules (csrc/wrapper_plan.h), compiled for the host: what
-the kernels read and write stays inside what the rules lay out, over the sizes,
-stream counts, token counts and CU counts that the entry points take."""
+"""The launch rules (csrc/wrapper_plan.h, csrc/proj_plan.h), compiled for the host:
+what the kernels read and write stays inside what the rules lay out, over the
+sizes, stream counts, token counts and CU counts that the entry points take."""
 import ctypes
 import os
 import shutil
@@ -11,7 +11,13 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mhc_ascend_amd", "csrc")
 
 SOURCE = r"""
+#include "proj_plan.h"
 #include "wrapper_plan.h"
+extern "C" void stream_split(int64_t B, int64_t K, int np, int mt, int64_t slots, int64_t* out) {
+    const mhc::StreamFill f = mhc::stream_fill_of(B, K, np, mt, 128, 64, slots);
+    out[0] = mhc::stream_ksplit(f); out[1] = f.groups; out[2] = f.stages; out[3] = f.kmax;
+    out[4] = mhc::stream_fill_splits(f);
+}
 extern "C" void fold_split(int bf16, int64_t B, int64_t C, int np, int cus, int* out) {
     const mhc::WfoldSplit s = mhc::wfold_split(bf16, B, C, np, cus);
     out[0] = s.ks; out[1] = s.chunk; out[2] = s.steps;
@@ -51,3 +57,26 @@ def test_fold_splits_all_hold_steps(plan, bf16, cus):
                 assert ks >= 1 and chunk >= 1 and steps * 32 >= C, what
                 assert (ks - 1) * chunk < steps <= ks * chunk, what
                 assert not bf16 or chunk % 2 == 0, what
+
+
+def test_stream_splits_are_those_of_the_full_search(plan):
+    """The split count steps over counts that cannot win; trying every one in turn
+    gives the same (rounds of workgroups x (stages per split + 3), a larger count
+    only where that is 2% less)."""
+    out = (ctypes.c_int64 * 5)()
+    for n in (11, 12, 16, 24, 32, 48, 64):
+        for C in (32, 64, 256, 512, 1280, 2048, 4096, 12288):
+            for B in (1, 2, 7, 16, 32, 33, 64, 100, 128, 300, 512, 1000, 1500, 4096, 70000):
+                for slots in (256, 512, 768):
+                    mt = 4 if B > 32 else 2
+                    plan.stream_split(ctypes.c_int64(B), ctypes.c_int64(n * C), n * n + 2 * n, mt,
+                                      ctypes.c_int64(slots), out)
+                    ks, groups, stages, kmax, fill = list(out)
+                    assert groups == -(-B // (16 * mt)) * -(-(n * n + 2 * n) // 128) and stages == -(-n * C // 64)
+                    assert kmax == max(1, min((stages + 1) // 2, -(-4096 // B))) and 1 <= fill <= kmax
+                    best, best_cost = 1, None
+                    for k in range(1, kmax + 1):
+                        cost = -(-groups * k // slots) * (-(-stages // k) + 3)
+                        if best_cost is None or cost * 50 < best_cost * 49:
+                            best, best_cost = k, cost
+                    assert ks == best, (n, C, B, slots, ks, best)
