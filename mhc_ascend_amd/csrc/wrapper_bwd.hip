@@ -29,6 +29,7 @@
 // n = 16, 4096 x 2048 fp32: 39 us for 905 through stream rows in memory.
 #include "mhc_device.h"
 #include "mhc_internal.h"
+#include "wrapper_plan.h"
 
 namespace mhc {
 
@@ -87,6 +88,7 @@ __device__ __forceinline__ void vlds_put4(char* p, const float (&v)[4]) {
 
 constexpr int kVbThreads = 512;
 constexpr int kVbCols = kVbThreads / 64 * 16;
+static_assert(kVbCols == kWbwdCols, "the host's column blocks");
 constexpr int kVbEp = kWgEp + 4;  // the record, then s (padded to 16 bytes)
 
 }  // namespace
@@ -656,43 +658,17 @@ __global__ __launch_bounds__(256) void wrap_sums_kernel(WrapSums a) {
 // Host side
 // ---------------------------------------------------------------------------
 // bf16 'decay' past n = 8 would need a product per stream beside 2n > 16
-// rows: those shapes keep the kernels of wrapper_gen.hip.
+// rows, and rows of more than 1.86M channels a tile of less than one round: those
+// shapes keep the kernels of wrapper_gen.hip.
 bool wbwd_shape_ok(int dt, int n, bool decay, int64_t C) {
     return n >= 2 && n <= kWgMaxN && C >= 8 && C % 8 == 0 && C <= (int64_t(1) << 21) &&
-           (n <= 8 || dt != kBF16 || !decay);
+           wbwd_max_tile(C, dp_stride(2 * n + n * n)) >= kWbwdRound && (n <= 8 || dt != kBF16 || !decay);
 }
 
 int wbwd_streams(int dt, int n, bool decay) { return dt == kBF16 && decay ? n : 2; }
 
-// rows of a tile: each buffer (4 C bytes a row at most, or dP's row) under 2 GiB
-// with the pipeline's overrun
-static int64_t wbwd_max_tile(int n, int64_t C) {
-    const int64_t row = C > dp_stride(2 * n + n * n) ? C : dp_stride(2 * n + n * n);
-    return ((int64_t(1) << 31) - 1) / (row * 4) - 6 * 32;
-}
-
-// Token tiles: one workgroup fits a CU (250 VGPRs, 8 waves), so column blocks x
-// tiles is one to four rounds of workgroups, whichever leaves the fewest CUs
-// idle in the last one (at 56 column blocks one round has 224 workgroups and
-// took 1.42 ms at n = 8, two have 504 and took 1.28); at least 96 tokens each,
-// at most wbwd_max_tile.
 int wbwd_tiles(int n, int64_t B, int64_t C) {
-    const int64_t gx = (C + kVbCols - 1) / kVbCols;
-    const int64_t cus = device_cu_count();
-    int64_t tiles = 1, best = 0;
-    for (int64_t k = 1; k <= 4; ++k) {
-        const int64_t fill = k * cus / gx * gx * 1000 / (k * cus);
-        if (fill > best + 20) {
-            best = fill;
-            tiles = k * cus / gx;
-        }
-    }
-    const int64_t by_stage = (B + 95) / 96;
-    if (tiles > by_stage) tiles = by_stage;
-    if (tiles < 1) tiles = 1;
-    const int64_t mt = wbwd_max_tile(n, C) / 96 * 96;
-    if (mt >= 96 && (B + tiles - 1) / tiles > mt) tiles = (B + mt - 1) / mt;
-    return (int)tiles;
+    return (int)wbwd_split(B, C, dp_stride(2 * n + n * n), device_cu_count());
 }
 
 size_t wbwd_fold_bytes(int n, int64_t C) { return n > 8 ? (size_t)4 * n * C * sizeof(float) : 0; }
@@ -703,9 +679,8 @@ hipError_t launch_wbwd(int dt, int n, bool decay, const float* g, const void* re
                        int tiles, int64_t B, int64_t C, hipStream_t s) {
     if (B == 0) return hipSuccess;
     if (!wbwd_shape_ok(dt, n, decay, C) || tiles < 1 || (n > 8 && !fold)) return hipErrorInvalidValue;
-    int64_t tile = (B + tiles - 1) / tiles;
-    tile = (tile + 95) / 96 * 96;
-    if (tile > wbwd_max_tile(n, C)) return hipErrorInvalidValue;
+    const int64_t tile = wbwd_tile(B, tiles);
+    if (tile > wbwd_max_tile(C, dp_stride)) return hipErrorInvalidValue;
     const int Ci = (int)C;
     if (n > 8) {
         int64_t blocks = ((int64_t)2 * n * C + 255) / 256;

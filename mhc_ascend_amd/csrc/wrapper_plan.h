@@ -65,4 +65,42 @@ inline WfoldSplit wfold_split(bool bf16, int64_t B, int64_t C, int np, int cus) 
     return s;
 }
 
+// ---- dynamic-H backward (wrapper_bwd.hip) --------------------------------------
+constexpr int kWbwdCols = 128;   // channels per workgroup
+constexpr int kWbwdRound = 96;   // tokens of a round of its pipeline (three stages)
+
+// Rows of a tile: each buffer (4 C bytes a row at most, or dP's row) under 2 GiB
+// with the pipeline's overrun of six stages.
+inline int64_t wbwd_max_tile(int64_t C, int64_t dp_row) {
+    return ((int64_t(1) << 31) - 1) / ((C > dp_row ? C : dp_row) * 4) - 6 * 32;
+}
+
+// Tokens of each of `tiles` tiles.
+inline int64_t wbwd_tile(int64_t B, int64_t tiles) {
+    return ((B + tiles - 1) / tiles + kWbwdRound - 1) / kWbwdRound * kWbwdRound;
+}
+
+// Token tiles: one workgroup fits a CU (250 VGPRs, 8 waves), so column blocks x
+// tiles is one to four rounds of workgroups, whichever leaves the fewest CUs
+// idle in the last one (at 56 column blocks one round has 224 workgroups and
+// took 1.42 ms at n = 8, two have 504 and took 1.28); whole pipeline rounds each,
+// at most wbwd_max_tile (which holds one round at least).
+inline int64_t wbwd_split(int64_t B, int64_t C, int64_t dp_row, int64_t cus) {
+    const int64_t gx = (C + kWbwdCols - 1) / kWbwdCols;
+    int64_t tiles = 1, best = 0;
+    for (int64_t k = 1; k <= 4; ++k) {
+        const int64_t fill = k * cus / gx * gx * 1000 / (k * cus);
+        if (fill > best + 20) {
+            best = fill;
+            tiles = k * cus / gx;
+        }
+    }
+    const int64_t rounds = (B + kWbwdRound - 1) / kWbwdRound;
+    if (tiles > rounds) tiles = rounds;
+    if (tiles < 1) tiles = 1;
+    const int64_t mt = wbwd_max_tile(C, dp_row) / kWbwdRound * kWbwdRound;
+    if (mt >= kWbwdRound && wbwd_tile(B, tiles) > mt) tiles = (B + mt - 1) / mt;
+    return tiles;
+}
+
 }  // namespace mhc

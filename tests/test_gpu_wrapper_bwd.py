@@ -24,3 +24,9 @@ def test_shapes(device, n, T, C, dtype, mode):
 def test_many_tiles(device, dtype):
     # one column block: as many token tiles as CUs, a tile of four stages
     _run(device, 5, 256 * 97, 64, dtype, "decay", seed=3)
+
+
+def test_widest_rows(device):
+    """n = 2 past 1.86M channels, where a tile's 2 GiB hold less than one round of
+    stages: the backward runs on the kernels for other shapes."""
+    _run(device, 2, 3, 1_900_032, torch.float32, "zero", seed=4)

@@ -18,6 +18,10 @@ extern "C" void stream_split(int64_t B, int64_t K, int np, int mt, int64_t slots
     out[0] = mhc::stream_ksplit(f); out[1] = f.groups; out[2] = f.stages; out[3] = f.kmax;
     out[4] = mhc::stream_fill_splits(f);
 }
+extern "C" void bwd_split(int64_t B, int64_t C, int64_t dp_row, int64_t cus, int64_t* out) {
+    out[0] = mhc::wbwd_split(B, C, dp_row, cus); out[1] = mhc::wbwd_tile(B, out[0]);
+    out[2] = mhc::wbwd_max_tile(C, dp_row);
+}
 extern "C" void fold_split(int bf16, int64_t B, int64_t C, int np, int cus, int* out) {
     const mhc::WfoldSplit s = mhc::wfold_split(bf16, B, C, np, cus);
     out[0] = s.ks; out[1] = s.chunk; out[2] = s.steps;
@@ -80,3 +84,20 @@ def test_stream_splits_are_those_of_the_full_search(plan):
                         if best_cost is None or cost * 50 < best_cost * 49:
                             best, best_cost = k, cost
                     assert ks == best, (n, C, B, slots, ks, best)
+
+
+@pytest.mark.parametrize("cus", [1, 64, 256, 304])
+def test_backward_tiles(plan, cus):
+    """Token tiles of the wrapper's backward: whole pipeline rounds that cover the
+    tokens, and within the 2 GiB of a tile's buffers wherever that
+    holds one round."""
+    out = (ctypes.c_int64 * 3)()
+    for n in (2, 5, 8, 12, 32):
+        dp_row = -(-(n * n + 2 * n) // 32) * 32
+        for C in (8, 64, 120, 1024, 1040, 4096, 7168, 16392, 100000, 1 << 20, 1_860_000, 1_900_032, 1 << 21):
+            for B in (1, 31, 96, 97, 193, 1000, 2047, 4096, 24832, 65536, 1_000_003):
+                plan.bwd_split(ctypes.c_int64(B), ctypes.c_int64(C), ctypes.c_int64(dp_row), ctypes.c_int64(cus), out)
+                tiles, tile, most = list(out)
+                what = (n, C, B, tiles, tile, most)
+                assert tiles >= 1 and tile % 96 == 0 and B <= tiles * tile, what
+                assert tile <= most or most < 96, what
