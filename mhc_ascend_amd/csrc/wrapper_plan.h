@@ -83,8 +83,8 @@ inline int64_t wbwd_tile(int64_t B, int64_t tiles) {
 // Token tiles: one workgroup fits a CU (250 VGPRs, 8 waves), so column blocks x
 // tiles is one to four rounds of workgroups, whichever leaves the fewest CUs
 // idle in the last one (at 56 column blocks one round has 224 workgroups and
-// took 1.42 ms at n = 8, two have 504 and took 1.28); whole pipeline rounds each,
-// at most wbwd_max_tile (which holds one round at least).
+// took 1.42 ms at n = 8, two have 504 and took 1.28); whole pipeline rounds each
+// and none without tokens, at most wbwd_max_tile (which holds one round at least).
 inline int64_t wbwd_split(int64_t B, int64_t C, int64_t dp_row, int64_t cus) {
     const int64_t gx = (C + kWbwdCols - 1) / kWbwdCols;
     int64_t tiles = 1, best = 0;
@@ -100,7 +100,8 @@ inline int64_t wbwd_split(int64_t B, int64_t C, int64_t dp_row, int64_t cus) {
     if (tiles < 1) tiles = 1;
     const int64_t mt = wbwd_max_tile(C, dp_row) / kWbwdRound * kWbwdRound;
     if (mt >= kWbwdRound && wbwd_tile(B, tiles) > mt) tiles = (B + mt - 1) / mt;
-    return tiles;
+    const int64_t tile = wbwd_tile(B, tiles);
+    return tile > 0 ? (B + tile - 1) / tile : 1;
 }
 
 }  // namespace mhc

@@ -22,7 +22,7 @@ def test_shapes(device, n, T, C, dtype, mode):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_many_tiles(device, dtype):
-    # one column block: as many token tiles as CUs, a tile of four stages
+    # one column block: half as many token tiles as CUs, of two rounds of stages
     _run(device, 5, 256 * 97, 64, dtype, "decay", seed=3)
 
 
