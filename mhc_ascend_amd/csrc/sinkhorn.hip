@@ -83,8 +83,10 @@ __global__ __launch_bounds__(256) void sinkhorn_bwd_kernel(const float* __restri
 // issues more instructions in total, so it is used for batches that leave the
 // chip latency-bound; large batches (throughput-bound) keep one row per lane,
 // except where that form's adjoint recomputes its history (n = 5..8 past
-// SkHist's iterations: O(iters^2) steps).
-constexpr int64_t kSkElMaxBatch = 16384;
+// SkHist's iterations: O(iters^2) steps).  n = 5..8, whose matrix takes a whole
+// wave: 8.9 us for 47 at 2048 matrices, 20 iterations, backward; forward 9.5 for
+// 8.2 at 8192.
+constexpr int64_t sk_el_max_batch(int n) { return n <= 4 ? 16384 : 4096; }
 template <int S>
 __global__ __launch_bounds__(256) void sinkhorn_el_fwd_kernel(const float* __restrict__ inp, float* __restrict__ out,
                                                               int n, int64_t batch, int iters, float eps) {
@@ -225,12 +227,29 @@ __global__ __launch_bounds__(skb::kThreads) void sinkhorn_b32_kernel(const float
     }
 }
 
-// Both directions of 9 <= n <= 32 (grad_out null: forward); false: the shape
-// or the iteration count stays with the row-per-lane kernels.
+// Both directions of 9 <= n <= 32 (grad_out null: forward); false: the shape,
+// the batch or the iteration count stays with the row-per-lane kernels.
+//
+// A matrix per wave or workgroup has the short chain, the row-per-lane kernels
+// the fewer instructions a matrix: past the batch that fills the chip they are
+// faster forward (20 iterations, us, tiled / row per lane: n = 9 9.8 / 11.5 at
+// 2048, 33 / 14 at 8192; n = 16 10.5 / 20 at 2048, 34 / 28 at 8192; n = 17 11 / 24 at
+// 256, 44 / 27 at 2048; n = 32 47 / 51 at 2048, 170 / 96 at 8192).  Their adjoint
+// recomputes the state, iters^2 steps, so backward the line is the batch at few
+// iterations only (n = 9 at 131,072: 20 iterations 1086 / 1371, 10 611 / 394; n = 32
+// 5234 / 11,018, 3096 / 3221; at 2048 and 10 iterations 12 / 35 and 49 / 128).
+static bool sinkhorn_tiled(int n, int64_t batch, int iters, bool bwd) {
+    if (n <= 8 || n > skb::kN || batch > 0x7fffffff) return false;
+    const bool wave = n <= skw16::kN;
+    if (!bwd) return batch <= (wave ? 256 : 48) * (int64_t)n;
+    if (iters > (wave ? skw16::kTMax : skb::kTMax)) return false;
+    const int64_t steps = (int64_t)n * iters;
+    return steps >= (wave ? 170 : 300) || batch <= (wave ? 64 : 16) * steps;
+}
+
 static bool launch_sinkhorn_tiled(int n, const float* grad_out, const float* inp, float* out, int64_t batch, int iters,
                                   float eps, hipStream_t s) {
-    if (n <= 8 || n > skb::kN || batch > 0x7fffffff) return false;
-    if (grad_out && iters > (n <= skw16::kN ? skw16::kTMax : skb::kTMax)) return false;
+    if (!sinkhorn_tiled(n, batch, iters, grad_out != nullptr)) return false;
     if (n <= skw16::kN) {
         MHC_LAUNCH_GGL(sinkhorn_w16_kernel, dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, s, grad_out, inp, out, n,
                        batch, iters, eps);
@@ -272,7 +291,7 @@ hipError_t launch_sinkhorn_fwd(int n, const float* inp, float* out, int64_t batc
     const int64_t threads = batch * G;
     const unsigned blocks = (unsigned)((threads + 255) / 256);
     const int tok = timing_begin("sinkhorn_fwd", s);
-    if (n >= 3 && n <= 8 && batch < kSkElMaxBatch) {
+    if (n >= 3 && n <= 8 && batch < sk_el_max_batch(n)) {
         if (sk_el_size(n) == 4) {
             MHC_LAUNCH_GGL(sinkhorn_el_fwd_kernel<4>, dim3((unsigned)((batch * 16 + 255) / 256)), dim3(256), 0, s, inp,
                            out, n, batch, iters, eps);
@@ -300,7 +319,7 @@ hipError_t launch_sinkhorn_bwd(int n, const float* grad_out, const float* inp, f
     const unsigned blocks = (unsigned)((threads + 255) / 256);
     const int tok = timing_begin("sinkhorn_bwd", s);
     const bool recompute = n > 4 && n <= 8 && iters > SkHist<8>::TMAX;
-    if (n >= 3 && n <= 8 && (batch < kSkElMaxBatch || recompute)) {
+    if (n >= 3 && n <= 8 && (batch < sk_el_max_batch(n) || recompute)) {
         if (sk_el_size(n) == 4) {
             MHC_LAUNCH_GGL(sinkhorn_el_bwd_kernel<4>, dim3((unsigned)((batch * 16 + 255) / 256)), dim3(256), 0, s,
                            grad_out, inp, grad_inp, n, batch, iters, eps);

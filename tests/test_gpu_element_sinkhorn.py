@@ -62,3 +62,22 @@ def test_dynamic_coefficients(device, n, B, C, iters):
                                b_std=0.5)
     _check_dyn(_run_dyn(d, device, iters=iters), _oracle_dyn(d, iters=iters), torch.float32,
                f"n={n} B={B} C={C} T={iters}")
+
+
+# (n, batch, iters): one past the batch (and, backward, below the iterations) up
+# to which a matrix is spread over a wave or workgroup, and on it
+@pytest.mark.parametrize("n,B,iters", [(9, 2304, 5), (9, 2305, 5), (9, 2881, 5), (16, 4097, 10), (16, 5121, 5),
+                                       (17, 817, 5), (17, 1361, 5), (32, 1537, 9), (32, 2561, 5), (5, 4096, 12),
+                                       (8, 4097, 12)])
+def test_sinkhorn_batches_around_the_forms(device, n, B, iters):
+    g = torch.Generator().manual_seed(n + B + iters)
+    a = torch.exp(torch.randn(B, n, n, generator=g))
+    go = torch.randn(a.shape, generator=g)
+    ad = a.to(device).requires_grad_(True)
+    out = mhc.sinkhorn_knopp(ad, iters, 1e-8)
+    out.backward(go.to(device))
+    idx = torch.cat([torch.arange(40), torch.arange(B - 40, B)])
+    ref = torch.from_numpy(csk.sinkhorn_fwd(a[idx].double().numpy(), iters, 1e-8))
+    gref = torch.from_numpy(csk.sinkhorn_bwd(go[idx].double().numpy(), a[idx].double().numpy(), iters, 1e-8))
+    assert_close(out.cpu()[idx], ref, 1e-4, 1e-5, f"SK fwd n={n} B={B} T={iters}")
+    assert_close(ad.grad.cpu()[idx], gref, 1e-3, max(grad_atol(gref, 1e-5), 1e-6), f"SK bwd n={n} B={B} T={iters}")
