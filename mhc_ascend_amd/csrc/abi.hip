@@ -1097,7 +1097,7 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
     const int64_t K = (int64_t)n * hidden;
     const float* w32 = saved + d.w_off;
     hipError_t e = hipSuccess;
-    int rows_w = w.grid, rows_p = w.tiles, rows_c = w.cblocks;
+    int rows_w = w.grid, rows_p = w.tiles, rows_c = dyn_coef_bwd_rows(n, batch, num_iters, true);
     if (batch == 0) {
         rows_w = rows_c = 1;
         e = launch_fill_zero(dw_part, hidden, s);
@@ -1614,7 +1614,7 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
                      ((uintptr_t)grad_out | (uintptr_t)residual | (uintptr_t)branch | (uintptr_t)grad_residual |
                       (uintptr_t)grad_branch) % 16 == 0;
     hipError_t e = hipSuccess;
-    int rows_w = fold ? w.ftiles : w.dtiles, rows_c = w.cblocks;
+    int rows_w = fold ? w.ftiles : w.dtiles, rows_c = dyn_coef_bwd_rows(n, tokens, num_iters, rows == np);
     if (tokens == 0) {
         rows_w = rows_c = 1;
         e = launch_fill_zero(dw_part, hidden, s);
@@ -1639,12 +1639,12 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
                                 phi_post, (float*)(ws + w.phif_off), grad_residual, grad_branch, dw_part, part,
                                 w.wtiles, tokens, hidden, s);
             const int nst = wbwd_streams(dtype, n, decay);
-            const bool few = w.cblocks <= kWrapSumsMaxRows;
+            const bool few = rows_c <= kWrapSumsMaxRows;
             if (e == hipSuccess)
                 e = launch_wrap_sums(WrapSums{part, (int64_t)nst * rows * hidden, (int64_t)rows * hidden, hidden,
                                               w.wtiles, nst, rows, n, np, hidden, decay, grad_phi, dw_part, w.wtiles,
                                               weight_dtype == kBF16, grad_weight, few ? cpart : nullptr,
-                                              few ? w.cblocks : 0, grad_b, grad_alpha, 0},
+                                              few ? rows_c : 0, grad_b, grad_alpha, 0},
                                      s);
             if (few || e != hipSuccess) return hip_status(e);
         }
@@ -1925,7 +1925,7 @@ int mhc_wrapper_dynamic_bwd(const float* grad_out, const void* residual, const v
     const bool res_rows = !wrap_res_grad_vanishes(num_iters, sinkhorn_eps);
     const int npo = res_rows ? np : 2 * n;
     hipError_t e = hipSuccess;
-    int rows_p = w.tiles, rows_c = w.cblocks;
+    int rows_p = w.tiles, rows_c = dyn_coef_bwd_rows(n, tokens, num_iters, res_rows);
     if (tokens == 0) {
         rows_p = rows_c = 1;
         e = launch_fill_zero(dw_part, hidden, s);

@@ -1242,6 +1242,16 @@ __global__ __launch_bounds__(skb::kThreads) void dyn_coef32_bwd_kernel(
 constexpr int kCoefUnroll = 8;
 constexpr int64_t kCoefSplitTok = 1024;
 
+// Tokens up to which the spread forms of n = 5..8 (an element per lane) and 9..16
+// (a token per wave; half as many at n = 16) are taken in the forward: their chain
+// is shorter but they issue more instructions a token, and past this the chip is
+// full.  Spread / row per lane, 20 iterations, us: n = 8 8.0 / 8.3 at 4096
+// tokens, 12.4 / 9.4 at 8192, 68.7 / 41 at 65,536; n = 9 18.4 / 19.1, 31 / 22,
+// 189 / 86; n = 16 13 / 16 at 2048, 21.6 / 17.9 at 4096, 194 / 148 at 65,536.  (The
+// backwards keep the spread forms, whose history stays in registers: n = 8 184 /
+// 315 at 65,536, n = 16 155 / 258 at 16,384.)
+constexpr int64_t kCoefElMaxTok = 4096;
+
 template <int S, int QS>
 __global__ __launch_bounds__(256) void dyn_coef_el_fwd_kernel(
     const float* __restrict__ p_part, const float* __restrict__ ss_part, int ks, int64_t B, int64_t K,
@@ -2508,7 +2518,7 @@ hipError_t launch_dyn_coef_fwd(int n, const float* p_part, const float* ss_part,
                                const float* b_post, const float* b_res, float* coef, float* p_out, float* rh,
                                int iters, float sk_eps, float rms_eps, hipStream_t s) {
     if (B == 0) return hipSuccess;
-    if (coef_el_n(n)) {
+    if (coef_el_n(n) && (n <= 4 || B <= kCoefElMaxTok)) {
 #define MHC_DCE_FWD(S_, QS_)                                                                                       \
     MHC_LAUNCH_GGL((dyn_coef_el_fwd_kernel<S_, QS_>), dim3((unsigned)((B * S_ * S_ * QS_ + 255) / 256)), dim3(256), 0, \
                        s, p_part, ss_part, ks, B, K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, n,   \
@@ -2523,12 +2533,12 @@ hipError_t launch_dyn_coef_fwd(int n, const float* p_part, const float* ss_part,
 #undef MHC_DCE_FWD
         return hipGetLastError();
     }
-    if (n > 8 && n <= skw16::kN) {
+    if (n > 8 && n <= skw16::kN && B <= (n < skw16::kN ? kCoefElMaxTok : kCoefElMaxTok / 2)) {
         MHC_LAUNCH_GGL(dyn_coef_w16_fwd_kernel, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, p_part, ss_part, ks, B,
                        K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, n, iters, sk_eps, rms_eps);
         return hipGetLastError();
     }
-    if (generic_layer_n(n)) {
+    if (generic_layer_n(n) && !coef_el_n(n)) {
 #define MHC_DCG_FWD(NM_)                                                                                          \
     MHC_LAUNCH_GGL((dyn_coef_gen_fwd_kernel<NM_>), dim3((unsigned)((B * NM_ + 255) / 256)), dim3(256), 0, s,     \
                        p_part, ss_part, ks, B, K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, n,   \
@@ -2542,20 +2552,44 @@ hipError_t launch_dyn_coef_fwd(int n, const float* p_part, const float* ss_part,
                            K, a_pre, a_post, a_res, b_pre, b_post, b_res, coef, p_out, rh, iters, sk_eps, rms_eps);
         return hipGetLastError();
     }
-    if (n != 2) return hipErrorInvalidValue;
     const int64_t threads = B * pow2ceil(n);
     const unsigned blocks = (unsigned)((threads + 255) / 256);
-    MHC_LAUNCH_GGL((dyn_coef_fwd_kernel<2>), dim3(blocks), dim3(256), 0, s, p_part, ss_part, ks, B, K, a_pre, a_post,
-                   a_res, b_pre, b_post, b_res, coef, p_out, rh, iters, sk_eps, rms_eps);
+#define MHC_DC_FWD(N_)                                                                                             \
+    MHC_LAUNCH_GGL((dyn_coef_fwd_kernel<N_>), dim3(blocks), dim3(256), 0, s, p_part, ss_part, ks, B, K, a_pre, a_post, \
+                   a_res, b_pre, b_post, b_res, coef, p_out, rh, iters, sk_eps, rms_eps)
+    switch (n) {
+        case 2: MHC_DC_FWD(2); break;
+        case 5: MHC_DC_FWD(5); break;
+        case 6: MHC_DC_FWD(6); break;
+        case 7: MHC_DC_FWD(7); break;
+        case 8: MHC_DC_FWD(8); break;
+        case 16: MHC_DC_FWD(16); break;
+        default: return hipErrorInvalidValue;
+    }
+#undef MHC_DC_FWD
     return hipGetLastError();
 }
 
+// The backward of n = 5..8 with a row per lane: past kCoefElMaxTok tokens and up
+// to the iterations that its register history holds (n = 8, 10 iterations: 25 us
+// for 35 at 16,384 tokens, 69 for 123 at 65,536).
+static bool coef_bwd_rows_per_lane(int n, int64_t B, int iters, bool res_rows) {
+    return res_rows && n >= 5 && n <= 8 && B > kCoefElMaxTok && iters <= SkHist<8>::TMAX;
+}
+
 // Rows of the db / dalpha partials: one per workgroup, or one per token for
-// n >= 16 and for the generic-n kernel.
-int dyn_coef_bwd_blocks(int n, int64_t B) {
+// n > 8.
+int dyn_coef_bwd_rows(int n, int64_t B, int iters, bool res_rows) {
+    if (coef_bwd_rows_per_lane(n, B, iters, res_rows)) return (int)((B * pow2ceil(n) + 255) / 256);
     if (coef_el_n(n)) return dyn_coef_el_bwd_blocks(n, B);
     if (n >= 16 || generic_layer_n(n)) return (int)(B < 1 ? 1 : B);
     return (int)((B * pow2ceil(n) + 255) / 256);
+}
+
+// The most of them over the iterations.
+int dyn_coef_bwd_blocks(int n, int64_t B) {
+    const int a = dyn_coef_bwd_rows(n, B, 0, true), b = dyn_coef_bwd_rows(n, B, SkHist<8>::TMAX + 1, true);
+    return a > b ? a : b;
 }
 
 // Lane groups (token slots) of the n >= 16 coefficient backward: a whole
@@ -2600,6 +2634,20 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
                                const float* b_res, float* dp_out, float* s_out, float* part, int iters, float sk_eps,
                                float* hist, hipStream_t s, bool res_rows) {
     if (B == 0) return hipSuccess;
+    if (coef_bwd_rows_per_lane(n, B, iters, res_rows)) {
+        const unsigned rblocks = (unsigned)dyn_coef_bwd_rows(n, B, iters, res_rows);
+#define MHC_DCR_BWD(N_)                                                                                             \
+    MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<N_, true>), dim3(rblocks), dim3(256), 0, s, scal, coef, p, rh, B, K, a_pre, \
+                   a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps)
+        switch (n) {
+            case 5: MHC_DCR_BWD(5); break;
+            case 6: MHC_DCR_BWD(6); break;
+            case 7: MHC_DCR_BWD(7); break;
+            default: MHC_DCR_BWD(8); break;
+        }
+#undef MHC_DCR_BWD
+        return hipGetLastError();
+    }
     if (coef_el_n(n)) {
         const unsigned eblocks = (unsigned)dyn_coef_el_bwd_blocks(n, B);
 #define MHC_DCE_BWD(S_, RES_)                                                                                         \
@@ -2613,7 +2661,10 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
 #undef MHC_DCE_BWD
         return hipGetLastError();
     }
-    if (n > 8 && n <= skw16::kN && res_rows && iters <= skw16::kTMax) {
+    // (few iterations of a small matrix past kCoefElMaxTok tokens: n = 9, 10
+    // iterations, 16,384 tokens 88 us for 71 of the row-per-lane form with hist)
+    if (n > 8 && n <= skw16::kN && res_rows && iters <= skw16::kTMax &&
+        (n == skw16::kN || B <= kCoefElMaxTok || n * iters >= 110 || !hist)) {
         MHC_LAUNCH_GGL(dyn_coef_w16_bwd_kernel, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, scal, coef, p, rh, B, K,
                        a_pre, a_post, a_res, b_res, dp_out, s_out, part, n, iters, sk_eps);
         return hipGetLastError();
@@ -2681,7 +2732,7 @@ hipError_t launch_dyn_coef_bwd(int n, const float* scal, const float* coef, cons
         return hipGetLastError();
     }
     if (n != 2) return hipErrorInvalidValue;
-    const unsigned blocks = (unsigned)dyn_coef_bwd_blocks(n, B);
+    const unsigned blocks = (unsigned)dyn_coef_bwd_rows(n, B, iters, res_rows);
     if (res_rows) {
         MHC_LAUNCH_GGL((dyn_coef_bwd_kernel<2, true>), dim3(blocks), dim3(256), 0, s, scal, coef, p, rh, B, K, a_pre,
                            a_post, a_res, b_res, dp_out, s_out, part, iters, sk_eps);

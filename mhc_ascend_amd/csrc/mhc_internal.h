@@ -316,6 +316,8 @@ hipError_t launch_dyn_coef_fwd(int n, const float* p_part, const float* ss_part,
                                const float* a_pre, const float* a_post, const float* a_res, const float* b_pre,
                                const float* b_post, const float* b_res, float* coef, float* p_out, float* rh,
                                int iters, float sk_eps, float rms_eps, hipStream_t s);
+// (dyn_coef_bwd_rows of a call; dyn_coef_bwd_blocks: the most, for the workspace)
+int dyn_coef_bwd_rows(int n, int64_t B, int iters, bool res_rows);
 int dyn_coef_bwd_blocks(int n, int64_t B);
 // n >= 16: the Sinkhorn adjoint's per-iteration history lives in a region
 // of kSkHistBytes (hist; null for n < 16), split into token slots of

@@ -81,3 +81,13 @@ def test_sinkhorn_batches_around_the_forms(device, n, B, iters):
     gref = torch.from_numpy(csk.sinkhorn_bwd(go[idx].double().numpy(), a[idx].double().numpy(), iters, 1e-8))
     assert_close(out.cpu()[idx], ref, 1e-4, 1e-5, f"SK fwd n={n} B={B} T={iters}")
     assert_close(ad.grad.cpu()[idx], gref, 1e-3, max(grad_atol(gref, 1e-5), 1e-6), f"SK bwd n={n} B={B} T={iters}")
+
+
+# one past the tokens up to which the coefficients are spread (4096, half of it
+# at n = 16), on both sides of the 12 iterations of the row form's history and of
+# n iters = 110
+@pytest.mark.parametrize("n,B,iters", [(5, 4097, 12), (6, 4097, 10), (7, 4100, 12), (8, 4097, 12), (8, 4097, 13),
+                                       (9, 4097, 12), (9, 4097, 13), (16, 2049, 10), (12, 4097, 20)])
+def test_dynamic_coefficients_of_many_tokens(device, n, B, iters):
+    d = R.dynamic_layer_inputs(B, n, 32, seed=n + B + iters, x_dtype=torch.float32, alpha=0.1, phi_std=0.02, b_std=0.5)
+    _check_dyn(_run_dyn(d, device, iters=iters), _oracle_dyn(d, iters=iters), torch.float32, f"n={n} B={B} T={iters}")
