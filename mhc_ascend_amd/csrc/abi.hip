@@ -972,21 +972,19 @@ int mhc_layer_dynamic_infer(const void* x, int32_t x_dtype, const void* packed, 
 
 // dx of bf16 x is rounded to bf16 once, from the fp32 sum of the row pass's
 // stream part and the projection's terms, as the reference's fp32 autograd
-// does.  With one 32-row projection tile (n <= 4) on the register-row
+// does.  With one 32-row projection tile at n = 2 and 4 on the register-row
 // kernels and hidden % 128 == 0 the stream part travels as fp16 against a
 // power-of-two scale (11 significant bits; one scale exponent per half wave
 // of the row kernel and token, in the workspace) and the projection kernel
 // rounds the sum: each element's stream part then enters the sum with a
 // relative error of at most 2^-11 (an eighth of the bf16 half-ulp) down to
 // 2^-28 of its group's largest element, and within 2^-39 of that largest
-// element below.  Otherwise (n >= 8, rows the channel-loop kernels take,
-// other hidden sizes) x is upcast once (exactly) and dx accumulates in fp32
-// across the kernels.
-// aligned: rows_aligned() of the call's arrays (without it n = 3 takes the
-// element-wise rows).
-static bool dyn_bwd_f32_acc(int32_t n, int32_t hidden, int32_t x_dtype, bool aligned) {
+// element below.  Otherwise (n = 3, n >= 5, rows the channel-loop kernels take,
+// other hidden sizes) dx accumulates in fp32 across the kernels, which read x
+// itself or an exact fp32 copy of it.
+static bool dyn_bwd_f32_acc(int32_t n, int32_t hidden, int32_t x_dtype) {
     return x_dtype == kBF16 &&
-           (2 * n + n * n > kProjTile || layer_bwd_is_wide(n, hidden) || hidden % 128 != 0 || !aligned);
+           (odd_row_n(n) || 2 * n + n * n > kProjTile || layer_bwd_is_wide(n, hidden) || hidden % 128 != 0);
 }
 
 struct DynBwdWs {
@@ -1001,7 +999,7 @@ static DynBwdWs dyn_bwd_ws(int64_t batch, int32_t n, int32_t hidden, int32_t x_d
     DynBwdWs w{};
     const int64_t np = 2 * n + n * n;
     const int64_t K = (int64_t)n * hidden;
-    w.wdt = dyn_bwd_f32_acc(n, hidden, x_dtype, aligned) ? kF32 : x_dtype;
+    w.wdt = dyn_bwd_f32_acc(n, hidden, x_dtype) ? kF32 : x_dtype;
     w.grid = batch > 0 ? layer_bwd_grid(w.wdt, n, batch, hidden, aligned) : 1;
     w.cblocks = batch > 0 ? dyn_coef_bwd_blocks(n, batch) : 1;
     w.tiles = batch > 0 ? proj_bwd_tiles(w.wdt, batch, (int64_t)n * hidden) : 1;
@@ -1086,10 +1084,12 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
     // (direct: the pass over all output tiles and the row kernel read bf16 x
     // itself, where x and dx take 16-byte pieces and the rows fit registers:
     // n = 8, 4096 x 2048 bf16 583 us of kernels with the fp32 copy of x, 497
-    // without)
-    const bool all_tiles = batch > 0 && w.wdt == kF32 && proj_bwd_tiles_path(2 * n + n * n, batch);
-    const bool direct = all_tiles && (w.wdt == x_dtype || (((uintptr_t)x | (uintptr_t)grad_x) % 16 == 0 &&
-                                                           layer_bwd_f32_dx_ok(n, hidden, aligned)));
+    // without; n = 3 runs that pass for this, one tile)
+    const bool bf16_direct = x_dtype == kBF16 && ((uintptr_t)x | (uintptr_t)grad_x) % 16 == 0 &&
+                             layer_bwd_f32_dx_ok(n, hidden, aligned);
+    const bool all_tiles = batch > 0 && w.wdt == kF32 &&
+                           (proj_bwd_tiles_path(2 * n + n * n, batch) || (n == 3 && bf16_direct));
+    const bool direct = all_tiles && (w.wdt == x_dtype || bf16_direct);
     const void* xk = w.wdt != x_dtype && !direct ? (const void*)xw : x;
     void* dxk = w.wdt != x_dtype ? (void*)dxw : grad_x;
     const DynSaved d = dyn_saved(batch, n, hidden);
@@ -1105,8 +1105,9 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
     } else {
         if (w.wdt != x_dtype && !direct) e = launch_weight_f32(x, x_dtype, batch * K, xw, s);
         if (e == hipSuccess)
-            e = launch_layer_bwd(direct ? x_dtype : w.wdt, n, direct && x_dtype == kBF16 ? 2 : 1, grad_out, xk, w32, saved + d.coef_off, np, dxk, dw_part, scal, w.grid,
-                                 batch, hidden, rmsnorm_eps, (float*)(ws + w.rows_off), s, pscale, aligned);
+            e = launch_layer_bwd(direct ? x_dtype : w.wdt, n, direct && x_dtype == kBF16 ? 2 : 1, grad_out, xk, w32,
+                                 saved + d.coef_off, np, dxk, dw_part, scal, w.grid, batch, hidden, rmsnorm_eps,
+                                 (float*)(ws + w.rows_off), s, pscale, aligned);
         if (e == hipSuccess)
             e = launch_dyn_coef_bwd(n, scal, saved + d.coef_off, saved + d.p_off, saved + d.rh_off, batch, K,
                                     alpha_pre, alpha_post, alpha_res, b_res, dp, stok, cpart, num_iters, sinkhorn_eps,
@@ -1118,10 +1119,13 @@ int mhc_layer_dynamic_bwd(const float* grad_out, const void* x, int32_t x_dtype,
     const bool one_sum = batch > 0 && np <= kProjTile && !proj_bwd_wide_path(w.wdt, np, batch) &&
                          column_sums_direct(rows_p) && column_sums_direct(rows_w) && column_sums_direct(rows_c);
     if (one_sum) {
-        if (e == hipSuccess)
+        if (e == hipSuccess && all_tiles)
+            e = launch_proj_bwd_tiles(x_dtype, x, dp, dp_stride(np), stok, phi_pre, phi_post, phi_res, n, np,
+                                      (const float*)dxk, grad_x, phip, rows_p, batch, K, s);
+        else if (e == hipSuccess)
             e = launch_proj_bwd(w.wdt, xk, dp, dp_stride(np), stok, phi_pre, phi_post, phi_res, n, 0, np, dxk, true,
                                 phip, rows_p, batch, K, s, pscale, w.groups);
-        if (e == hipSuccess && w.wdt != x_dtype) e = launch_cast_bf16(dxw, batch * K, grad_x, s);
+        if (e == hipSuccess && w.wdt != x_dtype && !direct) e = launch_cast_bf16(dxw, batch * K, grad_x, s);
         if (e == hipSuccess) {
             ColSumJobs jobs{};
             jobs.j[0] = ColSumJob{phip, grad_phi, nullptr, (int64_t)np * K, rows_p, (int)(np * K), 0, 0, 0};

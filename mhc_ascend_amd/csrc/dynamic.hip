@@ -1994,7 +1994,7 @@ __global__ __launch_bounds__(64 * kPbNW<TX>()) __attribute__((amdgpu_waves_per_e
 
 // ---------------------------------------------------------------------------
 // The projection backward over OT = 2 or 3 output tiles at once (33..96 rows:
-// n = 5..8, past the tokens of the small-np kernels): proj_bwd_mfma_kernel's
+// n = 5..8, past the tokens of the small-np kernels; OT = 1: bf16 x of n = 3): proj_bwd_mfma_kernel's
 // stages with every tile's dP in LDS and its Phi^T fragments and dPhi sums in
 // registers, so x and the stream part are read once and dx is written once, in
 // x's type (TX; the stream part dx_in is fp32).  Bound by its bytes, 6 B read
@@ -3486,7 +3486,7 @@ hipError_t launch_proj_bwd_tiles(int x_dtype, const void* x, const float* dP, in
                                  const float* phi_pre, const float* phi_post, const float* phi_res, int n_pre, int np,
                                  const float* dx_in, void* dx, float* dphi_part, int tiles, int64_t B, int64_t K,
                                  hipStream_t s) {
-    if (!proj_bwd_tiles_path(np, B) || K % 32 != 0 || tiles < 1 || !s_tok) return hipErrorInvalidValue;
+    if (np < 1 || np > 3 * kProjTile || K % 32 != 0 || tiles < 1 || !s_tok) return hipErrorInvalidValue;
     int64_t tile = (B + tiles - 1) / tiles;
     tile = ((tile + 63) / 64) * 64;
     if (tile > proj_bwd_max_tile(kF32, K)) return hipErrorInvalidValue;
@@ -3496,7 +3496,9 @@ hipError_t launch_proj_bwd_tiles(int x_dtype, const void* x, const float* dP, in
     MHC_LAUNCH_GGL((proj_bwd_tiles_kernel<TX_, OT_>), grid, dim3(256), 0, s, (const TX_*)x, dP, dp_stride, s_tok,    \
                    phi_pre, phi_post, phi_res, n_pre, np, dx_in, (TX_*)dx, dphi_part, B, K, tile)
     if (x_dtype == kBF16) {
-        if (np <= 2 * kProjTile) {
+        if (np <= kProjTile) {
+            MHC_PBT(bf16_t, 1);
+        } else if (np <= 2 * kProjTile) {
             MHC_PBT(bf16_t, 2);
         } else {
             MHC_PBT(bf16_t, 3);

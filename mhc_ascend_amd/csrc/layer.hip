@@ -1003,11 +1003,12 @@ static const void* pick_bwd(int x_dtype, int n, int vpt, int mode, bool pf) {
     return fn;
 }
 
-// mode 2: bf16 x, fp32 dx (n = 5..8, whose projection backward adds to it)
+// mode 2: bf16 x, fp32 dx (n = 3, 5..8, whose projection backward adds to it)
 static const void* pick_bwd_f32_dx(int n, int vpt, bool pf) {
     const void* fn = nullptr;
 #define MHC_BWD_FN2(N_) MHC_PICK_VPT(vpt, fn = pf ? bwd_fn<bf16_t, N_, V_, 2, true>() : bwd_fn<bf16_t, N_, V_, 2, false>())
     switch (n) {
+        case 3: { MHC_BWD_FN2(3); break; }
         case 5: { MHC_BWD_FN2(5); break; }
         case 6: { MHC_BWD_FN2(6); break; }
         case 7: { MHC_BWD_FN2(7); break; }
@@ -1155,7 +1156,7 @@ static RowTiling bwd_tiling(int64_t C, int n, int64_t B = 0) {
 bool layer_bwd_is_wide(int n, int64_t C) { return bwd_tiling(C, n).vpt <= 0; }
 
 bool layer_bwd_f32_dx_ok(int n, int64_t C, bool aligned) {
-    return n >= 5 && n <= 8 && row_path(bwd_tiling(C, n), n, C, aligned) == RowPath::kRegs;
+    return (n == 3 || (n >= 5 && n <= 8)) && row_path(bwd_tiling(C, n), n, C, aligned) == RowPath::kRegs;
 }
 
 int layer_bwd_part_groups(int x_dtype, int n, int64_t C) {

@@ -385,8 +385,8 @@ hipError_t launch_proj_bwd_wide(const float* x, const float* dP, int dp_stride, 
                                 const float* phi_pre, const float* phi_post, const float* phi_res, int n_pre, int np,
                                 float* dx, bool accumulate, float* dphi, void* scratch, int64_t B, int64_t K,
                                 hipStream_t s);
-// 33..96 projection rows past the wide path's tokens (proj_bwd_tiles_path), all
-// rows in one pass: dx = dx_in (fp32) + s x + dP . Phi in x's type (fp32: dx_in
+// 33..96 projection rows past the wide path's tokens (proj_bwd_tiles_path), and
+// the 15 of n = 3 with bf16 x, all rows in one pass: dx = dx_in (fp32) + s x + dP . Phi in x's type (fp32: dx_in
 // may be dx), dphi_part[tiles][np][K]; 16-byte aligned x and dx.
 bool proj_bwd_tiles_path(int np, int64_t B);
 hipError_t launch_proj_bwd_tiles(int x_dtype, const void* x, const float* dP, int dp_stride, const float* s_tok,
