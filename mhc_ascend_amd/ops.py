@@ -1,7 +1,8 @@
 """Autograd functions over the HIP kernels (mirror of src/python/mhc/ops.py).
 
 The autograd nodes of the layers, the wrapper and the stand-alone operators
-are C++ (csrc/autograd.cpp); the projection's is the one Python Function.
+are C++ (csrc/autograd.cpp); the projection's is a Python Function, and so are
+the operators' where a Python one is needed (_NodeFunction).
 
 Public functional ops keep the reference's names, arguments and defaults.
 Documented differences from the Ascend implementation (all toward the
@@ -27,15 +28,41 @@ from . import _lib, native
 _STREAM_PROJ_ROWS = 128
 
 
+class _NodeFunction(torch.autograd.Function):
+    """A stand-alone operator's autograd function.  ``apply`` runs its C++ node;
+    under ``torch.jit.trace``, which records Python functions only, and for
+    subclasses it runs ``forward`` / ``backward``, over the same entries."""
+
+    @classmethod
+    def apply(cls, *args):
+        if "node" not in vars(cls) or torch.jit.is_tracing():
+            return super().apply(*args)
+        return cls.node(*args)
+
+
 # =============================================================================
 # Sinkhorn-Knopp (ops.py:32-80)
 # =============================================================================
 
-class SinkhornKnoppFunction:
+class SinkhornKnoppFunction(_NodeFunction):
     """Sinkhorn-Knopp doubly stochastic normalisation of [B, n, n]."""
 
     @staticmethod
-    def apply(inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) -> torch.Tensor:
+    def forward(ctx, inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) -> torch.Tensor:
+        out = native.sinkhorn_knopp_fwd(inp, num_iters, eps)
+        ctx.save_for_backward(inp, out)
+        ctx.num_iters = num_iters
+        ctx.eps = eps
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out: torch.Tensor):
+        inp, out = ctx.saved_tensors
+        grad_inp = native.sinkhorn_knopp_bwd(grad_out.float().contiguous(), inp, out, ctx.num_iters, ctx.eps)
+        return grad_inp, None, None
+
+    @staticmethod
+    def node(inp, num_iters=20, eps=1e-8):
         return _lib.autograd().sinkhorn_knopp(inp, int(num_iters), float(eps))
 
 
@@ -48,11 +75,24 @@ def sinkhorn_knopp(inp: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) ->
 # RMSNorm (ops.py:87-136)
 # =============================================================================
 
-class RMSNormFunction:
+class RMSNormFunction(_NodeFunction):
     """Root Mean Square normalisation of [B, C] rows."""
 
     @staticmethod
-    def apply(inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
+    def forward(ctx, inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
+        out, rms = native.rmsnorm_fwd(inp, weight, eps)
+        ctx.save_for_backward(inp, weight, rms)
+        ctx.eps = eps
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out: torch.Tensor):
+        inp, weight, rms = ctx.saved_tensors
+        grad_inp, grad_weight = native.rmsnorm_bwd(grad_out, inp, weight, rms)
+        return grad_inp.to(inp.dtype), grad_weight, None
+
+    @staticmethod
+    def node(inp, weight, eps=1e-5):
         return _lib.autograd().rmsnorm(inp, weight, float(eps))
 
 
@@ -65,11 +105,23 @@ def rmsnorm(inp: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch
 # Stream aggregate (ops.py:143-188)
 # =============================================================================
 
-class StreamAggregateFunction:
+class StreamAggregateFunction(_NodeFunction):
     """out = sum_i sigmoid(H_pre_raw[:, i]) * inp[:, i]."""
 
     @staticmethod
-    def apply(inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor:
+    def forward(ctx, inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor:
+        out, h_act = native.stream_aggregate_fwd(inp, H_pre_raw)
+        ctx.save_for_backward(inp, h_act)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out: torch.Tensor):
+        inp, h_act = ctx.saved_tensors
+        gx, _, graw = native._aggregate_bwd(grad_out, inp, h_act, True)
+        return gx.to(inp.dtype), graw
+
+    @staticmethod
+    def node(inp, H_pre_raw):
         return _lib.autograd().stream_aggregate(inp, H_pre_raw)
 
 
@@ -82,11 +134,23 @@ def stream_aggregate(inp: torch.Tensor, H_pre_raw: torch.Tensor) -> torch.Tensor
 # Stream distribute-mix-add (ops.py:195-265)
 # =============================================================================
 
-class StreamDistributeMixAddFunction:
+class StreamDistributeMixAddFunction(_NodeFunction):
     """out[:, i] = 2 sigmoid(H_post_raw[:, i]) * y_norm + sum_j M[:, i, j] x[:, j]."""
 
     @staticmethod
-    def apply(y_norm: torch.Tensor, H_post_raw: torch.Tensor, M: torch.Tensor, x_inp: torch.Tensor) -> torch.Tensor:
+    def forward(ctx, y_norm, H_post_raw, M, x_inp):
+        out, h_act = native.stream_distribute_mix_add_fwd(y_norm, H_post_raw, M, x_inp)
+        ctx.save_for_backward(x_inp, y_norm, M, h_act)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        x_inp, y_norm, M, h_act = ctx.saved_tensors
+        gx, gy, gM, _, graw = native._distribute_bwd(grad_out, x_inp, y_norm, M, h_act, True)
+        return gy.to(y_norm.dtype), graw, gM, gx.to(x_inp.dtype)
+
+    @staticmethod
+    def node(y_norm, H_post_raw, M, x_inp):
         return _lib.autograd().stream_distribute_mix_add(y_norm, H_post_raw, M, x_inp)
 
 
