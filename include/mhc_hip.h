@@ -330,6 +330,11 @@ size_t mhc_wrapper_dynamic_fwd_workspace_size(int64_t tokens, int32_t n, int32_t
  * streams inside its projection and keeps no stream rows.  No counterpart
  * in the reference; for callers that size the workspace per call. */
 size_t mhc_wrapper_dynamic_fwd_workspace_size_for(int64_t tokens, int32_t n, int32_t hidden, int32_t dtype);
+/* What a forward on these rows needs, at most the query above: no share that
+ * only other shapes or unaligned rows use.  No counterpart in the reference;
+ * the backward's (below) likewise. */
+size_t mhc_wrapper_dynamic_fwd_workspace_need(const void* residual, const void* branch, int32_t dtype, int64_t tokens,
+                                              int32_t n, int32_t hidden);
 int mhc_wrapper_dynamic_fwd(const void* residual, const void* branch, int32_t dtype, int32_t residual_mode,
                             const void* weight, int32_t weight_dtype, const float* phi_pre, const float* phi_post,
                             const float* phi_res, const float* alpha_pre, const float* alpha_post,
@@ -347,6 +352,10 @@ size_t mhc_wrapper_dynamic_bwd_workspace_size(int64_t tokens, int32_t n, int32_t
  * workspace per call. */
 size_t mhc_wrapper_dynamic_bwd_workspace_size_for(int64_t tokens, int32_t n, int32_t hidden, int32_t dtype,
                                                   int32_t residual_mode, int32_t num_iters, float sinkhorn_eps);
+size_t mhc_wrapper_dynamic_bwd_workspace_need(const float* grad_out, const void* residual, const void* branch,
+                                              const void* grad_residual, const void* grad_branch, int32_t dtype,
+                                              int32_t residual_mode, int64_t tokens, int32_t n, int32_t hidden,
+                                              int32_t num_iters, float sinkhorn_eps);
 int mhc_wrapper_dynamic_bwd(const float* grad_out, const void* residual, const void* branch, int32_t dtype,
                             int32_t residual_mode, int32_t weight_dtype, const float* phi_pre, const float* phi_post,
                             const float* phi_res, const float* alpha_pre, const float* alpha_post,

@@ -1411,17 +1411,21 @@ static WfoldWs wfold_ws(int32_t dtype, int64_t tokens, int32_t n, int32_t hidden
     return w;
 }
 
-static size_t wgen_fwd_need(const WgenFwdWs& w, int32_t dtype, int32_t n, int32_t hidden, int64_t tokens) {
-    if (wfold_ok(n, hidden)) return wfold_ws(dtype, tokens, n, hidden).total;
-    return w.x_off + align256((size_t)tokens * n * hidden * dtype_size(dtype));
+// What a call needs: the copies only for rows that are not 16-byte aligned.
+static size_t wgen_fwd_need(int32_t dtype, int32_t n, int32_t hidden, int64_t tokens, bool aligned) {
+    if (wfold_ok(n, hidden)) {
+        const WfoldWs f = wfold_ws(dtype, tokens, n, hidden);
+        return aligned ? f.copy_off : f.total;
+    }
+    return wgen_fwd_ws(tokens, n, hidden).x_off + align256((size_t)tokens * n * hidden * dtype_size(dtype));
 }
 
 // The size queries' answer.  They keep the relation that callers dividing one
 // buffer between storage types count on: fp32 rows, and bf16 rows that the
 // streaming projection could not rebuild (up to 32 projection rows, fewer than
 // 1024 tokens, hidden % 64 != 0), reserve the stream rows in their own dtype.
-static size_t wgen_fwd_size(const WgenFwdWs& w, int32_t dtype, int32_t n, int32_t hidden, int64_t tokens) {
-    const size_t need = wgen_fwd_need(w, dtype, n, hidden, tokens);
+static size_t wgen_fwd_size(int32_t dtype, int32_t n, int32_t hidden, int64_t tokens) {
+    const size_t need = wgen_fwd_need(dtype, n, hidden, tokens, false);
     if (!wfold_ok(n, hidden) || (proj_one_pass(dtype, 2 * n + n * n, tokens) && hidden % 64 == 0)) return need;
     return need + align256((size_t)tokens * n * hidden * dtype_size(dtype));
 }
@@ -1507,8 +1511,21 @@ static WgenBwdWs wgen_bwd_ws(int64_t tokens, int32_t n, int32_t hidden, bool dyn
 // The run-time-n backward keeps the stream rows X and dX (the last regions
 // of its workspace) only when the H_res rows of dP do not vanish or the
 // shape is not one for the fold kernels.
-static size_t wgen_bwd_need(const WgenBwdWs& w, int32_t n, int32_t hidden, int32_t num_iters, float sinkhorn_eps) {
-    return wgen_fold_ok(n, hidden) && wrap_res_grad_vanishes(num_iters, sinkhorn_eps) ? w.x_off : w.total;
+static size_t wgen_bwd_need(const WgenBwdWs& w, int32_t n, int32_t hidden, int32_t num_iters, float sinkhorn_eps,
+                            bool one) {
+    return one || (wgen_fold_ok(n, hidden) && wrap_res_grad_vanishes(num_iters, sinkhorn_eps)) ? w.x_off : w.total;
+}
+
+// wbwd_kernel takes whole 16-byte pieces of aligned rows; bf16 'decay' past
+// n = 8, C % 8 != 0 and unaligned rows keep the kernels of wrapper_gen.hip.  dPhi,
+// d r and d b at n = 8 (65,536 x 7168 bf16): 1.30 ms against 3.2; fp32 n = 16 (4096
+// x 2048): 50 us against 905
+static bool wgen_bwd_one(int32_t dtype, int32_t n, bool decay, int32_t hidden, int64_t tokens, int32_t num_iters,
+                         float sinkhorn_eps, std::initializer_list<const void*> rows) {
+    uintptr_t a = 0;
+    for (const void* p : rows) a |= (uintptr_t)p;
+    return tokens > 0 && wrap_res_grad_vanishes(num_iters, sinkhorn_eps) && a % 16 == 0 &&
+           wbwd_shape_ok(dtype, n, decay, hidden);
 }
 
 static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dtype, bool decay, const void* weight,
@@ -1523,22 +1540,19 @@ static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dt
     // the weight's fp32 copy: its own launch, or inside the folded pack's
     hipError_t e = wfold ? hipSuccess : launch_weight_f32(weight, weight_dtype, hidden, w32, s);
     if (e != hipSuccess || tokens == 0) return hip_status(e);
-    const WgenFwdWs w = wgen_fwd_ws(tokens, n, hidden);
-    if (!workspace || workspace_bytes < wgen_fwd_need(w, dtype, n, hidden, tokens))
+    const bool rows16 = ((uintptr_t)residual | (uintptr_t)branch) % 16 == 0;
+    if (!workspace || workspace_bytes < wgen_fwd_need(dtype, n, hidden, tokens, rows16))
         return fail(MHC_ERR_WORKSPACE,
                     "wrapper_dynamic_fwd: workspace smaller than mhc_wrapper_dynamic_fwd_workspace_size_for()");
     const int64_t K = (int64_t)n * hidden;
     const int np = 2 * n + n * n;
     char* pw = (char*)workspace;
-    void* X = (char*)workspace + w.x_off;
-    float* pp = (float*)(pw + w.p.p_off);
-    float* ss = (float*)(pw + w.p.ss_off);
-    bf16_raw_t* phib = (bf16_raw_t*)(pw + w.p.phib_off);
-    int ks = w.p.ks;
+    float *pp = nullptr, *ss = nullptr;
+    int ks = 1;
     if (wfold) {
         const WfoldWs f = wfold_ws(dtype, tokens, n, hidden);
         const void *pres = residual, *pbr = branch;
-        if ((uintptr_t)residual % 16 != 0 || (uintptr_t)branch % 16 != 0) {
+        if (!rows16) {
             char* c = pw + f.copy_off;
             char* c2 = c + align256((size_t)tokens * hidden * dtype_size(dtype));
             e = launch_wfold_copy(dtype, residual, c, branch, c2, tokens * hidden, s);
@@ -1552,6 +1566,12 @@ static int wgen_dynamic_fwd(const void* residual, const void* branch, int32_t dt
             e = launch_wfold_proj(dtype, n, decay, pres, pbr, phi_pre, phi_post, phi_res, weight, weight_dtype, w32, pw,
                                   pp, ss, tokens, hidden, ks, s);
     } else {
+        const WgenFwdWs w = wgen_fwd_ws(tokens, n, hidden);
+        void* X = pw + w.x_off;
+        bf16_raw_t* phib = (bf16_raw_t*)(pw + w.p.phib_off);
+        pp = (float*)(pw + w.p.p_off);
+        ss = (float*)(pw + w.p.ss_off);
+        ks = w.p.ks;
         e = launch_wgen_synth(dtype, dtype, n, decay, residual, branch, X, tokens, hidden, s);
         if (e == hipSuccess && w.p.stream) {
             e = launch_proj_stream(dtype, X, (bf16_raw_t*)(pw + w.p.xpl_off), phi_pre, phi_post, phi_res, n, nullptr,
@@ -1590,7 +1610,9 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
                                              " the fused wrapper needs num_iters >= 1 and sinkhorn_eps <= 1e-6 "
                                              "(the H_res gradients then vanish)");
     const WgenBwdWs w = wgen_bwd_ws(tokens, n, hidden, true);
-    if (!workspace || workspace_bytes < wgen_bwd_need(w, n, hidden, num_iters, sinkhorn_eps))
+    const bool one = wgen_bwd_one(dtype, n, decay, hidden, tokens, num_iters, sinkhorn_eps,
+                                  {grad_out, residual, branch, grad_residual, grad_branch});
+    if (!workspace || workspace_bytes < wgen_bwd_need(w, n, hidden, num_iters, sinkhorn_eps, one))
         return fail(MHC_ERR_WORKSPACE,
                     "wrapper_dynamic_bwd: workspace smaller than mhc_wrapper_dynamic_bwd_workspace_size_for()");
     char* ws = (char*)workspace;
@@ -1610,13 +1632,6 @@ static int wgen_dynamic_bwd(const float* grad_out, const void* residual, const v
     const int64_t K = (int64_t)n * hidden;
     // the fold kernels' shapes carry the pre / post rows without stream rows
     const bool fold = rows < np && wgen_fold_ok(n, hidden);
-    // wbwd_kernel takes whole 16-byte pieces of aligned rows; bf16 'decay' past
-    // n = 8, C % 8 != 0 and unaligned rows keep the kernels below.  dPhi, d r and
-    // d b at n = 8 (65,536 x 7168 bf16): 1.30 ms against 3.2; fp32 n = 16 (4096 x
-    // 2048): 50 us against 905
-    const bool one = tokens > 0 && rows < np && wbwd_shape_ok(dtype, n, decay, hidden) &&
-                     ((uintptr_t)grad_out | (uintptr_t)residual | (uintptr_t)branch | (uintptr_t)grad_residual |
-                      (uintptr_t)grad_branch) % 16 == 0;
     hipError_t e = hipSuccess;
     int rows_w = fold ? w.ftiles : w.dtiles, rows_c = dyn_coef_bwd_rows(n, tokens, num_iters, rows == np);
     if (tokens == 0) {
@@ -1756,8 +1771,7 @@ static WrapFwdWs wrap_fwd_ws(int64_t tokens, int32_t n, int32_t hidden) {
 size_t mhc_wrapper_dynamic_fwd_workspace_size(int64_t tokens, int32_t n, int32_t hidden) {
     if (tokens < 0 || n < 1 || hidden < 1) return 0;
     if (!wrap_fused4(n, hidden, true)) {
-        const WgenFwdWs w = wgen_fwd_ws(tokens, n, hidden);
-        const size_t a = wgen_fwd_size(w, kF32, n, hidden, tokens), b = wgen_fwd_size(w, kBF16, n, hidden, tokens);
+        const size_t a = wgen_fwd_size(kF32, n, hidden, tokens), b = wgen_fwd_size(kBF16, n, hidden, tokens);
         return a > b ? a : b;
     }
     return wrap_fwd_ws(tokens, n, hidden).total;
@@ -1766,7 +1780,15 @@ size_t mhc_wrapper_dynamic_fwd_workspace_size(int64_t tokens, int32_t n, int32_t
 size_t mhc_wrapper_dynamic_fwd_workspace_size_for(int64_t tokens, int32_t n, int32_t hidden, int32_t dtype) {
     if (tokens < 0 || n < 1 || hidden < 1 || !valid_dtype(dtype)) return 0;
     if (!wrap_fused4(n, hidden, true))
-        return wgen_fwd_size(wgen_fwd_ws(tokens, n, hidden), dtype, n, hidden, tokens);
+        return wgen_fwd_size(dtype, n, hidden, tokens);
+    return wrap_fwd_ws(tokens, n, hidden).total;
+}
+
+size_t mhc_wrapper_dynamic_fwd_workspace_need(const void* residual, const void* branch, int32_t dtype, int64_t tokens,
+                                              int32_t n, int32_t hidden) {
+    if (tokens < 0 || n < 1 || hidden < 1 || !valid_dtype(dtype)) return 0;
+    if (!wrap_fused4(n, hidden, true))
+        return wgen_fwd_need(dtype, n, hidden, tokens, ((uintptr_t)residual | (uintptr_t)branch) % 16 == 0);
     return wrap_fwd_ws(tokens, n, hidden).total;
 }
 
@@ -1882,7 +1904,19 @@ size_t mhc_wrapper_dynamic_bwd_workspace_size_for(int64_t tokens, int32_t n, int
                                                   int32_t residual_mode, int32_t num_iters, float sinkhorn_eps) {
     if (tokens < 0 || n < 1 || hidden < 1) return 0;
     if (!wrap_fused4(n, hidden, true))
-        return wgen_bwd_need(wgen_bwd_ws(tokens, n, hidden, true), n, hidden, num_iters, sinkhorn_eps);
+        return wgen_bwd_need(wgen_bwd_ws(tokens, n, hidden, true), n, hidden, num_iters, sinkhorn_eps, false);
+    return wrap_bwd_ws(tokens, n, hidden, dtype, true, residual_mode == MHC_WRAPPER_DECAY).total;
+}
+
+size_t mhc_wrapper_dynamic_bwd_workspace_need(const float* grad_out, const void* residual, const void* branch,
+                                              const void* grad_residual, const void* grad_branch, int32_t dtype,
+                                              int32_t residual_mode, int64_t tokens, int32_t n, int32_t hidden,
+                                              int32_t num_iters, float sinkhorn_eps) {
+    if (tokens < 0 || n < 1 || hidden < 1) return 0;
+    if (!wrap_fused4(n, hidden, true))
+        return wgen_bwd_need(wgen_bwd_ws(tokens, n, hidden, true), n, hidden, num_iters, sinkhorn_eps,
+                             wgen_bwd_one(dtype, n, residual_mode == MHC_WRAPPER_DECAY, hidden, tokens, num_iters,
+                                          sinkhorn_eps, {grad_out, residual, branch, grad_residual, grad_branch}));
     return wrap_bwd_ws(tokens, n, hidden, dtype, true, residual_mode == MHC_WRAPPER_DECAY).total;
 }
 

@@ -57,9 +57,9 @@ using torch::autograd::tensor_list;
     X(mhc_stream_distribute_mix_add_fwd)      \
     X(mhc_stream_distribute_mix_add_bwd)      \
     X(mhc_wrapper_dynamic_saved_size)         \
-    X(mhc_wrapper_dynamic_fwd_workspace_size_for) \
+    X(mhc_wrapper_dynamic_fwd_workspace_need) \
     X(mhc_wrapper_dynamic_fwd)                \
-    X(mhc_wrapper_dynamic_bwd_workspace_size_for) \
+    X(mhc_wrapper_dynamic_bwd_workspace_need) \
     X(mhc_wrapper_dynamic_bwd)                \
     X(mhc_wrapper_static_fwd)                 \
     X(mhc_wrapper_static_bwd_workspace_size)  \
@@ -418,8 +418,8 @@ struct DynamicWrapper : public torch::autograd::Function<DynamicWrapper> {
         Tensor out = at::empty({T, C}, f32);
         Tensor saved =
             at::empty({(int64_t)(lib.mhc_wrapper_dynamic_saved_size(T, (int32_t)n, (int32_t)C) / 4)}, f32);
-        const size_t wsb = lib.mhc_wrapper_dynamic_fwd_workspace_size_for(T, (int32_t)n, (int32_t)C,
-                                                                          dtype_code(r.scalar_type()));
+        const size_t wsb = lib.mhc_wrapper_dynamic_fwd_workspace_need(
+            r.data_ptr(), b.data_ptr(), dtype_code(r.scalar_type()), T, (int32_t)n, (int32_t)C);
         Tensor ws = workspace(wsb, r);
         check(lib.mhc_wrapper_dynamic_fwd(r.data_ptr(), b.data_ptr(), dtype_code(r.scalar_type()), (int32_t)mode,
                                           w.data_ptr(), dtype_code(w.scalar_type()), fp(ph[0]), fp(ph[1]), fp(ph[2]),
@@ -454,8 +454,9 @@ struct DynamicWrapper : public torch::autograd::Function<DynamicWrapper> {
         Tensor galpha = at::empty({3}, f32);
         Tensor gbias = at::empty({np}, f32);
         const int dt = dtype_code(r.scalar_type());
-        const size_t wsb = lib.mhc_wrapper_dynamic_bwd_workspace_size_for(T, (int32_t)n, (int32_t)C, dt, mode,
-                                                                          (int32_t)cfg[2], (float)cfg[3]);
+        const size_t wsb = lib.mhc_wrapper_dynamic_bwd_workspace_need(
+            fp(g), r.data_ptr(), b.data_ptr(), gr.data_ptr(), gb.data_ptr(), dt, mode, T, (int32_t)n, (int32_t)C,
+            (int32_t)cfg[2], (float)cfg[3]);
         Tensor ws = workspace(wsb, r);
         check(lib.mhc_wrapper_dynamic_bwd(fp(g), r.data_ptr(), b.data_ptr(), dt, mode, dtype_code(w.scalar_type()),
                                           fp(sv[4]), fp(sv[5]), fp(sv[6]), fp(sv[7]), fp(sv[8]), fp(sv[9]),

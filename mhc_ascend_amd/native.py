@@ -678,7 +678,7 @@ def wrapper_dynamic_fwd(residual: torch.Tensor, branch: torch.Tensor, residual_m
     lib = _lib.load()
     saved = torch.empty((lib.mhc_wrapper_dynamic_saved_size(T, n, C) // 4,), dtype=torch.float32, device=dev)
     with _lib.on_device(dev):
-        wsb = lib.mhc_wrapper_dynamic_fwd_workspace_size_for(T, n, C, dtype_code(r.dtype))
+        wsb = lib.mhc_wrapper_dynamic_fwd_workspace_need(ptr(r), ptr(b), dtype_code(r.dtype), T, n, C)
         ws = _ws(dev, wsb)
         call("mhc_wrapper_dynamic_fwd", ptr(r), ptr(b), dtype_code(r.dtype), mode, ptr(w), dtype_code(w.dtype),
              ptr(pp), ptr(pq), ptr(pr), ptr(a[0]), ptr(a[1]), ptr(a[2]), ptr(bp), ptr(bq), ptr(br), ptr(out),
@@ -712,8 +712,9 @@ def wrapper_dynamic_bwd(grad_out: torch.Tensor, residual: torch.Tensor, branch: 
     galpha = torch.empty((3,), dtype=torch.float32, device=dev)
     gbias = torch.empty((np_,), dtype=torch.float32, device=dev)
     with _lib.on_device(dev):
-        wsb = _lib.load().mhc_wrapper_dynamic_bwd_workspace_size_for(T, n, C, dtype_code(r.dtype), mode,
-                                                                     int(sinkhorn_iters), float(sinkhorn_eps))
+        wsb = _lib.load().mhc_wrapper_dynamic_bwd_workspace_need(ptr(g), ptr(r), ptr(b), ptr(gr), ptr(gb),
+                                                                 dtype_code(r.dtype), mode, T, n, C,
+                                                                 int(sinkhorn_iters), float(sinkhorn_eps))
         ws = _ws(dev, wsb)
         call("mhc_wrapper_dynamic_bwd", ptr(g), ptr(r), ptr(b), dtype_code(r.dtype), mode, dtype_code(wdt), ptr(pp),
              ptr(pq), ptr(pr), ptr(a[0]), ptr(a[1]), ptr(a[2]), ptr(br), ptr(saved), ptr(gr), ptr(gb), ptr(gw),

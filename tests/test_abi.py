@@ -171,6 +171,35 @@ def test_wrapper_forward_workspace_for_dtype_on_host():
     assert lib.mhc_wrapper_dynamic_fwd_workspace_size_for(4096, 4, 4096, 1) == full
 
 
+def test_wrapper_workspace_need_on_host():
+    """What a wrapper call on given rows needs: no stream rows on hidden % 8 == 0,
+    copies of residual and branch only for rows that are not 16-byte aligned, X and
+    dX only where no kernel rebuilds the streams, never more than the size
+    queries; one byte less is refused before any launch."""
+    lib = _lib.load()
+    fwd, bwd = lib.mhc_wrapper_dynamic_fwd_workspace_need, lib.mhc_wrapper_dynamic_bwd_workspace_need
+    for n, C, T in ((8, 7168, 65536), (5, 1024, 300), (3, 96, 4096), (12, 512, 2000), (32, 1024, 700)):
+        for dt, size in ((0, 4), (1, 2)):
+            full = lib.mhc_wrapper_dynamic_fwd_workspace_size_for(T, n, C, dt)
+            need, shifted = fwd(64, 128, dt, T, n, C), fwd(64, 130, dt, T, n, C)
+            assert shifted - need >= 2 * T * C * size and shifted <= full, (n, C, T, dt)
+            if dt == 0:
+                assert full - need >= (n + 2) * T * C * size, (n, C, T)
+            for mode in (0, 1):
+                full = lib.mhc_wrapper_dynamic_bwd_workspace_size_for(T, n, C, dt, mode, 20, 1e-8)
+                need = bwd(64, 64, 64, 64, 64, dt, mode, T, n, C, 20, 1e-8)
+                other = bwd(64, 64, 64, 68, 64, dt, mode, T, n, C, 20, 1e-8)
+                assert need <= other <= full, (n, C, T, dt, mode)
+                if n > 8 and C < 2048 and (dt == 0 or mode == 1):
+                    assert other - need >= 8 * n * C * T, (n, C, T, dt, mode)
+                assert bwd(64, 64, 64, 64, 64, dt, mode, T, n, C, 20, 0.1) == \
+                    lib.mhc_wrapper_dynamic_bwd_workspace_size_for(T, n, C, dt, mode, 20, 0.1)
+    need = fwd(64, 128, 0, 300, 5, 1024)
+    rc = lib.mhc_wrapper_dynamic_fwd(64, 128, 0, 0, 64, 0, 64, 64, 64, 64, 64, 64, 64, 64, 64, 64, 64, 64, need - 1,
+                                     300, 5, 1024, 20, 1e-8, 1e-5, None)
+    assert rc == -3, lib.mhc_last_error()
+
+
 def test_cpu_tensors_raise_no_fallback():
     import mhc_ascend_amd as mhc
     x = torch.rand(2, 4, 4)
