@@ -148,24 +148,21 @@ __global__ __launch_bounds__(256) void wfold_pack_kernel(const float* __restrict
             if (ok) load_run<float, 8>(row + (int64_t)j * C, d);
         };
         ld(0, vr);
-        if (decay) {
-            float m = 1.f;
-            double md = 1.0;
-            for (int j = 2; j < n; ++j) {
-                md *= 0.1;
-                m = (float)md;
-                ld(j, v);
+        double md = 1.0;
+        for (int j = 2; j < n; ++j) {
+            md *= 0.1;
+            const float m = decay ? (float)md : 0.f;  // (0 Phi_j: NaN where Phi_j is not finite, as X_j Phi_j is)
+            ld(j, v);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) vr[e] = fmaf(m, v[e], vr[e]);
-                if (j - 2 < nres) {
+            for (int e = 0; e < 8; ++e) vr[e] = fmaf(m, v[e], vr[e]);
+            if (j - 2 < nres) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] = -v[e];
-                    put(j == 2 ? 6 : 5 + j, v);
-                    if (j == 2) {
+                for (int e = 0; e < 8; ++e) v[e] = -v[e];
+                put(j == 2 ? 6 : 5 + j, v);
+                if (j == 2) {
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) v[e] -= bf16_to_f32(f32_to_bf16(v[e]));
-                        put(7, v);
-                    }
+                    for (int e = 0; e < 8; ++e) v[e] -= bf16_to_f32(f32_to_bf16(v[e]));
+                    put(7, v);
                 }
             }
         }

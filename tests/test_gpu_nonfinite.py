@@ -196,3 +196,23 @@ def test_inference_nonfinite_token(device, value):
         out = layer(x.to(device))
     _masks_match(out, ref, "inference out")
     assert torch.isfinite(out[1:]).all()
+
+
+@pytest.mark.parametrize("n,C", [(5, 64), (16, 40), (3, 96), (8, 12)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wrapper_zero_streams_meet_nonfinite_projections(device, n, C, dtype):
+    """'zero' mode: a stream of zeros times an infinite entry of its projection is
+    NaN, in every token, also where the streams are not formed."""
+    g = torch.Generator().manual_seed(n)
+    wrap = mhc.MHCResidualWrapper(C, n, residual_mode="zero")
+    with torch.no_grad():
+        wrap.mhc.phi_pre[0, 2 * C + 7] = float("inf")
+    layer = wrap.mhc
+    ps = [layer.rmsnorm_weight.detach().double()] + [getattr(layer, k).detach().double() for k in DYN]
+    r, b = torch.randn(6, C, generator=g).to(dtype), torch.randn(6, C, generator=g).to(dtype)
+    ref = R.mhc_residual_wrapper(r.double(), b.double(),
+                                 lambda X: R.mhc_layer_dynamic(X, *ps, 20, 1e-8, 1e-5, dtype=torch.float64), n, "zero")
+    assert not torch.isfinite(ref).any()
+    with torch.no_grad():
+        out = wrap.to(device)(r.to(device), b.to(device))
+    _masks_match(out, ref, f"out n={n} C={C} {dtype}")
