@@ -2018,9 +2018,6 @@ int mhc_wrapper_static_fwd(const void* residual, const void* branch, int32_t dty
     hipError_t e = launch_static_coef(n, h_pre, h_post, h_res, weight, weight_dtype, hidden, saved, num_iters,
                                       sinkhorn_eps, s);
     if (e != hipSuccess) return hip_status(e);
-    if (!wrap_fused4(n, hidden, false))
-        return hip_status(launch_wrow_fwd(dtype, n, residual_mode == MHC_WRAPPER_DECAY, residual, branch,
-                                          saved + saved_w_offset(n), saved, 0, out, tokens, hidden, rmsnorm_eps, s));
     return hip_status(launch_wrow_fwd(dtype, n, residual_mode == MHC_WRAPPER_DECAY, residual, branch,
                                       saved + saved_w_offset(n), saved, 0, out, tokens, hidden, rmsnorm_eps, s));
 }
