@@ -1160,7 +1160,7 @@ bool layer_bwd_f32_dx_ok(int n, int64_t C, bool aligned) {
 }
 
 int layer_bwd_part_groups(int x_dtype, int n, int64_t C) {
-    (void)x_dtype;  // the fp16 stream part is that of bf16 x at n <= 4
+    (void)x_dtype;  // the fp16 stream part is that of bf16 x at n = 2 and 4
     const RowTiling t = bwd_tiling(C, n);
     return t.vpt > 0 ? t.threads / 32 : 0;
 }

@@ -161,6 +161,7 @@ hipError_t launch_layer_fwd(int x_dtype, int n, const void* x, const float* w, c
 //         mhc_device.h) with the scale exponents
 //         dx_scale[B][layer_bwd_part_groups] (register rows and
 //         C % 128 == 0 only: other bf16 x rows are an error here).
+// mode 2: mode 1 with bf16 x and an fp32 dx (layer_bwd_f32_dx_ok).
 // scratch: layer_bwd_scratch_bytes (the channel-chunked wide backward's
 // partial row sums; 0 bytes and unused otherwise).
 hipError_t launch_layer_bwd(int x_dtype, int n, int mode, const float* g, const void* x, const float* w,
@@ -177,7 +178,7 @@ size_t layer_bwd_scratch_bytes(int x_dtype, int n, int64_t B, int64_t C, bool al
 // kernels of wide.hip rather than the register rows.
 bool layer_fwd_is_wide(int n, int64_t C);
 bool layer_bwd_is_wide(int n, int64_t C);
-// launch_layer_bwd takes mode 2: mode 1 with bf16 x and an fp32 dx
+// launch_layer_bwd takes mode 2: register rows of n = 3, 5..8
 bool layer_bwd_f32_dx_ok(int n, int64_t C, bool aligned);
 hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t s);
 // p0[0, n0) and p1[0, n1) = +0 while c[0] + .. + c[nc - 1] is finite, NaN

@@ -11,7 +11,9 @@
 // fp32 rows and 'zero' need two products for dPhi, dP^T r and dP^T b: the
 // streams past the second are w_j r to fp32 rounding, so the sum kernel writes
 // w_j times the first one's total.  bf16 'decay' rows keep one per stream (the
-// rounding of X_j is 2^-9 of it).
+// rounding of X_j is 2^-9 of it).  In the sums over streams a rounding is left
+// out only where it is under fp32's 2^-24 of r: from stream 7 on in xa (2^-9 w_j),
+// from stream 4 on in s sum_j w_j X_j (2^-9 w_j^2).
 //
 // The stage structure is wrap_proj_bwd_kernel's (wrapper.hip): 8 waves x 16
 // channels, 32-token stages of r, b and G in LDS, fetched three stages ahead
@@ -436,7 +438,7 @@ __global__ __launch_bounds__(kVbThreads) __attribute__((amdgpu_waves_per_eu(2)))
             const float hp[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
             // xa = cr r + h_1 b (+ the rounded streams): without them every
             // stream of r is a multiple of it (e1.w = sum_j w_j h_j); with them
-            // stream 7 (1e-6 r) joins the multiple
+            // stream 7 joins the multiple (its rounding is 2^-9 1e-6 = 2^-29 of r)
             const float cr = XS ? (NST > 7 ? fmaf(hp[7], kWrapMult[7], hp[0]) : hp[0]) : e1.w;
             const int col = wc0 + 4 * lg;
             const int boff = t * PITCH + col * (int)sizeof(TX);
@@ -460,7 +462,7 @@ __global__ __launch_bounds__(kVbThreads) __attribute__((amdgpu_waves_per_eu(2)))
                         const float x0 = __uint_as_float(x2 << 16), x1 = __uint_as_float(x2 & 0xffff0000u);
                         xav[i] = fmaf(hp[j], x0, xav[i]);
                         xav[i + 1] = fmaf(hp[j], x1, xav[i + 1]);
-                        if (j < 4) {  // wsq holds the streams past the fourth
+                        if (j < 4) {  // wsq holds the others as w_j^2 r: 2^-9 w_4^2 < 2^-28
                             sxv[i] = fmaf(kWrapMult[j], x0, sxv[i]);
                             sxv[i + 1] = fmaf(kWrapMult[j], x1, sxv[i + 1]);
                         }
